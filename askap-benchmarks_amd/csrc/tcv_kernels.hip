@@ -140,6 +140,12 @@ __global__ __launch_bounds__(256) void k_read_stream(const uint4 *__restrict__ p
 // attic/tConvolveMPI/Benchmark.cc:293-322 and current/tConvolveMPI/Benchmark.cc:610-643.
 // Same expression order as the reference; contraction off so every product and
 // quotient is rounded exactly as on the host.
+// A block walks the visibilities in strides of the grid and adds its w-plane
+// histogram (LDS) to the device's once, at its end.  One visibility a thread
+// made every 256 visibilities add up to wSize counters that all blocks share,
+// and those atomics bound the kernel: 655 us for 1 M samples x 8 channels and
+// 129 planes, against 64 us with at most four blocks a CU, each starting
+// its flush at a bin of its own.
 __global__ __launch_bounds__(256) void k_offsets(
     const double *__restrict__ u, const double *__restrict__ v,
     const double *__restrict__ w, int nSamples, const double *__restrict__ freq,
@@ -156,9 +162,11 @@ __global__ __launch_bounds__(256) void k_offsets(
         __syncthreads();
     }
     const int total = nSamples * nChan;
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    int isBad = 0;
-    if (idx < total) {
+    const int stride = gridDim.x * blockDim.x;
+    int nBad = 0;
+    // 64-bit: idx + stride may pass 2^31 for totals near it
+    for (long long at = blockIdx.x * blockDim.x + threadIdx.x; at < total; at += stride) {
+        const int idx = (int)at;
         const int i = idx / nChan;
         const int chan = idx - i * nChan;
         const double f = freq[chan];
@@ -196,7 +204,7 @@ __global__ __launch_bounds__(256) void k_offsets(
         const bool planeOk = woff >= 0 && woff < wSize;
         const int half = s / 2;
         // footprint rows [iv, iv + s), columns [iu - s/2, iu - s/2 + s)
-        isBad = !planeOk || iu - half < 0 || iv < 0 || iu - half + s > gSize ||
+        nBad += !planeOk || iu - half < 0 || iv < 0 || iu - half + s > gSize ||
                 iv + s > gSize;
         iuOut[idx] = iu;
         ivOut[idx] = iv;
@@ -208,12 +216,15 @@ __global__ __launch_bounds__(256) void k_offsets(
         }
     }
     // one atomic per wave for the out-of-range count
-    const unsigned long long nb = __builtin_popcountll(__ballot(isBad));
-    if ((threadIdx.x & 63) == 0 && nb) atomicAdd(bad, nb);
+    for (int o = 32; o > 0; o >>= 1) nBad += __shfl_xor(nBad, o, 64);
+    if ((threadIdx.x & 63) == 0 && nBad) atomicAdd(bad, (unsigned long long)nBad);
     if (useLdsHist) {
         __syncthreads();
-        for (int k = threadIdx.x; k < wSize; k += blockDim.x)
+        const int first = (int)((blockIdx.x * 37u) % (unsigned)wSize);
+        for (int j = threadIdx.x; j < wSize; j += blockDim.x) {
+            const int k = j + first < wSize ? j + first : j + first - wSize;
             if (hist[k]) atomicAdd(&numPerPlane[k], (unsigned long long)hist[k]);
+        }
     }
 }
 
@@ -2195,7 +2206,8 @@ tcv_status launch_offsets(tcv_ctx *ctx, const double *u, const double *v,
     const int useLds = (d_numPerPlane && wSize <= 8192) ? 1 : 0;
     const size_t lds = useLds ? (size_t)wSize * 4 : 0;
     ProfScope ps(ctx, "offsets");
-    hipLaunchKernelGGL(k_offsets, dim3((total + 255) / 256), dim3(256), lds, ctx->stream,
+    const int blocks = (int)std::min<long long>(((long long)total + 255) / 256, (long long)std::max(1, ctx->cus) * 4);
+    hipLaunchKernelGGL(k_offsets, dim3(blocks), dim3(256), lds, ctx->stream,
                        u, v, w, nSamples, d_freq, nChan, cellSize, wCellSize, wSize,
                        gSize, overSample, d_sSize, d_cOffset0, iu, iv, wPlane, cOffset,
                        d_numPerPlane, d_bad, useLds);

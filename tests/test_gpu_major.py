@@ -179,3 +179,29 @@ def test_major_cycle_small_vs_oracle(ctx):
         got_model_vis = mc.model_vis.download()
         assert rel_err(got_model_vis, mvis) <= 1e-4, it
         assert rel_err(mc.data.download(), d) <= 1e-4, it
+
+
+@pytest.mark.parametrize("nSamples,nChan,wSize", [(1, 1, 33), (255, 3, 9000), (70001, 5, 129), (300000, 2, 33)])
+def test_offsets_histogram_over_strides(ctx, nSamples, nChan, wSize):
+    """Index set-up with fewer and more visibilities than one stride of the
+    grid, and more planes than the LDS histogram holds: the offsets, the plane
+    counts and the out-of-range count equal the oracle's."""
+    rng = np.random.default_rng(nSamples)
+    u, v, w = (rng.uniform(-900, 900, nSamples) for _ in range(3))
+    freq = (1.4e9 - 2.0e5 * np.arange(nChan) / nChan) / 2.998e8
+    cell, wcs, g, os_, s = 5.0, 2.0 * 1000 * freq[0] / wSize, 1024, 8, 9
+    du, dv, dw = (ctx.to_device(a) for a in (u, v, w))
+    iu, iv, wp, co, npp, bad = tcv.init_offsets(ctx, du, dv, dw, freq, cell, wcs, wSize, g, os_, [s], None,
+                                                want_wplane=True, allow_out_of_range=True)
+    f = np.tile(freq, nSamples)
+    us, vs, ws = (f * np.repeat(a, nChan) / c for a, c in ((u, cell), (v, cell), (w, wcs)))
+    a, b = np.floor(us).astype(np.int64), np.floor(vs).astype(np.int64)
+    plane = wSize // 2 + np.trunc(ws).astype(np.int64)
+    fu, fv = (os_ * (us - a)).astype(np.int64), (os_ * (vs - b)).astype(np.int64)
+    iu_r, iv_r = a + g // 2, b + g // 2
+    assert np.array_equal(iu.download(), iu_r) and np.array_equal(iv.download(), iv_r)
+    assert np.array_equal(wp.download(), plane)
+    assert np.array_equal(co.download(), (s * s * (fu + os_ * (fv + os_ * plane))).astype(np.int32))
+    ok = (plane >= 0) & (plane < wSize)
+    out = ~ok | (iu_r - s // 2 < 0) | (iv_r < 0) | (iu_r - s // 2 + s > g) | (iv_r + s > g)
+    assert np.array_equal(npp, np.bincount(plane[ok], minlength=wSize)) and bad == out.sum()
