@@ -27,8 +27,8 @@ struct tcv_ctx {
     int *d_bcast = nullptr;
     // autotuner results per workload class
     std::map<std::string, tcv_tuning> tuned;
-    // major cycle: FFT plans per grid size, grow-only Hogbom workspace
-    std::map<int, void *> fftPlans;
+    // major cycle: FFT plans and twiddle factors per grid size, grow-only workspace
+    std::map<int, void *> fftPlans, fftTwiddles;
     void *majorWs = nullptr;
     size_t majorWsBytes = 0;
     // device address of the fixed scratch array of tcv_grid_noalloc on this
@@ -39,6 +39,11 @@ struct tcv_ctx {
 
 // Looks up the scratch array's address on the context's device (tcv_noalloc.hip).
 void noalloc_setup(tcv_ctx *ctx);
+
+// The shifted 2-D transform by the library's own two passes (tcv_fft.hip), for
+// power-of-two sizes of 256 to 4096.
+bool fft_pow2_supported(int n);
+tcv_status fft_pow2_run(tcv_ctx *ctx, float2 *g, int n, int forward, int fix, float scale);
 
 // Frees the major-cycle resources of a context (tcv_major.hip).
 void major_release(tcv_ctx *ctx);

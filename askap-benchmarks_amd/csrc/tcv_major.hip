@@ -301,6 +301,8 @@ void major_release(tcv_ctx *ctx)
 {
     for (auto &kv : ctx->fftPlans) hipfftDestroy((hipfftHandle)kv.second);
     ctx->fftPlans.clear();
+    for (auto &kv : ctx->fftTwiddles) (void)hipFree(kv.second);
+    ctx->fftTwiddles.clear();
     if (ctx->majorWs) (void)hipFree(ctx->majorWs);
     ctx->majorWs = nullptr;
     ctx->majorWsBytes = 0;
@@ -330,11 +332,18 @@ static tcv_status fft_run(tcv_ctx *ctx, float *d_grid, int gSize, int forward, i
     if (!ctx) return TCV_ERR_INVALID;
     if (!d_grid || gSize < 2 || (gSize & 1) || gSize > 65534)
         return tcv_fail(ctx, TCV_ERR_INVALID, "fftExec: gSize must be even (the shift is by gSize/2)");
+    float2 *g = reinterpret_cast<float2 *>(d_grid);
+    // Powers of two of 256 to 4096: two passes of our own with the modulation
+    // folded in (4096^2: 121 us, against 281 us of the library's four passes
+    // between two of k_checker); other sizes and larger ones through hipFFT.
+    if (fft_pow2_supported(gSize)) {
+        ProfScope ps(ctx, "fft");
+        return fft_pow2_run(ctx, g, gSize, forward, fix, scale);
+    }
     hipfftHandle h;
     tcv_status st = fft_plan(ctx, gSize, &h);
     if (st != TCV_OK) return st;
     ProfScope ps(ctx, "fft");
-    float2 *g = reinterpret_cast<float2 *>(d_grid);
     const dim3 grid((gSize / 2 + 255) / 256, gSize);
     hipLaunchKernelGGL(k_checker, grid, dim3(256), 0, ctx->stream, g, gSize, 0, 1.f);
     TCV_HIP(ctx, hipGetLastError());

@@ -181,6 +181,25 @@ def test_major_cycle_small_vs_oracle(ctx):
         assert rel_err(mc.data.download(), d) <= 1e-4, it
 
 
+@pytest.mark.parametrize("g", [256, 512, 1024, 2048])
+@pytest.mark.parametrize("forward", [True, False])
+def test_fft_power_of_two_passes(ctx, g, forward):
+    """Every length of the two-pass transform, and its fftFix output.  FP32
+    rounding of about 2 log2(g) butterfly levels, each within 2^-23 of values
+    that grow with the transform, stays below 40 x 2^-23 = 4.8e-6 of the maximum."""
+    rng = np.random.default_rng(2 * g + forward)
+    x = _img(rng, g)
+    want = O.fft_exec(x, forward)
+    d = ctx.to_device(x)
+    M.fftExec(ctx, d, g, forward)
+    assert rel_err(d.download(), want) <= 4.8e-6
+    d = ctx.to_device(x)
+    M.fftExecFix(ctx, d, g, forward, 1.0 / g)
+    got = d.download()
+    assert np.all(got.imag == 0)
+    assert np.abs(got.real - want.real / g).max() <= 4.8e-6 * np.abs(want).max() / g
+
+
 @pytest.mark.parametrize("nSamples,nChan,wSize", [(1, 1, 33), (255, 3, 9000), (70001, 5, 129), (300000, 2, 33)])
 def test_offsets_histogram_over_strides(ctx, nSamples, nChan, wSize):
     """Index set-up with fewer and more visibilities than one stride of the
