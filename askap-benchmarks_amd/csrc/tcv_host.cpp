@@ -91,6 +91,7 @@ tcv_status tcv_create(int device, tcv_ctx **out)
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) != hipSuccess) return fail(TCV_ERR_DEVICE);
     ctx->cus = prop.multiProcessorCount;
+    ctx->coopLaunch = prop.cooperativeLaunch != 0;
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess)
         return fail(TCV_ERR_DEVICE);
     if (hipEventCreate(&ctx->timer0) != hipSuccess || hipEventCreate(&ctx->timer1) != hipSuccess)

@@ -12,6 +12,7 @@
 struct tcv_ctx {
     int device = 0;
     int cus = 0;
+    bool coopLaunch = false;   // the device launches cooperative grids
     hipStream_t stream = nullptr;
     std::string err;
     hipEvent_t timer0 = nullptr, timer1 = nullptr;

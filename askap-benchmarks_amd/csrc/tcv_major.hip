@@ -117,32 +117,13 @@ __device__ __forceinline__ void block_peak(unsigned long long k, unsigned long l
     }
 }
 
-// real part of a complex image into a float plane (and back)
-__global__ __launch_bounds__(256) void k_real_plane(const float2 *__restrict__ src,
-                                                    float *__restrict__ dst, long long n)
-{
-    long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    const long long stride = (long long)gridDim.x * blockDim.x;
-    for (; i < n; i += stride) dst[i] = src[i].x;
-}
+// the residual's real plane back into the complex image
 __global__ __launch_bounds__(256) void k_real_writeback(float2 *__restrict__ dst,
                                                         const float *__restrict__ src, long long n)
 {
     long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
     const long long stride = (long long)gridDim.x * blockDim.x;
     for (; i < n; i += stride) dst[i].x = src[i];
-}
-
-// peak of a float plane into *key (zeroed beforehand)
-__global__ __launch_bounds__(256) void k_peak(const float *__restrict__ img, unsigned n,
-                                              unsigned long long *key)
-{
-    unsigned long long best = 0;
-    for (unsigned i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) {
-        const unsigned long long k = peak_key(img[i], i);
-        best = k > best ? k : best;
-    }
-    block_peak(best, key);
 }
 
 struct HogbomArgs {
@@ -268,6 +249,225 @@ __global__ __launch_bounds__(256) void k_hogbom_step(HogbomArgs a, int i)
     block_peak(best, a.keys + (i + 1) % 3);
 }
 
+// Peak of the real parts of a complex image into *key (zeroed beforehand), and
+// with PLANE the real parts into a float plane as well: one read of the image.
+// Two pixels a load, four loads in flight (4096^2: 36 us alone, 68 us as an
+// extraction and a reduction of the plane).
+template <bool PLANE>
+__global__ __launch_bounds__(256) void k_peak_complex(const float2 *__restrict__ img, long long n,
+                                                      float *__restrict__ plane, unsigned long long *key)
+{
+    constexpr int U = 4;
+    const long long pairs = n >> 1, stride = (long long)gridDim.x * 256;
+    unsigned best = 0, at = 0;   // |re| bits, index; a thread's indices ascend
+    bool any = false;
+    float val = 0.f;
+    auto take = [&](float v, long long i) {
+        const unsigned a = __float_as_uint(v) & 0x7fffffffu;
+        if (a > best || !any) {
+            best = a;
+            at = (unsigned)i;
+            val = v;
+            any = true;
+        }
+    };
+    for (long long p = blockIdx.x * 256LL + threadIdx.x; p < pairs; p += U * stride) {
+        float4 v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long long q = p + u * stride;
+            v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (q < pairs) __builtin_memcpy(&v[u], img + 2 * q, 16);   // images need only 8-byte alignment
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const long long q = p + u * stride;
+            if (q >= pairs) break;
+            if constexpr (PLANE) *reinterpret_cast<float2 *>(plane + 2 * q) = make_float2(v[u].x, v[u].z);
+            take(v[u].x, 2 * q);
+            take(v[u].z, 2 * q + 1);
+        }
+    }
+    if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) {
+        const float v = img[n - 1].x;
+        if constexpr (PLANE) plane[n - 1] = v;
+        take(v, n - 1);
+    }
+    block_peak(any ? peak_key(val, at) : 0ull, key);
+}
+
+// The whole Hogbom loop in one launch, for residuals that fit the registers of
+// the workgroups that run together (up to 2^24 pixels: 64 a lane): every thread
+// keeps GPT groups of four adjacent residual pixels from the first iteration to
+// the last (columns x..x+3 of GPT rows), so an iteration reads only the PSF.  Each iteration ends with one
+// exchange among the workgroups: every workgroup publishes its peak in a slot of
+// its own and reads all the others' (two sets of slots by turns: a workgroup is
+// never more than one iteration ahead of the slowest, which must still find the
+// set before).  A slot holds the peak's key and the iteration's number (8 bits)
+// in one 64-bit word, so nothing else needs ordering.  The host launches it
+// cooperatively, so all workgroups are resident; the wait is bounded all the
+// same (*fail is set and every workgroup leaves).
+// Key: |v| bits << 25 | (2^24 - 1 - index) << 1 | sign, as peak_key orders them.
+// Bound: the PSF's read, 67 MB at 4096^2 from the Infinity Cache, and the
+// exchange.  13.4 us an iteration at 4096^2, against 35.5 us for
+// k_hogbom_step, which also reads and writes the residual (201 MB).
+struct HogbomLoop {
+    float2 *res;                     // complex residual, W x W (real parts updated)
+    const float *psf;                // PSF real plane, PW x PW, kPsfPad floats on each side
+    float2 *model;                   // complex model image
+    const unsigned long long *psfKey;   // PSF peak (peak_key)
+    unsigned long long *slots;       // 2 x kSlots, zeroed
+    unsigned long long *first;       // first residual peak (peak_key)
+    int *fail;
+    int W, PW, niters;
+    int C;                           // column groups of four a row, rounded up to a power of two
+    float gain;
+};
+constexpr int kSlots = 1024;
+constexpr int kPsfPad = 64;   // floats before and after the plane that a group of four may read (unused)
+
+__device__ __forceinline__ unsigned long long loop_key(unsigned absBits, unsigned idx, bool neg)
+{
+    return ((unsigned long long)absBits << 25) | ((unsigned long long)(0xffffffu - idx) << 1) | (neg ? 1u : 0u);
+}
+
+template <int GPT>
+__global__ __launch_bounds__(1024) void k_hogbom_loop(HogbomLoop a)
+{
+#pragma clang fp contract(off)
+    constexpr int kBlk = GPT < 4 ? GPT : 4;   // groups whose PSF reads are issued together
+    constexpr unsigned long long kSpin = 1ull << 24;   // polls of about a microsecond
+    __shared__ unsigned s_abs[16];
+    __shared__ unsigned long long s_key, s_win[16];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int W = a.W, PW = a.PW, nWG = gridDim.x;
+    // the workgroup's threads cover 1024 / C rows of C column groups a step
+    const int x = (tid & (a.C - 1)) * 4, rows = 1024 / a.C;
+    const int y0 = (int)blockIdx.x * rows + tid / a.C, dy = nWG * rows;   // row i: y0 + i * dy
+    float v[GPT][4];
+#pragma unroll
+    for (int i = 0; i < GPT; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            v[i][c] = y0 + i * dy < W && x + c < W ? a.res[(size_t)(y0 + i * dy) * W + x + c].x : 0.f;
+    const unsigned long long kp = *a.psfKey;
+    const unsigned ppos = key_index(kp);
+    const int px = (int)(ppos % (unsigned)PW), py = (int)(ppos / (unsigned)PW);
+    if (tid == 0) s_key = 0ull;
+    for (int it = 0;; ++it) {
+        // opaque copies: the rows' positions are worked out again in every
+        // iteration instead of being kept in registers across them
+        int yb = y0, xa = x;
+        asm volatile("" : "+v"(yb), "+v"(xa));
+        // this workgroup's peak: the largest |v| first, then its first pixel
+        unsigned m = 0;
+#pragma unroll
+        for (int i = 0; i < GPT; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) m = max(m, __float_as_uint(v[i][c]) & 0x7fffffffu);
+        unsigned wm = m;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) wm = max(wm, (unsigned)__shfl_xor((int)wm, o, 64));
+        if (lane == 0) s_abs[wave] = wm;
+        __syncthreads();
+        unsigned bm = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) bm = max(bm, s_abs[w]);
+        if (m == bm) {
+            unsigned idx = ~0u;
+            bool neg = false;
+            // a thread's indices ascend with i and c: the first one stays.  (The
+            // sign is shifted out: masked as above, the compiler would keep the
+            // masked values from there in registers.)
+#pragma unroll
+            for (int i = GPT - 1; i >= 0; --i)
+#pragma unroll
+                for (int c = 3; c >= 0; --c)
+                    if (__float_as_uint(v[i][c]) << 1 == bm << 1 && yb + i * dy < W && xa + c < W) {
+                        idx = (unsigned)(yb + i * dy) * (unsigned)W + (unsigned)(xa + c);
+                        neg = v[i][c] < 0.f;
+                    }
+            if (idx != ~0u) atomicMax(&s_key, loop_key(bm, idx, neg));
+        }
+        __syncthreads();
+        const unsigned long long tag = (unsigned long long)((it + 1) & 0xff) << 56;
+        unsigned long long *slots = a.slots + (it & 1) * kSlots;
+        if (tid == 0)
+            __hip_atomic_store(slots + blockIdx.x, s_key | tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        unsigned long long k = 0;
+        if (tid < nWG) {
+            for (unsigned long long n = 0; n < kSpin; ++n) {
+                k = __hip_atomic_load(slots + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (k >> 56 == tag >> 56) break;
+                k = ~0ull;   // still the wrong one when the wait ends
+            }
+        }
+        if (tid < nWG || wave * 64 < nWG) k = wave_max_u64(k);
+        if (lane == 0) s_win[wave] = k;
+        __syncthreads();
+        unsigned long long win = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) win = s_win[w] > win ? s_win[w] : win;
+        if (win == ~0ull) {
+            if (tid == 0) *a.fail = 1;
+            break;
+        }
+        win &= (1ull << 56) - 1;
+        const unsigned absBits = (unsigned)(win >> 25), pos = 0xffffffu - (unsigned)((win >> 1) & 0xffffffu);
+        const float peak = __uint_as_float(absBits | ((unsigned)(win & 1) << 31));
+        if (tid == 0) {
+            s_key = 0ull;
+            if (it == 0 && blockIdx.x == 0) *a.first = peak_key(peak, pos);
+        }
+        if (it == a.niters) break;
+        const int rx = (int)(pos % (unsigned)W), ry = (int)(pos / (unsigned)W);
+        const int diffx = rx - px, diffy = ry - px;   // as in the reference
+        const int startx = max(0, rx - px), starty = max(0, ry - py);
+        const int stopx = min(W - 1, rx + (PW - px - 1)), stopy = min(W - 1, ry + (PW - py - 1));
+        const float amp = a.gain * peak;
+        // one thread makes every model update, so that they follow each other;
+        // not in a wave that waits for the slots
+        if (blockIdx.x == 0 && tid == 1023) a.model[pos].x = a.model[pos].x + peak * a.gain;
+        bool col[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) col[c] = xa + c >= startx && xa + c <= stopx;
+        const bool colSome = xa <= stopx && xa + 3 >= startx;
+        // row y takes PSF row y - diffy where both exist
+        const int yLo = max(starty, diffy), yHi = min(stopy, PW - 1 + diffy);
+        const int at0 = (yb - diffy) * PW + (xa - diffx);   // down to -3 and up to PW * PW + 2: see kPsfPad
+#pragma unroll
+        for (int i0 = 0; i0 < GPT; i0 += kBlk) {
+            float4 p[kBlk];
+            bool row[kBlk];
+#pragma unroll
+            for (int b = 0; b < kBlk; ++b) {
+                const int y = yb + (i0 + b) * dy;
+                row[b] = colSome && y >= yLo && y <= yHi;
+                __builtin_memcpy(&p[b], a.psf + (row[b] ? at0 + (i0 + b) * dy * PW : 0), 16);
+            }
+#pragma unroll
+            for (int b = 0; b < kBlk; ++b) {
+                const float t[4] = {p[b].x, p[b].y, p[b].z, p[b].w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float u = v[i0 + b][c] - amp * t[c];
+                    v[i0 + b][c] = row[b] && col[c] ? u : v[i0 + b][c];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);   // PSF reads of kBlk rows in flight: the registers' bound
+        }
+    }
+    // on a failed wait the residual is left as it was
+    if (__hip_atomic_load(a.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+    int yw = y0, xw = x;
+    asm volatile("" : "+v"(yw), "+v"(xw));   // addresses worked out anew, not kept since the loads
+#pragma unroll
+    for (int i = 0; i < GPT; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (yw + i * dy < W && xw + c < W) a.res[(size_t)(yw + i * dy) * W + xw + c].x = v[i][c];
+}
+
 int stream_blocks(tcv_ctx *ctx, long long n, int perThread = 1)
 {
     const long long want = (n + 256LL * perThread - 1) / (256LL * perThread);
@@ -324,6 +524,46 @@ static tcv_status major_ws(tcv_ctx *ctx, size_t bytes, void **p)
         ctx->majorWsBytes = bytes;
     }
     *p = ctx->majorWs;
+    return TCV_OK;
+}
+
+// The one-launch loop: residuals of up to 2^24 pixels (64 registers a lane on
+// every CU; the keys' 24-bit index) on devices that launch cooperatively, and PSFs
+// whose tap index fits an int.
+static int hogbom_groups(const tcv_ctx *ctx, long long width, int *C, unsigned *nWG)
+{
+    *C = 1;
+    while (*C * 4LL < width) *C *= 2;
+    if (*C > 1024) return 0;
+    const long long rows = 1024 / *C;   // rows a workgroup covers in one step
+    for (int gpt = 1; gpt <= 16; gpt *= 2) {
+        const long long n = (width + rows * gpt - 1) / (rows * gpt);
+        if (n <= std::min(ctx->cus, kSlots)) {
+            *nWG = (unsigned)n;
+            return gpt;
+        }
+    }
+    return 0;
+}
+
+static bool hogbom_loop_fits(const tcv_ctx *ctx, long long width, long long psfWidth)
+{
+    int C;
+    unsigned nWG;
+    return ctx->coopLaunch && width <= 4096 && psfWidth <= 32768 && hogbom_groups(ctx, width, &C, &nWG) > 0;
+}
+
+static tcv_status launch_hogbom_loop(tcv_ctx *ctx, HogbomLoop a)
+{
+    unsigned nWG = 0;
+    const int gpt = hogbom_groups(ctx, a.W, &a.C, &nWG);
+    const void *k = gpt == 1   ? (const void *)k_hogbom_loop<1>
+                    : gpt == 2 ? (const void *)k_hogbom_loop<2>
+                    : gpt == 4 ? (const void *)k_hogbom_loop<4>
+                    : gpt == 8 ? (const void *)k_hogbom_loop<8>
+                               : (const void *)k_hogbom_loop<16>;
+    void *args[] = {&a};
+    TCV_HIP(ctx, hipLaunchCooperativeKernel(k, dim3(nWG), dim3(1024), args, 0, ctx->stream));
     return TCV_OK;
 }
 
@@ -398,19 +638,15 @@ tcv_status tcv_find_peak(tcv_ctx *ctx, const float *d_image, long long nPixels, 
     if (!ctx) return TCV_ERR_INVALID;
     if (!d_image || nPixels < 1 || nPixels > 0xffffffffLL || !maxVal || !maxPos)
         return tcv_fail(ctx, TCV_ERR_INVALID, "tcv_find_peak: bad argument (1 <= nPixels < 2^32)");
-    const size_t planeB = ((size_t)nPixels * 4 + 255) & ~size_t(255);
     void *ws;
-    tcv_status st = major_ws(ctx, planeB + 256, &ws);
+    tcv_status st = major_ws(ctx, 256, &ws);
     if (st != TCV_OK) return st;
-    float *plane = (float *)ws;
-    unsigned long long *key = (unsigned long long *)((char *)ws + planeB);
+    unsigned long long *key = (unsigned long long *)ws;
     ProfScope ps(ctx, "find_peak");
     st = launch_fill_u32(ctx, key, 0u, 2);
     if (st != TCV_OK) return st;
-    hipLaunchKernelGGL(k_real_plane, dim3(stream_blocks(ctx, nPixels, 4)), dim3(256), 0,
-                       ctx->stream, (const float2 *)d_image, plane, nPixels);
-    hipLaunchKernelGGL(k_peak, dim3(stream_blocks(ctx, nPixels, 4)), dim3(256), 0, ctx->stream,
-                       plane, (unsigned)nPixels, key);
+    hipLaunchKernelGGL(k_peak_complex<false>, dim3(stream_blocks(ctx, nPixels, 8)), dim3(256), 0,
+                       ctx->stream, (const float2 *)d_image, nPixels, (float *)nullptr, key);
     TCV_HIP(ctx, hipGetLastError());
     unsigned long long k = 0;
     TCV_HIP(ctx, hipMemcpyAsync(&k, key, 8, hipMemcpyDeviceToHost, ctx->stream));
@@ -433,50 +669,63 @@ tcv_status tcv_hogbom(tcv_ctx *ctx, float *d_residual, long long width, const fl
         width * width > 0xffffffffLL || psfWidth * psfWidth > 0xffffffffLL)
         return tcv_fail(ctx, TCV_ERR_INVALID, "tcv_hogbom: bad argument (widths below 65536)");
     const long long n = width * width, pn = psfWidth * psfWidth;
-    const size_t resB = ((size_t)n * 4 + 255) & ~size_t(255);
-    const size_t psfB = ((size_t)pn * 4 + 255) & ~size_t(255);
+    const bool loop = hogbom_loop_fits(ctx, width, psfWidth);
+    // PSF plane | keys, failure flag | slots of the loop, or residual plane
+    const size_t psfB = ((size_t)(pn + 2 * kPsfPad) * 4 + 255) & ~size_t(255);
+    const size_t resB = loop ? 2 * kSlots * sizeof(unsigned long long) : ((size_t)n * 4 + 255) & ~size_t(255);
     void *ws;
-    tcv_status st = major_ws(ctx, resB + psfB + 256, &ws);
+    tcv_status st = major_ws(ctx, psfB + 256 + resB, &ws);
     if (st != TCV_OK) return st;
-    float *res = (float *)ws;
-    float *psf = (float *)((char *)ws + resB);
-    unsigned long long *keys = (unsigned long long *)((char *)ws + resB + psfB);
+    float *psf = (float *)ws + kPsfPad;
+    unsigned long long *keys = (unsigned long long *)((char *)ws + psfB);
+    void *rest = (char *)ws + psfB + 256;
     ProfScope ps(ctx, "hogbom");
-    st = launch_fill_u32(ctx, keys, 0u, 8);
+    st = launch_fill_u32(ctx, keys, 0u, loop ? 64 + resB / 4 : 64);
     if (st != TCV_OK) return st;
-    hipLaunchKernelGGL(k_real_plane, dim3(stream_blocks(ctx, n, 4)), dim3(256), 0, ctx->stream,
-                       (const float2 *)d_residual, res, n);
-    hipLaunchKernelGGL(k_real_plane, dim3(stream_blocks(ctx, pn, 4)), dim3(256), 0, ctx->stream,
-                       (const float2 *)d_psf, psf, pn);
-    hipLaunchKernelGGL(k_peak, dim3(stream_blocks(ctx, pn, 4)), dim3(256), 0, ctx->stream, psf,
-                       (unsigned)pn, keys + 3);
-    hipLaunchKernelGGL(k_peak, dim3(stream_blocks(ctx, n, 4)), dim3(256), 0, ctx->stream, res,
-                       (unsigned)n, keys + 0);
+    hipLaunchKernelGGL(k_peak_complex<true>, dim3(stream_blocks(ctx, pn, 8)), dim3(256), 0, ctx->stream,
+                       (const float2 *)d_psf, pn, psf, keys + 3);
     TCV_HIP(ctx, hipGetLastError());
     unsigned long long first = 0;
-    if (dirtyPeakVal || dirtyPeakPos)
-        TCV_HIP(ctx, hipMemcpyAsync(&first, keys, 8, hipMemcpyDeviceToHost, ctx->stream));
-    HogbomArgs a{res, psf, (float2 *)d_model, keys, (int)width, (int)psfWidth, gain};
-    // four pixels a thread when the rows are whole float4s
-    const bool vec = width % 4 == 0;
-    const long long perRow = vec ? width / 4 : width;
-    const int bx = (int)std::min<long long>((perRow + 255) / 256, 64);
-    const int by = (int)std::max<long long>(1, std::min<long long>(width, (long long)ctx->cus * 8 / bx));
-    for (int i = 0; i < niters; ++i) {
-        if (vec)
-            hipLaunchKernelGGL(k_hogbom_step<true>, dim3(bx, by), dim3(256), 0, ctx->stream, a, i);
-        else
-            hipLaunchKernelGGL(k_hogbom_step<false>, dim3(bx, by), dim3(256), 0, ctx->stream, a, i);
+    int failed = 0;
+    if (loop) {
+        HogbomLoop a{(float2 *)d_residual, psf, (float2 *)d_model, keys + 3, (unsigned long long *)rest,
+                     keys, (int *)(keys + 8), (int)width, (int)psfWidth, niters, 0, gain};
+        st = launch_hogbom_loop(ctx, a);
+        if (st != TCV_OK) return st;
+        if (dirtyPeakVal || dirtyPeakPos)
+            TCV_HIP(ctx, hipMemcpyAsync(&first, keys, 8, hipMemcpyDeviceToHost, ctx->stream));
+        if (psfPeakVal || psfPeakPos || dirtyPeakVal || dirtyPeakPos)
+            TCV_HIP(ctx, hipMemcpyAsync(&failed, a.fail, 4, hipMemcpyDeviceToHost, ctx->stream));
+    } else {
+        float *res = (float *)rest;
+        hipLaunchKernelGGL(k_peak_complex<true>, dim3(stream_blocks(ctx, n, 8)), dim3(256), 0, ctx->stream,
+                           (const float2 *)d_residual, n, res, keys + 0);
+        TCV_HIP(ctx, hipGetLastError());
+        if (dirtyPeakVal || dirtyPeakPos)
+            TCV_HIP(ctx, hipMemcpyAsync(&first, keys, 8, hipMemcpyDeviceToHost, ctx->stream));
+        HogbomArgs a{res, psf, (float2 *)d_model, keys, (int)width, (int)psfWidth, gain};
+        // four pixels a thread when the rows are whole float4s
+        const bool vec = width % 4 == 0;
+        const long long perRow = vec ? width / 4 : width;
+        const int bx = (int)std::min<long long>((perRow + 255) / 256, 64);
+        const int by = (int)std::max<long long>(1, std::min<long long>(width, (long long)ctx->cus * 8 / bx));
+        for (int i = 0; i < niters; ++i) {
+            if (vec)
+                hipLaunchKernelGGL(k_hogbom_step<true>, dim3(bx, by), dim3(256), 0, ctx->stream, a, i);
+            else
+                hipLaunchKernelGGL(k_hogbom_step<false>, dim3(bx, by), dim3(256), 0, ctx->stream, a, i);
+        }
+        TCV_HIP(ctx, hipGetLastError());
+        hipLaunchKernelGGL(k_real_writeback, dim3(stream_blocks(ctx, n, 4)), dim3(256), 0, ctx->stream,
+                           (float2 *)d_residual, (const float *)res, n);
+        TCV_HIP(ctx, hipGetLastError());
     }
-    TCV_HIP(ctx, hipGetLastError());
-    hipLaunchKernelGGL(k_real_writeback, dim3(stream_blocks(ctx, n, 4)), dim3(256), 0, ctx->stream,
-                       (float2 *)d_residual, (const float *)res, n);
-    TCV_HIP(ctx, hipGetLastError());
     unsigned long long pk = 0;
     if (psfPeakVal || psfPeakPos)
         TCV_HIP(ctx, hipMemcpyAsync(&pk, keys + 3, 8, hipMemcpyDeviceToHost, ctx->stream));
     if (psfPeakVal || psfPeakPos || dirtyPeakVal || dirtyPeakPos) {
         TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (failed) return tcv_fail(ctx, TCV_ERR_DEVICE, "tcv_hogbom: the workgroups lost each other");
         auto val = [](unsigned long long k) {
             const unsigned a2 = (unsigned)(k >> 33);
             float f;

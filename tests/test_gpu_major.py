@@ -200,6 +200,31 @@ def test_fft_power_of_two_passes(ctx, g, forward):
     assert np.abs(got.real - want.real / g).max() <= 4.8e-6 * np.abs(want).max() / g
 
 
+@pytest.mark.parametrize("g,pw", [(1, 1), (5, 5), (7, 1), (255, 2), (257, 300), (1024, 1024), (1500, 90),
+                                  (2051, 2051), (4096, 513), (4099, 64)])
+def test_hogbom_image_sizes(ctx, g, pw):
+    """The loop kernel's groupings (one, four and 16 rows a thread, rows that are
+    no multiple of four, one workgroup and all of them), PSFs of a few pixels,
+    wider than the image and off its edge, and an image beyond the loop
+    kernel; two pixels tie for the first peak."""
+    rng = np.random.default_rng(g + pw)
+    dirty = rng.standard_normal((g, g)).astype(np.float32).astype(np.complex64)
+    dirty.imag = 2.0
+    if g > 4:
+        dirty[g - 1, g - 2] = -9.0
+        dirty[g // 2, 1] = 9.0
+    psf = (0.05 * rng.standard_normal((pw, pw))).astype(np.complex64)
+    psf[pw // 3, pw // 2] = 2.0
+    niters = 6 if g > 1000 else 300
+    r_ref, m_ref, pk_ref, dk_ref = O.deconvolve(dirty, psf, None, niters, 0.1)
+    d_res, d_psf, d_model = ctx.to_device(dirty), ctx.to_device(psf), ctx.zeros((g, g), np.complex64)
+    pk, dk = M.deconvolve(ctx, d_res, g, d_psf, pw, d_model, niters, 0.1)
+    assert (pk, dk) == (pk_ref, dk_ref)
+    assert np.array_equal(d_res.download(), r_ref)
+    assert np.array_equal(d_model.download(), m_ref)
+    assert M.findPeak(ctx, d_res) == O.find_peak(r_ref)
+
+
 @pytest.mark.parametrize("nSamples,nChan,wSize", [(1, 1, 33), (255, 3, 9000), (70001, 5, 129), (300000, 2, 33)])
 def test_offsets_histogram_over_strides(ctx, nSamples, nChan, wSize):
     """Index set-up with fewer and more visibilities than one stride of the
