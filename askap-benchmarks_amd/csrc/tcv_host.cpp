@@ -633,12 +633,12 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
     n += align256(sizeof(int4) * p->maxItems);
     n += 3 * align256(sizeof(int) * (sh.nKeys + 1));
     n += 2 * align256(sizeof(int) * (slots + 1));
-    n += align256(sizeof(int) * 32);
+    n += align256(sizeof(int) * kMetaInts);
     n += align256(sizeof(int) * p->scanTmpLen);
     if (twoLists) {
         n += align256(sizeof(int4) * p->maxItemsG);
         n += 2 * align256(sizeof(int) * (slotsG + 1));
-        n += align256(sizeof(int) * 32);
+        n += align256(sizeof(int) * kMetaInts);
     }
     *bytes = n;
     return TCV_OK;
@@ -663,14 +663,14 @@ void plan_bind(tcv_plan *p, char *block)
     p->cursor = (int *)take(sizeof(int) * (sh.nKeys + 1));
     p->itemCount = (int *)take(sizeof(int) * (slots + 1));
     p->itemStart = (int *)take(sizeof(int) * (slots + 1));
-    p->meta = (int *)take(sizeof(int) * 32);
+    p->meta = (int *)take(sizeof(int) * kMetaInts);
     p->scanTmp = (int *)take(sizeof(int) * p->scanTmpLen);
     if (p->maxItemsG) {
         const long long slotsG = (long long)sh.phasesG * sh.nTiles;
         p->itemsG = (int4 *)take(sizeof(int4) * p->maxItemsG);
         p->itemCountG = (int *)take(sizeof(int) * (slotsG + 1));
         p->itemStartG = (int *)take(sizeof(int) * (slotsG + 1));
-        p->metaG = (int *)take(sizeof(int) * 32);
+        p->metaG = (int *)take(sizeof(int) * kMetaInts);
     } else {
         p->itemsG = p->items;
         p->itemCountG = p->itemCount;

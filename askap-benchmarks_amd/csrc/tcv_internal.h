@@ -131,7 +131,13 @@ struct JobDesc {
 };
 
 constexpr int kMaxPersistentBlocks = 8192;
-constexpr size_t kBatchQueueBytes = 1024;   // ints 0 and 16 + 16 q (q < 8) are used
+// Work-queue heads, one to a 128-byte line: atomics on one line are served one
+// after the other (12 ns each, measured), whichever of its words they go to.
+// With the eight heads of a plan on one line, spectral-scale gridding (8.4 M
+// visibilities, width 129) took 60.6 ms and degridding 53.4; apart 58.0 and 49.7.
+constexpr int kHeadInts = 32;
+constexpr int kMetaInts = 32 + 8 * kHeadInts;   // a plan's meta block (see tcv_plan::meta)
+constexpr size_t kBatchQueueBytes = 9 * kHeadInts * sizeof(int);   // the queue, then one head per XCD
 
 // Tiled kernels used when a tuning leaves the choice open.  Gridder: 1 tile in
 // registers, 2 tile in LDS, 3 registers with two columns per lane.  Degridder:
@@ -172,9 +178,9 @@ struct tcv_plan {
     int *cursor = nullptr;        // nKeys
     int *itemCount = nullptr;     // phases * nTiles + 1
     int *itemStart = nullptr;     // phases * nTiles + 1
-    int *meta = nullptr;          // 32 ints: [0] items [1] queue head [2] entries [3] bad,
+    int *meta = nullptr;          // kMetaInts: [0] items [1] queue head [2] entries [3] bad,
                                   // [4..5] the entries' cOffset range (see note_c_range),
-                                  // [8..15] per-XCD heads, [16..24] per-XCD item ranges
+                                  // [16..24] per-XCD item ranges, [32 + kHeadInts q] per-XCD heads
     // the gridder's work items (phasesG); the same buffers as above when
     // phasesG == phases
     int4 *itemsG = nullptr;

@@ -707,7 +707,8 @@ __global__ __launch_bounds__(256) void k_plan_items(int pass, PlanDevArgs a,
 }
 
 // meta: [0] items [1] queue head [2] entries [3] out of range [4..5] cOffset range
-//       [8..15] per-XCD queue heads, [16..24] per-XCD item ranges (XCD-major plans)
+//       [16..24] per-XCD item ranges (XCD-major plans), [32 + kHeadInts q] per-XCD
+//       queue heads
 __global__ void k_plan_meta(const int *__restrict__ itemStart, int nItemSlots,
                             const int *__restrict__ starts, long long nKeys, int xcdSlots,
                             int *__restrict__ meta)
@@ -716,7 +717,7 @@ __global__ void k_plan_meta(const int *__restrict__ itemStart, int nItemSlots,
         meta[0] = itemStart[nItemSlots];
         meta[1] = 0;
         meta[2] = starts[nKeys];
-        for (int x = 0; x < 8; ++x) meta[8 + x] = 0;
+        for (int x = 0; x < 8; ++x) meta[32 + kHeadInts * x] = 0;
         for (int x = 0; x <= 8; ++x)
             meta[16 + x] = xcdSlots ? itemStart[x * xcdSlots] : (x ? meta[0] : 0);
     }
@@ -724,7 +725,7 @@ __global__ void k_plan_meta(const int *__restrict__ itemStart, int nItemSlots,
 
 __global__ void k_reset_queue(int *meta)
 {
-    if (threadIdx.x < 8) meta[8 + threadIdx.x] = 0;
+    if (threadIdx.x < 8) meta[32 + kHeadInts * threadIdx.x] = 0;
     if (threadIdx.x == 0) meta[1] = 0;
 }
 
@@ -837,7 +838,7 @@ struct ItemSource {
 
     // Single job: items are XCD-major with per-XCD queues.  Batch: each XCD
     // walks its share of every job in job order (per-XCD prefix sums after the
-    // job prefix, counters at queue[16 + 16 q]), then takes from the others.
+    // job prefix, counters at queue[kHeadInts (1 + q)]), then takes from the others.
     int xcd;
     int *bcast;   // one slot per workgroup (kernels that keep LDS for their tile)
 
@@ -849,7 +850,7 @@ struct ItemSource {
     // next work item (one lane calls this); >= total() when none is left
     __device__ __forceinline__ int acquire() const
     {
-        if (!xcd) return atomicAdd(queue, 1);
+        if (!xcd) return (int)gridDim.x + atomicAdd(queue, 1);   // after the workgroups' first items
         // own XCD first (hardware XCC_ID register), then steal from the others
         const int x0 = (int)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 7);
         if constexpr (BATCH) {
@@ -859,7 +860,7 @@ struct ItemSource {
                 const int *px = prefix + n1 * (1 + q);
                 const int tot = px[nJobs];
                 if (tot == 0) continue;
-                const int i = atomicAdd(queue + 16 + 16 * q, 1);
+                const int i = atomicAdd(queue + kHeadInts * (1 + q), 1);
                 if (i >= tot) continue;
                 int lo = 0, hi = nJobs;   // px[lo] <= i < px[hi]
                 while (hi - lo > 1) {
@@ -874,7 +875,7 @@ struct ItemSource {
             const int q = (x0 + k) & 7;
             const int b = one.meta[16 + q], e = one.meta[17 + q];
             if (b >= e) continue;
-            const int i = atomicAdd(one.meta + 8 + q, 1);
+            const int i = atomicAdd(one.meta + 32 + kHeadInts * q, 1);
             if (b + i < e) return b + i;
         }
         return 0x7fffffff;
@@ -920,11 +921,12 @@ __device__ __forceinline__ int acquire_for_block(const ItemSource<BATCH> &src, i
     return item;
 }
 
-// The first item of a workgroup (thread 0 only; see acquire_for_block).
+// The first item of a workgroup (thread 0 only; see acquire_for_block).  The single
+// queue starts after the workgroups' first items, which are their own numbers.
 template <bool BATCH>
 __device__ __forceinline__ int first_item(const ItemSource<BATCH> &src)
 {
-    return threadIdx.x == 0 ? src.acquire() : 0;
+    return threadIdx.x != 0 ? 0 : src.xcd ? src.acquire() : (int)blockIdx.x;
 }
 
 // The TW x TH grid tile at (Bx, By) into LDS (a workgroup of 256 threads),
@@ -2305,7 +2307,7 @@ tcv_status plan_build_kernels(tcv_ctx *ctx, tcv_plan *p, const GeomDev &g)
     ProfScope ps(ctx, "plan");
     tcv_status st;
     if ((st = launch_fill_u32(ctx, p->counts, 0, (size_t)sh.nKeys + 1)) != TCV_OK) return st;
-    if ((st = launch_fill_u32(ctx, p->meta, 0, 32)) != TCV_OK) return st;
+    if ((st = launch_fill_u32(ctx, p->meta, 0, kMetaInts)) != TCV_OK) return st;
     const bool lds = sh.nKeys <= kLdsKeys;
     const int nb = lds ? (g.nVis + 256 * kBinVPT - 1) / (256 * kBinVPT) : (g.nVis + 255) / 256;
     auto bin = [&](int pass) -> tcv_status {
@@ -2381,7 +2383,7 @@ tcv_status plan_build_kernels(tcv_ctx *ctx, tcv_plan *p, const GeomDev &g)
         return st;
     if (p->metaG != p->meta) {
         // the out-of-range count lives in meta[3]; the gridder's meta gets its own copy
-        if ((st = launch_fill_u32(ctx, p->metaG, 0, 32)) != TCV_OK) return st;
+        if ((st = launch_fill_u32(ctx, p->metaG, 0, kMetaInts)) != TCV_OK) return st;
         if ((st = items(sh.phasesG, sh.xcdG, p->itemCountG, p->itemStartG, p->itemsG, p->metaG)) != TCV_OK)
             return st;
     }
@@ -2447,7 +2449,7 @@ __global__ void k_batch_prefix(const JobDesc *__restrict__ jobs, int nJobs, int 
         run += t == 0 ? m[0] : m[16 + t] - m[15 + t];
     }
     out[nJobs] = run;
-    queue[16 * t] = 0;   // t = 0: the single queue; t = 1 + q: XCD q's counter
+    queue[kHeadInts * t] = 0;   // t = 0: the single queue; t = 1 + q: XCD q's counter
 }
 
 // the pair gridder over column groups of CGW (TH gives every wave whole row groups)
