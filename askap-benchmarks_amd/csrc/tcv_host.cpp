@@ -551,8 +551,65 @@ static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 }  // extern "C"
 
+// Classes of kernel widths that an automatic plan takes by regions
+// (tcv_narrow.hip): the widest kernel of each, the region's cells a side and the
+// entries of a work item.  Re-bin + grid + degrid in us, tiles -> regions:
+//   widths 7-19, 3.8 M visibilities, 4096^2     671 + 1860 + 1685 -> 413 + 360 + 264
+//   widths 7-121, 5.4 M visibilities, 4096^2   1347 + 5217 + 2985 -> 1571 + 2065 + 1595
+//   width 19, 500 000, 4096^2 (8 keys a region) 443 + 450 + 396   -> 188 + 421 + 161
+//   width 15, 8000, 512^2                        75 + 35 + 42     -> 65 + 12 + 10
+// Widths 32-44 by regions of 64 cells were slower than tiles there (2155 + 2749 +
+// 1885 against 1900 + 2648 + 1658), and a class of widths up to 9 by regions of
+// 24 cells costs more binning (350) than it saves.
+struct WidthClass { int width, region, chunk; };
+constexpr WidthClass kClasses[] = {{19, 32, 128}, {31, 48, 64}};
+// Kernels of 20 to 31 only: a region's flush costs as much as two or three of
+// their footprints, so a job that is neither small nor dense keeps its tiles.
+// Width 31, 4096^2 (51 984 regions), re-bin + grid + degrid: 8000 visibilities
+// 102 + 92 + 89 -> 48 + 86 + 38; 64 000 132 + 127 + 115 -> 74 + 387 + 142;
+// 500 000 401 + 670 + 488 -> 189 + 733 + 338.
+constexpr int kSmallJob = 8192, kDenseRegion = 8;
+// Entries of the tiles' work items beside regions: the few wide visibilities
+// left fill no long ones (widths 7-121 above: 2842 + 1827 with 1024, 2022 + 1450
+// with 128, 2116 + 1480 with 512; 500 000 visibilities 1102 + 795 and 537 + 444).
+constexpr int kRestChunk = 128;
+
+// Array sizes that follow from a plan's shape, and the bytes of its buffers.
+static tcv_status plan_sizes(tcv_ctx *ctx, const tcv_geometry *g, tcv_plan *p, size_t *bytes);
+
+// The plan of the visibilities of widths [sLo, maxS] by regions of R x R cells.
+static tcv_status region_setup(tcv_ctx *ctx, const tcv_geometry *g, int R, int chunk, int maxS, int sLo, tcv_plan *p,
+                               size_t *bytes)
+{
+    PlanShape &sh = p->sh;
+    sh.region = R;
+    sh.bw = sh.bh = sh.region - maxS + 1;
+    sh.sLo = sLo;
+    sh.sHi = maxS;
+    sh.maxS = maxS;
+    sh.nTX = (g->gSize + sh.bw - 1) / sh.bw;
+    sh.nTY = (g->gSize + sh.bh - 1) / sh.bh;
+    sh.nTiles = sh.nTX * sh.nTY;
+    sh.phases = sh.phasesG = 1;
+    sh.xcd = sh.xcdG = 0;
+    sh.chunk = chunk;
+    // C-slice keys: enough to keep neighbouring entries on neighbouring slices,
+    // but no more (region, key) counters than about two a visibility
+    sh.k2 = 1;
+    while (sh.k2 < 2048 && (long long)sh.nTiles * sh.k2 < (long long)g->nVis) sh.k2 *= 2;
+    sh.maxEntries = std::max(1, g->nVis);
+    return plan_sizes(ctx, g, p, bytes);
+}
+
+// Whether a tuning leaves every choice of shape open.
+static bool open_shape(const tcv_tuning &t)
+{
+    return t.tile_w <= 0 && t.tile_h <= 0 && t.chunk <= 0 && t.slice_keys <= 0 && t.phases <= 0 && t.xcd_split < 0 &&
+           t.kernel <= 0 && t.degrid_kernel <= 0 && t.grid_phases <= 0 && t.grid_cols <= 0;
+}
+
 tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tuning, tcv_plan *p,
-                      size_t *bytes)
+                      size_t *bytes, bool tilesOnly)
 {
     int maxS = 0;
     tcv_status st = check_geometry(ctx, g, &maxS);
@@ -568,6 +625,27 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
     if (!tuning && ctx) {
         auto it = ctx->tuned.find(tuning_class(g));
         if (it != ctx->tuned.end()) t = it->second;
+    }
+    // a plan whose shape is left open takes its narrower kernels by regions
+    struct Part { int lo, hi, region, chunk; };
+    std::vector<Part> parts;   // the classes that the job's widths fall in
+    int tilesLo = 0;           // narrowest kernel left to the tiles
+    if (!tilesOnly && open_shape(t)) {
+        int least = maxS;
+        for (int k = 0; k < g->nPlanes; k++) least = std::min(least, g->sSize[k]);
+        const long long across = (g->gSize + kClasses[1].region - maxS) / std::max(1, kClasses[1].region - maxS + 1);
+        const bool sparse = least > kClasses[0].width && maxS <= kClasses[1].width && g->nVis > kSmallJob &&
+                            g->nVis < kDenseRegion * across * across;
+        if (least >= 2 && !sparse)   // pairs of taps need widths of two
+            for (const WidthClass &c : kClasses) {
+                int hi = 0;
+                for (int k = 0; k < g->nPlanes; k++)
+                    if (g->sSize[k] >= tilesLo && g->sSize[k] <= c.width) hi = std::max(hi, g->sSize[k]);
+                if (hi) parts.push_back({tilesLo, hi, c.region, c.chunk});
+                tilesLo = c.width + 1;
+            }
+        if (parts.empty()) tilesLo = 0;
+        else t.chunk = kRestChunk;
     }
     auto_tuning(maxS, g, &t);
     if (!tiled_config_supported(t.tile_w, t.tile_h))
@@ -606,12 +684,51 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
                         "tiles wider or taller than 64 need the pair kernels (code 3) and kernel widths "
                         "of at least 2");
     sh.minS = minS;
+    sh.region = 0;
+    sh.bw = sh.tw;
+    sh.bh = sh.th;
+    sh.sHi = 0x7fffffff;
+    p->parts.clear();
+    p->nVis = g->nVis;
+    p->gSize = g->gSize;
+    p->nPlanes = g->nPlanes;
+    p->cSize = g->cSize;
+    p->sSizeHost.assign(g->sSize, g->sSize + g->nPlanes);
+    sh.sLo = tilesLo;
     sh.nTX = (g->gSize + sh.tw - 1) / sh.tw;
     sh.nTY = (g->gSize + sh.th - 1) / sh.th;
     sh.nTiles = sh.nTX * sh.nTY;
     sh.maxS = maxS;
     const long long perVis = (long long)((maxS + sh.tw - 2) / sh.tw + 1) * ((maxS + sh.th - 2) / sh.th + 1);
     sh.maxEntries = std::max<long long>(1, (long long)g->nVis * perVis);
+    // (also where no tiles are used: what they are too large for is refused)
+    if ((st = plan_sizes(ctx, g, p, bytes)) != TCV_OK) return st;
+    // the classes' plans share one block with the tiles; the last one is the plan
+    // itself when nothing is left to the tiles
+    const bool tiles = tilesLo <= maxS;
+    size_t partBytes = 0;
+    for (size_t i = 0; i + (tiles ? 0 : 1) < parts.size(); ++i) {
+        p->parts.emplace_back(new tcv_plan());
+        tcv_plan *q = p->parts.back().get();
+        q->nVis = g->nVis;
+        q->gSize = g->gSize;
+        q->nPlanes = g->nPlanes;
+        q->cSize = g->cSize;
+        q->sh = sh;   // the fields that region_setup leaves
+        size_t more = 0;
+        st = region_setup(ctx, g, parts[i].region, parts[i].chunk, parts[i].hi, parts[i].lo, q, &more);
+        if (st != TCV_OK) return st;
+        partBytes += more;
+    }
+    if (!tiles)
+        st = region_setup(ctx, g, parts.back().region, parts.back().chunk, parts.back().hi, parts.back().lo, p, bytes);
+    *bytes += partBytes;
+    return st;
+}
+
+static tcv_status plan_sizes(tcv_ctx *ctx, const tcv_geometry *g, tcv_plan *p, size_t *bytes)
+{
+    PlanShape &sh = p->sh;
     sh.nKeys = (long long)sh.nTiles * sh.k2;
     if (sh.maxEntries >= 0x7fffffffLL || sh.nKeys >= 0x7fffffffLL)
         return tcv_fail(ctx, TCV_ERR_UNSUPPORTED, "plan too large for 32-bit entry indices");
@@ -619,11 +736,6 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
     const bool twoLists = sh.phasesG != sh.phases || sh.xcdG != sh.xcd;
     p->maxItemsG = twoLists ? sh.maxEntries / sh.chunk + (long long)sh.phasesG * sh.nTiles + 1 : 0;
     const long long slotsG = (long long)sh.phasesG * sh.nTiles;
-    p->nVis = g->nVis;
-    p->gSize = g->gSize;
-    p->nPlanes = g->nPlanes;
-    p->cSize = g->cSize;
-    p->sSizeHost.assign(g->sSize, g->sSize + g->nPlanes);
     const long long slots = (long long)sh.phases * sh.nTiles;
     p->scanTmpLen = std::max(scan_tmp_len(sh.nKeys), std::max(scan_tmp_len(slots), scan_tmp_len(slotsG)));
     size_t n = 0;
@@ -678,6 +790,12 @@ void plan_bind(tcv_plan *p, char *block)
         p->metaG = p->meta;
     }
     p->block = block;
+    for (auto &part : p->parts) {
+        plan_bind(part.get(), q);
+        q = part->blockEnd;
+        part->d_sSize = p->d_sSize;
+    }
+    p->blockEnd = q;
 }
 
 void mark_shared_grids(std::vector<JobDesc> &jobs)
@@ -762,6 +880,7 @@ tcv_status tcv_plan_build(tcv_ctx *ctx, tcv_plan *p, const tcv_geometry *g)
     gd.cSize = g->cSize;
     gd.sSize = g->d_wPlane ? p->d_sSize : nullptr;
     p->cSize = g->cSize;
+    for (auto &part : p->parts) part->cSize = g->cSize;
     p->geom = gd;
     p->hasGeom = true;
     return plan_build_kernels(ctx, p, gd);
@@ -787,6 +906,13 @@ tcv_status tcv_plan_info(tcv_ctx *ctx, tcv_plan *p, tcv_tuning *t, long long *en
     int meta[4] = {0, 0, 0, 0};   // items, queue head, entries, out of range
     TCV_HIP(ctx, hipMemcpyAsync(meta, p->meta, sizeof(meta), hipMemcpyDeviceToHost, ctx->stream));
     TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    for (auto &part : p->parts) {
+        int more[3] = {0, 0, 0};
+        TCV_HIP(ctx, hipMemcpyAsync(more, part->meta, sizeof(more), hipMemcpyDeviceToHost, ctx->stream));
+        TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        meta[0] += more[0];
+        meta[2] += more[2];
+    }
     if (items) *items = meta[0];
     if (entries) *entries = meta[2];
     if (outOfRange) *outOfRange = meta[3];
@@ -896,7 +1022,7 @@ tcv_status tcv_batch_create(tcv_ctx *ctx, int nJobs, const tcv_job *jobs, tcv_ba
     if (!ctx || !out || nJobs < 1 || !jobs) return tcv_fail(ctx, TCV_ERR_INVALID, "tcv_batch_create: bad argument");
     *out = nullptr;
     tcv_batch *b = new tcv_batch();
-    b->nJobs = nJobs;
+    std::vector<JobDesc> tiled, tiledD, narrow[2];
     for (int j = 0; j < nJobs; j++) {
         const tcv_job &J = jobs[j];
         if (!J.plan || !J.d_C || !J.d_grid) {
@@ -924,22 +1050,44 @@ tcv_status tcv_batch_create(tcv_ctx *ctx, int nJobs, const tcv_job *jobs, tcv_ba
     // its own job may still meet another job's item on the same cells, so those
     // jobs flush every tile with atomics.
     mark_shared_grids(b->host);
+    for (int j = 0; j < nJobs; j++) {
+        const tcv_job &J = jobs[j];
+        auto by_regions = [&](const tcv_plan *p) {
+            narrow[p->sh.region == kRegions[0] ? 0 : 1].push_back(
+                make_job_desc(p, true, J.d_data, J.d_C, (float2 *)J.d_grid, (float2 *)J.d_out, nullptr));
+        };
+        for (auto &q : J.plan->parts) by_regions(q.get());
+        if (J.plan->sh.region > 0) {
+            by_regions(J.plan);
+        } else {
+            tiled.push_back(b->host[j]);
+            tiledD.push_back(b->hostD[j]);
+        }
+    }
+    b->nJobs = (int)tiled.size();
     auto fail = [&](const char *m) {
         if (b->d_jobs) (void)hipFree(b->d_jobs);
         if (b->d_jobsD) (void)hipFree(b->d_jobsD);
         if (b->d_prefix) (void)hipFree(b->d_prefix);
         if (b->d_queue) (void)hipFree(b->d_queue);
+        for (JobDesc *d : b->d_narrow)
+            if (d) (void)hipFree(d);
         delete b;
         return tcv_fail(ctx, TCV_ERR_NOMEM, m);
     };
-    if (hipMalloc((void **)&b->d_jobs, sizeof(JobDesc) * nJobs) != hipSuccess ||
-        hipMalloc((void **)&b->d_jobsD, sizeof(JobDesc) * nJobs) != hipSuccess ||
-        hipMalloc((void **)&b->d_prefix, sizeof(int) * 9 * (nJobs + 1)) != hipSuccess ||
+    auto upload = [](JobDesc **d, const std::vector<JobDesc> &v) {
+        return hipMalloc((void **)d, sizeof(JobDesc) * std::max<size_t>(1, v.size())) == hipSuccess &&
+               (v.empty() || hipMemcpy(*d, v.data(), sizeof(JobDesc) * v.size(), hipMemcpyHostToDevice) == hipSuccess);
+    };
+    if (!upload(&b->d_jobs, tiled) || !upload(&b->d_jobsD, tiledD) ||
+        hipMalloc((void **)&b->d_prefix, sizeof(int) * 9 * (b->nJobs + 1)) != hipSuccess ||
         hipMalloc((void **)&b->d_queue, kBatchQueueBytes) != hipSuccess)
-        return fail("tcv_batch_create: allocation failed");
-    if (hipMemcpy(b->d_jobs, b->host.data(), sizeof(JobDesc) * nJobs, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(b->d_jobsD, b->hostD.data(), sizeof(JobDesc) * nJobs, hipMemcpyHostToDevice) != hipSuccess)
-        return fail("tcv_batch_create: upload failed");
+        return fail("tcv_batch_create: allocation or upload failed");
+    for (int r = 0; r < 2; ++r) {
+        b->nNarrow[r] = (int)narrow[r].size();
+        if (b->nNarrow[r] && !upload(&b->d_narrow[r], narrow[r]))
+            return fail("tcv_batch_create: allocation or upload failed");
+    }
     *out = b;
     return TCV_OK;
 }
@@ -954,6 +1102,8 @@ tcv_status tcv_batch_destroy(tcv_ctx *ctx, tcv_batch *b)
     (void)hipFree(b->d_jobsD);
     (void)hipFree(b->d_prefix);
     (void)hipFree(b->d_queue);
+    for (JobDesc *d : b->d_narrow)
+        if (d) (void)hipFree(d);
     delete b;
     return TCV_OK;
 }
@@ -1181,6 +1331,9 @@ tcv_status tcv_autotune(tcv_ctx *ctx, const tcv_geometry *g, const float *d_data
             t.chunk = ch;
             if ((st = consider(t)) != TCV_OK) return st;
         }
+        // the open tuning: narrower kernels by regions
+        if (minS <= kClasses[1].width && (st = consider(tcv_tuning{0, 0, 0, 0, 0, -1, 0, 0, 0, 0, 0, 0})) != TCV_OK)
+            return st;
     }
     if (!any) return tcv_fail(ctx, TCV_ERR_UNSUPPORTED, "tcv_autotune: no candidate could be planned");
     if (bestMs) *bestMs = bestT;

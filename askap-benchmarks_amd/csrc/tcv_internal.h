@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -80,6 +81,9 @@ struct GeomDev {
     int sUniform;      // kernel width when wPlane == nullptr
     int gSize;
     long long cSize;
+    // binning takes the visibilities of widths [sLo, sHi] and, when countBad is
+    // set, counts the out-of-range ones
+    int sLo = 0, sHi = 0x7fffffff, countBad = 1;
 };
 
 // Launchers implemented in tcv_kernels.hip.  All enqueue on ctx->stream.
@@ -125,6 +129,7 @@ struct JobDesc {
     // entry's is above cEdgeHi, may hold entries on the table's first or last
     // slice (entries are ordered by C-slice key within an item)
     int cEdgeLo, cEdgeHi;
+    int strideW, strideH;       // grid columns and rows from one tile (or region) to the next
     // 1 when another job of the same launch grids into an overlapping grid: a
     // work item that holds a tile alone then still flushes with atomics
     int sharedGrid;
@@ -133,8 +138,6 @@ struct JobDesc {
 constexpr int kMaxPersistentBlocks = 8192;
 // Work-queue heads, one to a 128-byte line: atomics on one line are served one
 // after the other (12 ns each, measured), whichever of its words they go to.
-// With the eight heads of a plan on one line, spectral-scale gridding (8.4 M
-// visibilities, width 129) took 60.6 ms and degridding 53.4; apart 58.0 and 49.7.
 constexpr int kHeadInts = 32;
 constexpr int kMetaInts = 32 + 8 * kHeadInts;   // a plan's meta block (see tcv_plan::meta)
 constexpr size_t kBatchQueueBytes = 9 * kHeadInts * sizeof(int);   // the queue, then one head per XCD
@@ -158,6 +161,11 @@ struct PlanShape {
     int tapBytes;          // stored tap size the tuning was chosen for (8 or 4)
     int itemEntries;       // entries per work item the automatic phase counts aimed at
     int gridCols;          // pair gridder: columns per load instruction (tcv_tuning.grid_cols)
+    // narrow-kernel plans (tcv_narrow.hip): cells a side of the regions, which
+    // overlap so that each footprint lies in one; 0: tiles of tw x th
+    int region;
+    int bw, bh;            // stride of the tiles or regions (tw, th for tiles)
+    int sLo, sHi;          // kernel widths the plan bins
     int nTX, nTY, nTiles;
     int maxS;
     long long maxEntries;  // upper bound on visibility x tile pairs
@@ -192,26 +200,35 @@ struct tcv_plan {
     GeomDev geom{};               // geometry of the last build (for batch rebuilds)
     bool hasGeom = false;
     void *block = nullptr;        // one device block holding every buffer above
+    char *blockEnd = nullptr;     // one past the last buffer in it
     bool ownsBlock = false;       // block from hipMalloc (else from a caller's arena)
+    // plans of further classes of kernel widths (by regions), in the same block
+    std::vector<std::unique_ptr<tcv_plan>> parts;
 };
 
 // Plan memory as one block: plan_setup fills the shape and returns the bytes
 // needed for geometry g; plan_bind carves the buffers out of such a block.
+// tilesOnly: no narrow-kernel regions (batches and servers run tiles).
 tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tuning, tcv_plan *p,
-                      size_t *bytes);
+                      size_t *bytes, bool tilesOnly = false);
 void plan_bind(tcv_plan *p, char *block);
 // Whether the plan bins in two levels (by tile in LDS, then by key per tile):
 // the tile histogram must fit the LDS binning kernel and the per-tile key
 // histogram one workgroup's LDS.
 bool plan_two_level(const PlanShape &sh);
 
+constexpr int kRegions[] = {32, 48};   // region sizes built (cells a side)
+
 struct tcv_batch {
-    int nJobs = 0;
+    int nJobs = 0;      // jobs that have tiles: d_jobs, d_jobsD
     int tw = 0, th = 0, kern = kDefaultGridKernel, dkern = kDefaultDegridKernel;
     int gridCols = 0;   // pair gridder column groups (PlanShape::gridCols of every plan)
     bool half = false;
     std::vector<JobDesc> host, hostD;   // gridder / degridder descriptors
     std::vector<tcv_plan *> plans;
+    // the jobs' parts by regions, one list per region size
+    JobDesc *d_narrow[2] = {nullptr, nullptr};
+    int nNarrow[2] = {0, 0};
     JobDesc *d_jobs = nullptr, *d_jobsD = nullptr;
     int *d_prefix = nullptr;      // 9 x (nJobs + 1): item prefix, then one per XCD
     int *d_queue = nullptr;       // kBatchQueueBytes: the queue and the per-XCD counters
@@ -236,6 +253,10 @@ tcv_status launch_grid_tiled(tcv_ctx *ctx, tcv_plan *p, const void *data, const 
                              float2 *grid, const HalfStorage *half);
 tcv_status launch_degrid_tiled(tcv_ctx *ctx, tcv_plan *p, const float2 *grid, const void *C,
                                float2 *out, const HalfStorage *half);
+// Narrow-kernel regions (tcv_narrow.hip): a job's launch, and one for the jobs of
+// a batch with regions of one size.
+tcv_status launch_narrow(tcv_ctx *ctx, const JobDesc &jd, int region, bool half, bool degrid);
+tcv_status launch_narrow_many(tcv_ctx *ctx, const JobDesc *d_jobs, int nJobs, int region, bool degrid);
 // one persistent launch over every job of the batch (prefix sum computed on the device)
 tcv_status launch_batch(tcv_ctx *ctx, tcv_batch *b, bool degrid);
 // attic C(w) taps in FP64 on the device, normalised by the FP64 sum of |C|

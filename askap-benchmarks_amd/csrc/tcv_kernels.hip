@@ -15,84 +15,10 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "tcv_device.h"
 #include "tcv_internal.h"
 
 namespace {
-
-constexpr unsigned kOOB = 0x80000000u;  // byte offset beyond any C buffer we accept
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, unsigned bytes)
-{
-    // word3 0x00020000: raw 32-bit buffer format used for untyped loads on gfx9.
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00020000);
-}
-
-// Load of wave-uniform data that no wave writes while the kernel runs (work
-// items, entries, visibilities, plane scales).  Through the constant address
-// space the compiler issues a scalar (SMEM) load into SGPRs, instead of a
-// vector load, a wait for it and readfirstlane.
-template <typename T>
-__device__ __forceinline__ T cload(const T *p, int i)
-{
-#if defined(__HIP_DEVICE_COMPILE__)
-    return ((const __attribute__((address_space(4))) T *)p)[i];
-#else
-    return p[i];   // the host pass only parses device functions
-#endif
-}
-
-// a * b for 0 <= a, b < 2^24, b wave-uniform: the full-rate 24-bit multiply,
-// written as the instruction so that the compiler cannot fold it into a
-// neighbouring expression as a quarter-rate 32- or 64-bit multiply
-__device__ __forceinline__ int umul24(int a, int b)
-{
-    int r;
-    asm("v_mul_u32_u24 %0, %1, %2" : "=v"(r) : "s"(b), "v"(a));
-    return r;
-}
-
-// a * b + c (24-bit unsigned a, b; b wave-uniform)
-__device__ __forceinline__ unsigned umad24(int a, int b, unsigned c)
-{
-    unsigned r;
-    asm("v_mad_u32_u24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
-    return r;
-}
-
-// a * b + c (24-bit signed a, b; b wave-uniform)
-__device__ __forceinline__ unsigned imad24(int a, int b, unsigned c)
-{
-    unsigned r;
-    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
-    return r;
-}
-
-__device__ __forceinline__ float2 load_c(__amdgpu_buffer_rsrc_t r, unsigned voff)
-{
-    return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0));
-}
-
-
-// Sum over the 64 lanes of a wave (all lanes must be active).  Four DPP
-// steps reduce each 16-lane row; four readlanes combine the rows.  The result
-// is wave-uniform.
-__device__ __forceinline__ float wave_sum(float x)
-{
-    auto dpp = [](float v, auto ctrl) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-            0, __builtin_bit_cast(int, v), decltype(ctrl)::value, 0xF, 0xF, false));
-    };
-    x += dpp(x, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
-    x += dpp(x, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
-    x += dpp(x, std::integral_constant<int, 0x141>{});  // row_half_mirror
-    x += dpp(x, std::integral_constant<int, 0x140>{});  // row_mirror
-    const int xi = __builtin_bit_cast(int, x);
-    const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 0));
-    const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 16));
-    const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 32));
-    const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(xi, 48));
-    return (r0 + r1) + (r2 + r3);
-}
 
 // ---- fill (graph-safe zeroing) ------------------------------------------------
 
@@ -232,6 +158,7 @@ __global__ __launch_bounds__(256) void k_offsets(
 struct VisGeom {
     int s, u0, v0, c0;
     bool ok;
+    bool mine;   // of the widths this binning takes
 };
 
 __device__ __forceinline__ VisGeom vis_geom(const GeomDev &g, int d)
@@ -256,6 +183,7 @@ __device__ __forceinline__ VisGeom vis_geom(const GeomDev &g, int d)
          r.v0 + s <= g.gSize && r.c0 >= 0 &&
          (long long)r.c0 + (long long)s * s <= g.cSize;
     r.ok = ok;
+    r.mine = s >= g.sLo && s <= g.sHi;
     return r;
 }
 
@@ -480,7 +408,8 @@ __global__ __launch_bounds__(SCAN_BS) void k_scan_apply(const int *__restrict__ 
 // ---- tiled path: plan kernels -------------------------------------------------
 
 struct PlanDevArgs {
-    int tw, th, nTX, k2, phases, chunk, nTiles, xcd;
+    int tw, th, nTX, k2, phases, chunk, nTiles, xcd;   // tw, th: the stride of the tiles or regions
+    int single;   // regions: a footprint belongs to the one its first cell falls on
     long long cSize;
 };
 
@@ -499,6 +428,38 @@ __device__ __forceinline__ void note_c_range(int cLo, int cHi, int *meta)
     }
 }
 
+// The C-slice key of an entry of a region plan: its place within the cOffset
+// range that the plan's visibilities use (k_plan_range), in k2 equal parts.
+// (Keys of the whole table would put a class of narrow kernels, which uses a
+// small part of it, into one or two keys: entries of different widths would
+// follow each other, and all would count in the same few counters.)
+struct KeyRange {
+    int lo;
+    double scale;
+};
+__device__ __forceinline__ KeyRange key_range(const int *meta, int k2)
+{
+    const int lo = (int)(0x7fffffffu - (unsigned)meta[4]), hi = meta[5] - 1;
+    return KeyRange{lo, (double)k2 / (double)max(1, hi + 1 - lo)};
+}
+__device__ __forceinline__ int range_key(const KeyRange &r, int c0, int k2)
+{
+    return min((int)((double)(c0 - r.lo) * r.scale), k2 - 1);
+}
+
+// Notes the used cOffset range of a region plan ahead of its binning.
+__global__ __launch_bounds__(256) void k_plan_range(GeomDev g, int *__restrict__ meta)
+{
+    int cLo = 0x7fffffff, cHi = -1;
+    for (int d = blockIdx.x * blockDim.x + threadIdx.x; d < g.nVis; d += gridDim.x * blockDim.x) {
+        const VisGeom vg = vis_geom(g, d);
+        if (!vg.ok || !vg.mine) continue;
+        cLo = min(cLo, vg.c0);
+        cHi = max(cHi, vg.c0);
+    }
+    note_c_range(cLo, cHi, meta);
+}
+
 // pass 0 counts (tile, slice-key) buckets; pass 1 scatters the entries.
 // A visibility with footprint [u0, u0+s) x [v0, v0+s) is entered once in every
 // tile its footprint overlaps.  Entry = {u0 | v0 << 16, cOffset, vis, s}.
@@ -514,12 +475,13 @@ __global__ __launch_bounds__(256) void k_plan_bin(int pass, GeomDev g, PlanDevAr
     if (d < g.nVis) {
         const VisGeom vg = vis_geom(g, d);
         if (!vg.ok) {
-            isBad = 1;
-        } else {
+            isBad = g.countBad;
+        } else if (vg.mine) {
             cLo = cHi = vg.c0;
-            const int key2 = (int)(((long long)vg.c0 * a.k2) / a.cSize);
-            const int tx0 = vg.u0 / a.tw, tx1 = (vg.u0 + vg.s - 1) / a.tw;
-            const int ty0 = vg.v0 / a.th, ty1 = (vg.v0 + vg.s - 1) / a.th;
+            const int key2 = a.single ? range_key(key_range(meta, a.k2), vg.c0, a.k2)
+                                      : (int)(((long long)vg.c0 * a.k2) / a.cSize);
+            const int tx0 = vg.u0 / a.tw, tx1 = a.single ? tx0 : (vg.u0 + vg.s - 1) / a.tw;
+            const int ty0 = vg.v0 / a.th, ty1 = a.single ? ty0 : (vg.v0 + vg.s - 1) / a.th;
             const int plane = g.wPlane ? g.wPlane[d] : 0;
             const int4 ent = make_int4(vg.u0 | (vg.v0 << 16), vg.c0, d, vg.s | (plane << 16));
             for (int ty = ty0; ty <= ty1; ++ty)
@@ -537,7 +499,7 @@ __global__ __launch_bounds__(256) void k_plan_bin(int pass, GeomDev g, PlanDevAr
     if (pass == 0) {
         const int nb = __builtin_popcountll(__ballot(isBad));
         if ((threadIdx.x & 63) == 0 && nb) atomicAdd(&meta[3], nb);
-        note_c_range(cLo, cHi, meta);
+        if (!a.single) note_c_range(cLo, cHi, meta);
     }
 }
 
@@ -570,14 +532,15 @@ __global__ __launch_bounds__(256) void k_plan_bin_lds(int pass, GeomDev g, PlanD
         if (d >= g.nVis) break;
         const VisGeom vg = vis_geom(g, d);
         if (!vg.ok) {
-            isBad++;
+            isBad += g.countBad;
             continue;
         }
+        if (!vg.mine) continue;
         cLo = min(cLo, vg.c0);
         cHi = max(cHi, vg.c0);
         const int key2 = (int)(((long long)vg.c0 * a.k2) / a.cSize);
-        const int tx0 = vg.u0 / a.tw, tx1 = (vg.u0 + vg.s - 1) / a.tw;
-        const int ty0 = vg.v0 / a.th, ty1 = (vg.v0 + vg.s - 1) / a.th;
+        const int tx0 = vg.u0 / a.tw, tx1 = a.single ? tx0 : (vg.u0 + vg.s - 1) / a.tw;
+        const int ty0 = vg.v0 / a.th, ty1 = a.single ? ty0 : (vg.v0 + vg.s - 1) / a.th;
         for (int ty = ty0; ty <= ty1; ++ty)
             for (int tx = tx0; tx <= tx1; ++tx) atomicAdd(&hist[(ty * a.nTX + tx) * a.k2 + key2], 1);
     }
@@ -599,10 +562,10 @@ __global__ __launch_bounds__(256) void k_plan_bin_lds(int pass, GeomDev g, PlanD
         const int d = base + r * blockDim.x + threadIdx.x;
         if (d >= g.nVis) break;
         const VisGeom vg = vis_geom(g, d);
-        if (!vg.ok) continue;
+        if (!vg.ok || !vg.mine) continue;
         const int key2 = (int)(((long long)vg.c0 * a.k2) / a.cSize);
-        const int tx0 = vg.u0 / a.tw, tx1 = (vg.u0 + vg.s - 1) / a.tw;
-        const int ty0 = vg.v0 / a.th, ty1 = (vg.v0 + vg.s - 1) / a.th;
+        const int tx0 = vg.u0 / a.tw, tx1 = a.single ? tx0 : (vg.u0 + vg.s - 1) / a.tw;
+        const int ty0 = vg.v0 / a.th, ty1 = a.single ? ty0 : (vg.v0 + vg.s - 1) / a.th;
         const int plane = g.wPlane ? g.wPlane[d] : 0;
         const int4 ent = make_int4(vg.u0 | (vg.v0 << 16), vg.c0, d, vg.s | (plane << 16));
         for (int ty = ty0; ty <= ty1; ++ty)
@@ -621,7 +584,8 @@ __global__ __launch_bounds__(256) void k_plan_bin_lds(int pass, GeomDev g, PlanD
 __global__ __launch_bounds__(256) void k_plan_tile_keys(PlanDevArgs a, const int *__restrict__ tileStart,
                                                         const int4 *__restrict__ tmp,
                                                         int4 *__restrict__ entries,
-                                                        int *__restrict__ starts)
+                                                        int *__restrict__ starts,
+                                                        const int *__restrict__ meta)
 {
     extern __shared__ int lds[];
     int *hist = lds, *cur = lds + a.k2;
@@ -629,8 +593,8 @@ __global__ __launch_bounds__(256) void k_plan_tile_keys(PlanDevArgs a, const int
     const int b = tileStart[t], e = tileStart[t + 1];
     // key = floor(cOffset * k2 / cSize) up to rounding: monotone in cOffset and
     // computed the same way in both passes (an FP64 product, no division)
-    const double scale = (double)a.k2 / (double)a.cSize;
-    auto key_of = [&](int c0) { return min((int)((double)c0 * scale), a.k2 - 1); };
+    const KeyRange kr = a.single ? key_range(meta, a.k2) : KeyRange{0, (double)a.k2 / (double)a.cSize};
+    auto key_of = [&](int c0) { return range_key(kr, c0, a.k2); };
     for (int k = threadIdx.x; k < a.k2; k += blockDim.x) hist[k] = 0;
     __syncthreads();
     for (int i = b + threadIdx.x; i < e; i += blockDim.x) atomicAdd(&hist[key_of(tmp[i].y)], 1);
@@ -680,7 +644,7 @@ __global__ __launch_bounds__(256) void k_plan_items(int pass, PlanDevArgs a,
     const int id = a.xcd ? ((p & 7) * (a.phases >> 3) + (p >> 3)) * a.nTiles + t : gid;
     const int cLo = (int)(0x7fffffffu - (unsigned)meta[4]), cHi = meta[5] - 1;
     int kLo = 0, kHi = a.k2 - 1;
-    if (cLo <= cHi) {
+    if (cLo <= cHi && !a.single) {
         const double scale = (double)a.k2 / (double)a.cSize;
         auto keyDiv = [&](int c) { return (int)(((long long)c * a.k2) / a.cSize); };
         auto keyMul = [&](int c) { return min((int)((double)c * scale), a.k2 - 1); };
@@ -708,7 +672,7 @@ __global__ __launch_bounds__(256) void k_plan_items(int pass, PlanDevArgs a,
 
 // meta: [0] items [1] queue head [2] entries [3] out of range [4..5] cOffset range
 //       [16..24] per-XCD item ranges (XCD-major plans), [32 + kHeadInts q] per-XCD
-//       queue heads
+//       queue heads (the binning cleared them)
 __global__ void k_plan_meta(const int *__restrict__ itemStart, int nItemSlots,
                             const int *__restrict__ starts, long long nKeys, int xcdSlots,
                             int *__restrict__ meta)
@@ -717,7 +681,6 @@ __global__ void k_plan_meta(const int *__restrict__ itemStart, int nItemSlots,
         meta[0] = itemStart[nItemSlots];
         meta[1] = 0;
         meta[2] = starts[nKeys];
-        for (int x = 0; x < 8; ++x) meta[32 + kHeadInts * x] = 0;
         for (int x = 0; x <= 8; ++x)
             meta[16 + x] = xcdSlots ? itemStart[x * xcdSlots] : (x ? meta[0] : 0);
     }
@@ -727,206 +690,6 @@ __global__ void k_reset_queue(int *meta)
 {
     if (threadIdx.x < 8) meta[32 + kHeadInts * threadIdx.x] = 0;
     if (threadIdx.x == 0) meta[1] = 0;
-}
-
-// ---- tap storage ---------------------------------------------------------------
-// FP32: complex64 taps (8 B).  FP16: (re, im) half pairs (4 B) scaled by the
-// max-abs of their w-plane; accumulation stays FP32.
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-
-template <bool HALF>
-struct Taps;
-
-template <>
-struct Taps<false> {
-    static constexpr unsigned kBytes = 8;
-    __device__ static __forceinline__ float2 load(__amdgpu_buffer_rsrc_t r, unsigned voff)
-    {
-        return load_c(r, voff);
-    }
-};
-
-template <>
-struct Taps<true> {
-    static constexpr unsigned kBytes = 4;
-    __device__ static __forceinline__ float2 load(__amdgpu_buffer_rsrc_t r, unsigned voff)
-    {
-        const half2_t h = __builtin_bit_cast(half2_t, __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0));
-        return make_float2((float)h.x, (float)h.y);
-    }
-};
-
-// Two consecutive taps (one 16-byte load for FP32, 8 bytes for FP16): the
-// vector memory path moves data per group of four lanes, so wider loads carry
-// twice the taps per unit of L1 throughput.
-template <bool HALF>
-__device__ __forceinline__ float4 load_pair(__amdgpu_buffer_rsrc_t r, unsigned voff)
-{
-    if constexpr (!HALF) {
-        return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
-    } else {
-        const uint2 u = __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0));
-        const half2_t a = __builtin_bit_cast(half2_t, u.x), b = __builtin_bit_cast(half2_t, u.y);
-        return make_float4((float)a.x, (float)a.y, (float)b.x, (float)b.y);
-    }
-}
-
-// Four consecutive FP16 taps in one 16-byte load.
-struct Quad {
-    float2 t0, t1, t2, t3;
-};
-
-__device__ __forceinline__ float2 half_tap(unsigned w)
-{
-    const half2_t h = __builtin_bit_cast(half2_t, w);
-    return make_float2((float)h.x, (float)h.y);
-}
-
-__device__ __forceinline__ Quad load_quad_half(__amdgpu_buffer_rsrc_t r, unsigned voff)
-{
-    const uint4 u = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
-    return Quad{half_tap(u.x), half_tap(u.y), half_tap(u.z), half_tap(u.w)};
-}
-
-// a or b by a lane-dependent flag, as a bit blend: a plain select of two
-// struct members can be rewritten by the compiler into an indexed load from
-// the stack, which would put the quadruples in scratch memory
-__device__ __forceinline__ float blend(bool pickB, float a, float b)
-{
-    const unsigned m = 0u - (unsigned)pickB;
-    return __uint_as_float((__float_as_uint(a) & ~m) | (__float_as_uint(b) & m));
-}
-
-// tap i of a quadruple for a lane-dependent i in [0, 4)
-__device__ __forceinline__ float2 pick4(const Quad &q, int i)
-{
-    const bool lo = i & 1, hi = i & 2;
-    const float ax = blend(lo, q.t0.x, q.t1.x), ay = blend(lo, q.t0.y, q.t1.y);
-    const float bx = blend(lo, q.t2.x, q.t3.x), by = blend(lo, q.t2.y, q.t3.y);
-    return make_float2(blend(hi, ax, bx), blend(hi, ay, by));
-}
-
-__device__ __forceinline__ int entry_width(int w) { return w & 0xFFFF; }
-__device__ __forceinline__ int entry_plane(const int4 &en, const JobDesc &d)
-{
-    return d.planeTaps > 0 ? en.y / d.planeTaps : (int)((unsigned)en.w >> 16);
-}
-
-template <bool HALF>
-__device__ __forceinline__ float2 vis_value(const JobDesc &d, const int4 &en)
-{
-    if constexpr (!HALF) {
-        if (!d.data) return make_float2(1.f, 0.f);   // PSF gridding: data == 1 + 0i
-        return cload(static_cast<const float2 *>(d.data), en.z);
-    } else {
-        const half2_t v = cload(static_cast<const half2_t *>(d.data), en.z);
-        const float sc = d.dataScale * cload(d.planeScale, entry_plane(en, d));
-        return make_float2((float)v.x * sc, (float)v.y * sc);
-    }
-}
-
-// Work-item source of the persistent kernels: one job (descriptor passed by
-// value) or a batch (descriptors in device memory, located through the
-// exclusive prefix sum of the jobs' item counts).
-template <bool BATCH>
-struct ItemSource {
-    JobDesc one;
-    const JobDesc *jobs;
-    const int *prefix;
-    int nJobs;
-    int *queue;
-
-    // Single job: items are XCD-major with per-XCD queues.  Batch: each XCD
-    // walks its share of every job in job order (per-XCD prefix sums after the
-    // job prefix, counters at queue[kHeadInts (1 + q)]), then takes from the others.
-    int xcd;
-    int *bcast;   // one slot per workgroup (kernels that keep LDS for their tile)
-
-    __device__ __forceinline__ int total() const
-    {
-        if constexpr (BATCH) return __builtin_amdgcn_readfirstlane(prefix[nJobs]);
-        else return __builtin_amdgcn_readfirstlane(one.meta[0]);
-    }
-    // next work item (one lane calls this); >= total() when none is left
-    __device__ __forceinline__ int acquire() const
-    {
-        if (!xcd) return (int)gridDim.x + atomicAdd(queue, 1);   // after the workgroups' first items
-        // own XCD first (hardware XCC_ID register), then steal from the others
-        const int x0 = (int)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 7);
-        if constexpr (BATCH) {
-            const int n1 = nJobs + 1;
-            for (int k = 0; k < 8; ++k) {
-                const int q = (x0 + k) & 7;
-                const int *px = prefix + n1 * (1 + q);
-                const int tot = px[nJobs];
-                if (tot == 0) continue;
-                const int i = atomicAdd(queue + kHeadInts * (1 + q), 1);
-                if (i >= tot) continue;
-                int lo = 0, hi = nJobs;   // px[lo] <= i < px[hi]
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (px[mid] <= i) lo = mid; else hi = mid;
-                }
-                return prefix[lo] + jobs[lo].meta[16 + q] + (i - px[lo]);
-            }
-            return 0x7fffffff;
-        }
-        for (int k = 0; k < 8; ++k) {
-            const int q = (x0 + k) & 7;
-            const int b = one.meta[16 + q], e = one.meta[17 + q];
-            if (b >= e) continue;
-            const int i = atomicAdd(one.meta + 32 + kHeadInts * q, 1);
-            if (b + i < e) return b + i;
-        }
-        return 0x7fffffff;
-    }
-    // item -> (job descriptor, local item index); wave-uniform
-    __device__ __forceinline__ void locate(int item, JobDesc &d, int &local) const
-    {
-        if constexpr (BATCH) {
-            int lo = 0, hi = nJobs;   // prefix[lo] <= item < prefix[hi]
-            while (hi - lo > 1) {
-                const int mid = (lo + hi) >> 1;
-                if (__builtin_amdgcn_readfirstlane(prefix[mid]) <= item) lo = mid; else hi = mid;
-            }
-            d = jobs[lo];
-            local = item - __builtin_amdgcn_readfirstlane(prefix[lo]);
-        } else {
-            d = one;
-            local = item;
-        }
-    }
-};
-
-// Next work item for the whole workgroup without spending LDS: thread 0
-// publishes the item it acquired during the previous one (`next`, taken from
-// the queue one item ahead so that the queue's latency overlaps the work) in
-// the workgroup's slot and acquires the following one.  Waiting for its memory
-// counters completes the store in the CU's L2 before the barrier (a
-// device-scope fence would also write back the L2), and the waves, all on the
-// same CU, read the slot from that L2.  The caller reaches another barrier
-// before thread 0 publishes again, so no wave can miss a value.  Every item
-// acquired is processed: the loop ends on the first one past the end.
-template <bool BATCH>
-__device__ __forceinline__ int acquire_for_block(const ItemSource<BATCH> &src, int &next, int nItems)
-{
-    if (threadIdx.x == 0) {
-        __hip_atomic_store(src.bcast + blockIdx.x, next, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __builtin_amdgcn_s_waitcnt(0);   // every counter of this wave drained
-    }
-    __syncthreads();
-    const int item = __builtin_amdgcn_readfirstlane(
-        __hip_atomic_load(src.bcast + blockIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    if (threadIdx.x == 0 && item < nItems) next = src.acquire();
-    return item;
-}
-
-// The first item of a workgroup (thread 0 only; see acquire_for_block).  The single
-// queue starts after the workgroups' first items, which are their own numbers.
-template <bool BATCH>
-__device__ __forceinline__ int first_item(const ItemSource<BATCH> &src)
-{
-    return threadIdx.x != 0 ? 0 : src.xcd ? src.acquire() : (int)blockIdx.x;
 }
 
 // The TW x TH grid tile at (Bx, By) into LDS (a workgroup of 256 threads),
@@ -2300,11 +2063,12 @@ static tcv_status scan_exclusive(tcv_ctx *ctx, const int *in, int *out, long lon
     return TCV_OK;
 }
 
-tcv_status plan_build_kernels(tcv_ctx *ctx, tcv_plan *p, const GeomDev &g)
+static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
 {
     const PlanShape &sh = p->sh;
-    PlanDevArgs a{sh.tw, sh.th, sh.nTX, sh.k2, sh.phases, sh.chunk, sh.nTiles, sh.xcd, g.cSize};
-    ProfScope ps(ctx, "plan");
+    g.sLo = sh.sLo;
+    g.sHi = sh.sHi;
+    PlanDevArgs a{sh.bw, sh.bh, sh.nTX, sh.k2, sh.phases, sh.chunk, sh.nTiles, sh.xcd, sh.region > 0, g.cSize};
     tcv_status st;
     if ((st = launch_fill_u32(ctx, p->counts, 0, (size_t)sh.nKeys + 1)) != TCV_OK) return st;
     if ((st = launch_fill_u32(ctx, p->meta, 0, kMetaInts)) != TCV_OK) return st;
@@ -2346,9 +2110,14 @@ tcv_status plan_build_kernels(tcv_ctx *ctx, tcv_plan *p, const GeomDev &g)
         }
         hipLaunchKernelGGL(k_plan_tile_keys, dim3(sh.nTiles), dim3(256), (size_t)2 * sh.k2 * sizeof(int),
                            ctx->stream, a, (const int *)tileStart, (const int4 *)p->entriesTmp,
-                           p->entries, p->starts);
+                           p->entries, p->starts, (const int *)p->meta);
         TCV_HIP(ctx, hipGetLastError());
     } else {
+        if (sh.region > 0 && g.nVis > 0) {
+            hipLaunchKernelGGL(k_plan_range, dim3(std::min((g.nVis + 255) / 256, ctx->cus * 4)), dim3(256), 0,
+                               ctx->stream, g, p->meta);
+            TCV_HIP(ctx, hipGetLastError());
+        }
         if ((st = bin(0)) != TCV_OK) return st;
         if ((st = scan_exclusive(ctx, p->counts, p->starts, sh.nKeys, p->scanTmp)) != TCV_OK)
             return st;
@@ -2388,6 +2157,16 @@ tcv_status plan_build_kernels(tcv_ctx *ctx, tcv_plan *p, const GeomDev &g)
             return st;
     }
     return TCV_OK;
+}
+
+tcv_status plan_build_kernels(tcv_ctx *ctx, tcv_plan *p, const GeomDev &g)
+{
+    ProfScope ps(ctx, "plan");
+    tcv_status st = plan_build_one(ctx, p, g);
+    GeomDev n = g;
+    n.countBad = 0;   // counted by the first
+    for (size_t i = 0; st == TCV_OK && i < p->parts.size(); ++i) st = plan_build_one(ctx, p->parts[i].get(), n);
+    return st;
 }
 
 // ---- tiled launch dispatch ----------------------------------------------------
@@ -2570,6 +2349,8 @@ JobDesc make_job_desc(const tcv_plan *p, bool forGrid, const void *data, const v
     d.planeScale = half ? half->planeScale : nullptr;
     d.cBytes = (unsigned)(p->cSize * (half ? 4 : 8));
     d.nTX = p->sh.nTX;
+    d.strideW = p->sh.bw;
+    d.strideH = p->sh.bh;
     d.gSize = p->gSize;
     d.planeTaps = half ? half->planeTaps : 0;
     d.dataScale = half ? half->dataScale : 1.f;
@@ -2584,6 +2365,13 @@ JobDesc make_job_desc(const tcv_plan *p, bool forGrid, const void *data, const v
 tcv_status launch_grid_tiled(tcv_ctx *ctx, tcv_plan *p, const void *data, const void *C,
                              float2 *grid, const HalfStorage *half)
 {
+    for (auto &q : p->parts) {
+        tcv_status st = launch_grid_tiled(ctx, q.get(), data, C, grid, half);
+        if (st != TCV_OK) return st;
+    }
+    if (p->sh.region > 0)
+        return launch_narrow(ctx, make_job_desc(p, true, data, C, grid, nullptr, half), p->sh.region,
+                             half != nullptr, false);
     ItemSource<false> src{make_job_desc(p, true, data, C, grid, nullptr, half), nullptr, nullptr, 0,
                           p->metaG + 1, p->sh.xcdG, ctx->d_bcast};
     hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, ctx->stream, p->metaG);
@@ -2609,6 +2397,13 @@ tcv_status launch_degrid_tiled(tcv_ctx *ctx, tcv_plan *p, const float2 *grid, co
                           nullptr, nullptr, 0, p->meta + 1, p->sh.xcd, ctx->d_bcast};
     tcv_status st = launch_fill_u32(ctx, out, 0, (size_t)p->nVis * 2);
     if (st != TCV_OK) return st;
+    for (auto &q : p->parts) {
+        // results stored into the cleared output, beside those the tiles add up
+        st = launch_narrow(ctx, make_job_desc(q.get(), false, nullptr, C, const_cast<float2 *>(grid), out, half),
+                           q->sh.region, half != nullptr, true);
+        if (st != TCV_OK) return st;
+    }
+    if (p->sh.region > 0) return launch_narrow(ctx, src.one, p->sh.region, half != nullptr, true);
     hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, ctx->stream, p->meta);
     TCV_HIP(ctx, hipGetLastError());
     // the FP16 four-tap degridder needs kernel widths of at least 4
@@ -2631,6 +2426,12 @@ tcv_status launch_batch(tcv_ctx *ctx, tcv_batch *b, bool degrid)
             tcv_status st = launch_fill_u32(ctx, d.out, 0, (size_t)d.nVis * 2);
             if (st != TCV_OK) return st;
         }
+    for (int r = 0; r < 2; ++r) {
+        if (!b->nNarrow[r]) continue;
+        tcv_status st = launch_narrow_many(ctx, b->d_narrow[r], b->nNarrow[r], kRegions[r], degrid);
+        if (st != TCV_OK) return st;
+    }
+    if (!b->nJobs) return TCV_OK;
     hipLaunchKernelGGL(k_batch_prefix, dim3(1), dim3(64), 0, ctx->stream,
                        (const JobDesc *)(degrid ? b->d_jobsD : b->d_jobs), b->nJobs, b->d_prefix,
                        b->d_queue);

@@ -67,7 +67,7 @@ extern "C" tcv_status tcv_grid_noalloc(tcv_ctx *ctx, const tcv_geometry *g, cons
     for (int keys = 2048;; keys /= 2) {
         p = tcv_plan{};
         const tcv_tuning t{0, 0, 0, keys, 0, -1, 0, 0, 0, 0, 0, 0};
-        tcv_status st = plan_setup(ctx, g, &t, &p, &bytes);
+        tcv_status st = plan_setup(ctx, g, &t, &p, &bytes, true);
         if (st != TCV_OK) return st;
         if (bytes <= TCV_NOALLOC_SCRATCH_BYTES || keys == 1) break;
     }

@@ -264,6 +264,10 @@ typedef struct {
                         64 on 128-wide tiles, else tile_w */
 } tcv_tuning;
 
+/* A tuning with every field open but tap_bytes and item_entries takes kernels up
+ * to 31 wide by overlapping regions of 32 or 48 cells a side that one wave
+ * grids or degrids (a job of widths 20 to 31 only, when it has at most 8192
+ * visibilities or at least 8 to a region), wider ones by tiles. */
 typedef struct tcv_plan tcv_plan;
 
 /* Allocates a plan for jobs of this geometry class (device buffers sized from

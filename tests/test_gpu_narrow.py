@@ -1,0 +1,168 @@
+"""Plans that take narrow kernels by regions: every width that a region size is
+built for (steps of the walk, odd and even, the widest of a class), grids that
+no region divides, the first and last slices of the table, widths mixed with
+wider ones, FP16 storage and batches.  Taps are multiples of 1/4 and values
+small integers, so every sum is exact and results equal the oracle's."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle as O
+import tcv
+
+pytestmark = pytest.mark.gpu
+
+
+def job(seed, widths, nVis, gSize, os_=2):
+    """Exact inputs with plane k of width widths[k]; the last visibilities lie on
+    the table's first and last slices, at the grid's corners."""
+    rng = np.random.default_rng(seed)
+    w = np.asarray(widths, np.int32)
+    size = w.astype(np.int64) ** 2 * os_ * os_
+    start = np.concatenate([[0], np.cumsum(size)])
+    plane = rng.integers(0, w.size, nVis).astype(np.int32)
+    plane[-4:] = (0, 0, w.size - 1, w.size - 1)
+    s = w[plane]
+    cell = rng.integers(0, os_ * os_, nVis)
+    cell[-4:] = (0, 0, os_ * os_ - 1, os_ * os_ - 1)
+    co = (start[plane] + cell * s * s).astype(np.int32)
+    half = s // 2
+    u0 = (rng.random(nVis) * (gSize - s + 1)).astype(np.int32)
+    v0 = (rng.random(nVis) * (gSize - s + 1)).astype(np.int32)
+    u0[-4:], v0[-4:] = (0, gSize - s[-3], 0, gSize - s[-1]), (0, gSize - s[-3], gSize - s[-2], 0)
+    cplx = lambda n, d: ((rng.integers(-4, 5, n) + 1j * rng.integers(-4, 5, n)) / d).astype(np.complex64)
+    return dict(w=w, plane=plane, co=co, iu=u0 + half, iv=v0, C=cplx(int(start[-1]), 4),
+                data=cplx(nVis, 1), grid=cplx(gSize * gSize, 1).reshape(gSize, gSize), gSize=gSize)
+
+
+def visibilities(ctx, j):
+    up = ctx.to_device
+    return tcv.Visibilities(ctx, up(j["iu"]), up(j["iv"]), up(j["co"]), j["w"], j["gSize"], j["C"].size,
+                            wPlane=up(j["plane"]))
+
+
+def reference(j):
+    pick = np.asarray([k for k in range(j["iu"].size) if j.get("ok") is None or j["ok"][k]])
+    args = j["iu"][pick], j["iv"][pick], j["co"][pick], j["C"]
+    g = O.grid(j["data"][pick], *args, j["gSize"], j["w"], wPlane=j["plane"][pick])
+    o = np.zeros(j["iu"].size, np.complex64)
+    o[pick] = O.degrid(j["grid"], *args, j["w"], wPlane=j["plane"][pick])
+    return g, o
+
+
+def run(ctx, plan, j):
+    g = ctx.zeros((j["gSize"], j["gSize"]), np.complex64)
+    plan.grid(ctx.to_device(j["data"]), ctx.to_device(j["C"]), g)
+    out = ctx.empty(j["iu"].size, np.complex64)
+    plan.degrid(ctx.to_device(j["grid"]), ctx.to_device(j["C"]), out)
+    return g.download(), out.download()
+
+
+@pytest.mark.parametrize("widths,nVis,gSize", [
+    ([2], 700, 33), ([3, 4], 2000, 65), ([5], 1, 7), ([7, 9, 8], 3000, 257), ([10, 11], 1500, 64),
+    ([12, 15], 2500, 127), ([16], 1025, 96), ([17, 18, 19], 4000, 200), ([19], 129, 19),
+    ([20, 21], 600, 61), ([22, 23], 3000, 130), ([24, 27], 2000, 255), ([28, 31], 2500, 100), ([30], 65, 30),
+    ([2, 9, 14, 19, 20, 31], 5000, 150), ([9, 19, 25, 40, 63], 4000, 201), ([7, 97], 2000, 300),
+    ([21, 33], 1500, 128)])
+def test_regions_equal_oracle(ctx, widths, nVis, gSize):
+    j = job(sum(widths) + nVis, widths, max(nVis, 4) if nVis > 1 else 4, gSize)
+    if nVis == 1:
+        for k in ("plane", "co", "iu", "iv", "data"):
+            j[k] = j[k][-1:]
+    gref, oref = reference(j)
+    plan = tcv.Plan(ctx, visibilities(ctx, j))
+    for _ in range(2):
+        g, o = run(ctx, plan, j)
+        assert np.array_equal(g, gref)
+        assert np.array_equal(o, oref)
+        plan.build()
+    # the same through tiles
+    tiles = tcv.Plan(ctx, visibilities(ctx, j), slice_keys=16)
+    g, o = run(ctx, tiles, j)
+    assert np.array_equal(g, gref) and np.array_equal(o, oref)
+
+
+def test_regions_out_of_range(ctx):
+    j = job(5, [9, 25, 65], 900, 140)
+    j["iu"][:3], j["iv"][3:6], j["co"][6:9] = 0, 139, j["C"].size
+    j["ok"] = np.arange(900) >= 9
+    plan = tcv.Plan(ctx, visibilities(ctx, j))
+    g, o = run(ctx, plan, j)
+    gref, oref = reference(j)
+    assert np.array_equal(g, gref) and np.array_equal(o, oref)
+    assert plan.info()["out_of_range"] == 9
+
+
+def test_regions_half_storage(ctx):
+    """FP16 holds these values exactly, up to the power-of-two scales."""
+    j = job(6, [9, 18, 31, 33], 1200, 110, os_=2)
+    starts = np.concatenate([[0], np.cumsum(j["w"].astype(np.int64) ** 2 * 4)])
+    Ch = tcv.HalfTable(ctx, ctx.to_device(j["C"]), 4, 0, starts)
+    dh = tcv.HalfVis(ctx, ctx.to_device(j["data"]))
+    plan = tcv.Plan(ctx, visibilities(ctx, j), tap_bytes=4)
+    gref, oref = reference(j)
+    g = ctx.zeros((110, 110), np.complex64)
+    plan.grid_half(dh, Ch, g)
+    out = ctx.empty(1200, np.complex64)
+    plan.degrid_half(ctx.to_device(j["grid"]), Ch, out)
+    # a stored value is within 2^-12 of itself and FP32 sums add 1e-6: both cells
+    # and results are sums whose terms' magnitudes bound the error
+    bound = lambda x: 2.5 * 2.0 ** -12 * x + 1e-4
+    mag = O.grid(np.full(1200, 8, np.complex64), j["iu"], j["iv"], j["co"],
+                 np.full(j["C"].size, 2, np.complex64), 110, j["w"], wPlane=j["plane"]).real
+    assert (np.abs(g.download() - gref) <= bound(mag)).all()
+    assert (np.abs(out.download() - oref) <= bound(16.0 * j["w"][j["plane"]] ** 2)).all()
+
+
+def test_regions_keep_non_finite_values_inside(ctx):
+    """An infinite tap, value or cell shows in what it belongs to and nowhere else."""
+    for s in (9, 25):
+        j = job(7 + s, [s], 300, 90)
+        n = s * s
+        j["co"][:] = np.where(j["co"] == 3 * n, 2 * n, j["co"])   # nobody's slice: all infinite
+        j["C"][3 * n:] = np.inf
+        j["iu"] = np.minimum(j["iu"], 90 - s - 1 + s // 2)   # nor the last column of the grid
+        j["grid"][:, 89] = np.nan
+        gref, oref = reference(j)
+        plan = tcv.Plan(ctx, visibilities(ctx, j))
+        g, o = run(ctx, plan, j)
+        assert np.array_equal(g, gref) and np.array_equal(o, oref)
+        j["data"][0] = np.inf
+        g, _ = run(ctx, plan, j)
+        x, y = j["iu"][0] - s // 2, j["iv"][0]
+        out = np.ones((90, 90), bool)
+        out[y:y + s, x:x + s] = False
+        assert np.array_equal(g[out], gref[out]) and not np.isfinite(g[~out]).any()
+
+
+def test_regions_in_a_batch(ctx):
+    """Automatic plans in a batch: jobs by regions, in part and by tiles alone; two
+    of them share a grid."""
+    from tcv.device import Batch
+    jobs = [job(11, [17, 19], 1500, 120), job(12, [31, 16], 900, 120), job(13, [8, 12, 19], 700, 77),
+            job(14, [15], 5000, 250)]
+    jobs.append(job(15, [9, 40], 800, 130))
+    plans = [tcv.Plan(ctx, visibilities(ctx, j), tile_w=16 if j is jobs[0] else 0) for j in jobs]
+    with pytest.raises(tcv.TcvError):   # tile shapes differ, as for plans without regions
+        Batch(ctx, [(p, ctx.to_device(j["data"]), ctx.to_device(j["C"]),
+                     ctx.zeros((j["gSize"],) * 2, np.complex64), None) for p, j in zip(plans, jobs)])
+    for pick in ([0, 2, 3], [1], [2, 3], [1, 4]):
+        hold = []
+        for k in pick:
+            j = jobs[k]
+            hold.append((plans[k], ctx.to_device(j["data"]), ctx.to_device(j["C"]),
+                         ctx.zeros((j["gSize"],) * 2, np.complex64), ctx.empty(j["iu"].size, np.complex64)))
+        b = Batch(ctx, hold)
+        for _ in range(3):
+            for h, k in zip(hold, pick):
+                h[3].zero()
+            b.run_graph(3)
+            for h, k in zip(hold, pick):
+                assert np.array_equal(h[3].download(), reference(jobs[k])[0]), k
+        for h, k in zip(hold, pick):
+            h[3].upload(jobs[k]["grid"])
+        b.degrid()
+        for h, k in zip(hold, pick):
+            assert np.array_equal(h[4].download(), reference(jobs[k])[1]), k
+        b.close()
