@@ -209,38 +209,52 @@ struct ItemSource {
         if constexpr (BATCH) return __builtin_amdgcn_readfirstlane(prefix[nJobs]);
         else return __builtin_amdgcn_readfirstlane(one.meta[0]);
     }
-    // next work item (one lane calls this); >= total() when none is left
+    // XCD q's share of the items and its i-th item
+    __device__ __forceinline__ int share(int q) const
+    {
+        if constexpr (BATCH) return prefix[(nJobs + 1) * (1 + q) + nJobs];
+        else return one.meta[17 + q] - one.meta[16 + q];
+    }
+    __device__ __forceinline__ int item_of(int q, int i) const
+    {
+        if constexpr (BATCH) {
+            const int *px = prefix + (nJobs + 1) * (1 + q);
+            int lo = 0, hi = nJobs;   // px[lo] <= i < px[hi]
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (px[mid] <= i) lo = mid; else hi = mid;
+            }
+            return prefix[lo] + jobs[lo].meta[16 + q] + (i - px[lo]);
+        } else {
+            return one.meta[16 + q] + i;
+        }
+    }
+    // Next work item (one lane calls this); >= total() when none is left.  The
+    // queues start after the workgroups' first items (first_item), so a list of
+    // no more items than workgroups takes no atomics (378 items, 1024 workgroups:
+    // gridding 85 us with, 74 without).
     __device__ __forceinline__ int acquire() const
     {
-        if (!xcd) return (int)gridDim.x + atomicAdd(queue, 1);   // after the workgroups' first items
+        if (!xcd) return (int)gridDim.x + atomicAdd(queue, 1);
         // own XCD first (hardware XCC_ID register), then steal from the others
         const int x0 = (int)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 7);
-        if constexpr (BATCH) {
-            const int n1 = nJobs + 1;
-            for (int k = 0; k < 8; ++k) {
-                const int q = (x0 + k) & 7;
-                const int *px = prefix + n1 * (1 + q);
-                const int tot = px[nJobs];
-                if (tot == 0) continue;
-                const int i = atomicAdd(queue + kHeadInts * (1 + q), 1);
-                if (i >= tot) continue;
-                int lo = 0, hi = nJobs;   // px[lo] <= i < px[hi]
-                while (hi - lo > 1) {
-                    const int mid = (lo + hi) >> 1;
-                    if (px[mid] <= i) lo = mid; else hi = mid;
-                }
-                return prefix[lo] + jobs[lo].meta[16 + q] + (i - px[lo]);
-            }
-            return 0x7fffffff;
-        }
         for (int k = 0; k < 8; ++k) {
             const int q = (x0 + k) & 7;
-            const int b = one.meta[16 + q], e = one.meta[17 + q];
-            if (b >= e) continue;
-            const int i = atomicAdd(one.meta + 32 + kHeadInts * q, 1);
-            if (b + i < e) return b + i;
+            const int tot = share(q), taken = ((int)gridDim.x + 7 - q) >> 3;
+            if (tot <= taken) continue;
+            int *head = BATCH ? queue + kHeadInts * (1 + q) : one.meta + 32 + kHeadInts * q;
+            const int i = taken + atomicAdd(head, 1);
+            if (i < tot) return item_of(q, i);
         }
         return 0x7fffffff;
+    }
+    // A workgroup's first item: its own number, or its place in the share of the XCD
+    // that workgroups are dealt to in turn (any other deal costs locality alone).
+    __device__ __forceinline__ int first() const
+    {
+        if (!xcd) return (int)blockIdx.x;
+        const int q = blockIdx.x & 7, i = blockIdx.x >> 3;
+        return i < share(q) ? item_of(q, i) : acquire();
     }
     // item -> (job descriptor, local item index); wave-uniform
     __device__ __forceinline__ void locate(int item, JobDesc &d, int &local) const
@@ -283,12 +297,11 @@ __device__ __forceinline__ int acquire_for_block(const ItemSource<BATCH> &src, i
     return item;
 }
 
-// The first item of a workgroup (thread 0 only; see acquire_for_block).  The single
-// queue starts after the workgroups' first items, which are their own numbers.
+// The first item of a workgroup (thread 0 only; see acquire_for_block).
 template <bool BATCH>
 __device__ __forceinline__ int first_item(const ItemSource<BATCH> &src)
 {
-    return threadIdx.x != 0 ? 0 : src.xcd ? src.acquire() : (int)blockIdx.x;
+    return threadIdx.x == 0 ? src.first() : 0;
 }
 
 }  // namespace

@@ -569,11 +569,6 @@ constexpr WidthClass kClasses[] = {{19, 32, 128}, {31, 48, 64}};
 // 102 + 92 + 89 -> 48 + 86 + 38; 64 000 132 + 127 + 115 -> 74 + 387 + 142;
 // 500 000 401 + 670 + 488 -> 189 + 733 + 338.
 constexpr int kSmallJob = 8192, kDenseRegion = 8;
-// Entries of the tiles' work items beside regions: the few wide visibilities
-// left fill no long ones (widths 7-121 above: 2842 + 1827 with 1024, 2022 + 1450
-// with 128, 2116 + 1480 with 512; 500 000 visibilities 1102 + 795 and 537 + 444).
-constexpr int kRestChunk = 128;
-
 // Array sizes that follow from a plan's shape, and the bytes of its buffers.
 static tcv_status plan_sizes(tcv_ctx *ctx, const tcv_geometry *g, tcv_plan *p, size_t *bytes);
 
@@ -592,6 +587,7 @@ static tcv_status region_setup(tcv_ctx *ctx, const tcv_geometry *g, int R, int c
     sh.nTiles = sh.nTX * sh.nTY;
     sh.phases = sh.phasesG = 1;
     sh.xcd = sh.xcdG = 0;
+    sh.adapt = 0;
     sh.chunk = chunk;
     // C-slice keys: enough to keep neighbouring entries on neighbouring slices,
     // but no more (region, key) counters than about two a visibility
@@ -645,8 +641,12 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
                 tilesLo = c.width + 1;
             }
         if (parts.empty()) tilesLo = 0;
-        else t.chunk = kRestChunk;
     }
+    // Work items sized on the device where every choice is open.  A plan with a
+    // tile shape given (batches give one) keeps the host's counts: among other jobs'
+    // items its own need no cutting (19 jobs of 5000-61 000 visibilities 11.2 ms,
+    // cut 11.9).
+    const bool adapt = !tilesOnly && open_shape(t) && t.item_entries <= 0;
     auto_tuning(maxS, g, &t);
     if (!tiled_config_supported(t.tile_w, t.tile_h))
         return tcv_fail(ctx, TCV_ERR_UNSUPPORTED, "tile shape not built");
@@ -665,6 +665,13 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
     sh.xcd = (t.xcd_split > 0 && sh.phases % 8 == 0) ? 1 : 0;
     sh.phasesG = std::min(t.grid_phases, sh.k2);
     sh.xcdG = (t.xcd_split > 0 && sh.phasesG % 8 == 0) ? 1 : 0;
+    sh.adapt = adapt;
+    if (adapt) {
+        sh.phaseBytes = t.tile_w * t.tile_h > 4096 ? kWidePhaseBytes : kDegridPhaseBytes;
+        sh.phases = sh.phasesG = std::max(1, default_phases(g->cSize, t.tap_bytes, sh.k2, g, maxS, t.tile_w, t.tile_h,
+                                                            sh.phaseBytes, kAdaptSlotEntries));
+        sh.xcd = sh.xcdG = 1;
+    }
     if (t.kernel < 1 || t.kernel > 4 || t.degrid_kernel < 1 || t.degrid_kernel > 4)
         return tcv_fail(ctx, TCV_ERR_INVALID, "tuning.kernel and degrid_kernel must be 0..4");
     sh.kern = t.kernel;
@@ -726,6 +733,12 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
     return st;
 }
 
+// Entries that a job of footprints of the widest kernel makes on average.
+static double entries_expected(const tcv_geometry *g, const PlanShape &sh)
+{
+    return g->nVis * (1.0 + (sh.maxS - 1.0) / sh.tw) * (1.0 + (sh.maxS - 1.0) / sh.th);
+}
+
 static tcv_status plan_sizes(tcv_ctx *ctx, const tcv_geometry *g, tcv_plan *p, size_t *bytes)
 {
     PlanShape &sh = p->sh;
@@ -733,8 +746,11 @@ static tcv_status plan_sizes(tcv_ctx *ctx, const tcv_geometry *g, tcv_plan *p, s
     if (sh.maxEntries >= 0x7fffffffLL || sh.nKeys >= 0x7fffffffLL)
         return tcv_fail(ctx, TCV_ERR_UNSUPPORTED, "plan too large for 32-bit entry indices");
     p->maxItems = sh.maxEntries / sh.chunk + (long long)sh.phases * sh.nTiles + 1;
-    const bool twoLists = sh.phasesG != sh.phases || sh.xcdG != sh.xcd;
-    p->maxItemsG = twoLists ? sh.maxEntries / sh.chunk + (long long)sh.phasesG * sh.nTiles + 1 : 0;
+    // chunks below sh.chunk hold n / kAdaptItems entries, rounded down, or kAdaptChunk
+    if (sh.adapt) p->maxItems += kAdaptItems + kAdaptItems / 16;
+    const bool twoLists = sh.adapt ? sh.phases > 1 && entries_expected(g, sh) > kAdaptItems * kAdaptChunk
+                                   : sh.phasesG != sh.phases || sh.xcdG != sh.xcd;
+    p->maxItemsG = twoLists ? p->maxItems - (long long)(sh.phases - sh.phasesG) * sh.nTiles : 0;
     const long long slotsG = (long long)sh.phasesG * sh.nTiles;
     const long long slots = (long long)sh.phases * sh.nTiles;
     p->scanTmpLen = std::max(scan_tmp_len(sh.nKeys), std::max(scan_tmp_len(slots), scan_tmp_len(slotsG)));
@@ -903,7 +919,7 @@ tcv_status tcv_plan_info(tcv_ctx *ctx, tcv_plan *p, tcv_tuning *t, long long *en
     if (t) *t = tcv_tuning{p->sh.tw, p->sh.th, p->sh.chunk, p->sh.k2, p->sh.phases, p->sh.xcd, p->sh.kern,
                            p->sh.dkern, p->sh.phasesG, p->sh.tapBytes, p->sh.itemEntries,
                            p->sh.gridCols};
-    int meta[4] = {0, 0, 0, 0};   // items, queue head, entries, out of range
+    int meta[12] = {0};   // items, queue head, entries, out of range, ..., [9] phases [10] chunk
     TCV_HIP(ctx, hipMemcpyAsync(meta, p->meta, sizeof(meta), hipMemcpyDeviceToHost, ctx->stream));
     TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
     for (auto &part : p->parts) {
@@ -912,6 +928,14 @@ tcv_status tcv_plan_info(tcv_ctx *ctx, tcv_plan *p, tcv_tuning *t, long long *en
         TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
         meta[0] += more[0];
         meta[2] += more[2];
+    }
+    if (t && p->sh.adapt) {
+        t->phases = t->grid_phases = meta[9];
+        t->chunk = meta[10];
+        if (p->metaG != p->meta) {
+            TCV_HIP(ctx, hipMemcpyAsync(&t->grid_phases, p->metaG + 9, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+            TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        }
     }
     if (items) *items = meta[0];
     if (entries) *entries = meta[2];

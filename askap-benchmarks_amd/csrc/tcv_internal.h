@@ -142,6 +142,13 @@ constexpr int kHeadInts = 32;
 constexpr int kMetaInts = 32 + 8 * kHeadInts;   // a plan's meta block (see tcv_plan::meta)
 constexpr size_t kBatchQueueBytes = 9 * kHeadInts * sizeof(int);   // the queue, then one head per XCD
 
+// Work items that the build sizes on the device: about kAdaptItems of them and no
+// fewer than kAdaptChunk entries each; C-slice phases leave kAdaptGrid entries to
+// a tile and phase on average, kAdaptDegrid for degridding.  kAdaptSlotEntries
+// bounds the (phase, tile) slots allocated, for entries spread over the whole grid.
+constexpr int kAdaptItems = 8192, kAdaptChunk = 32, kAdaptGrid = 56, kAdaptDegrid = 12;
+constexpr double kAdaptSlotEntries = 8;
+
 // Tiled kernels used when a tuning leaves the choice open.  Gridder: 1 tile in
 // registers, 2 tile in LDS, 3 registers with two columns per lane.  Degridder:
 // 1 registers, 2 LDS, 3 LDS with tap pairs.
@@ -166,6 +173,10 @@ struct PlanShape {
     int region;
     int bw, bh;            // stride of the tiles or regions (tw, th for tiles)
     int sLo, sHi;          // kernel widths the plan bins
+    // 1: the build chooses phases and chunk on the device (cut_of in tcv_kernels.hip),
+    // up to the counts here
+    int adapt;
+    double phaseBytes;     // taps a phase then spans
     int nTX, nTY, nTiles;
     int maxS;
     long long maxEntries;  // upper bound on visibility x tile pairs
@@ -188,6 +199,7 @@ struct tcv_plan {
     int *itemStart = nullptr;     // phases * nTiles + 1
     int *meta = nullptr;          // kMetaInts: [0] items [1] queue head [2] entries [3] bad,
                                   // [4..5] the entries' cOffset range (see note_c_range),
+                                  // [8] tiles with entries [9] phases [10] chunk,
                                   // [16..24] per-XCD item ranges, [32 + kHeadInts q] per-XCD heads
     // the gridder's work items (phasesG); the same buffers as above when
     // phasesG == phases

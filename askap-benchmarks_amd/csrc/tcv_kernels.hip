@@ -411,6 +411,9 @@ struct PlanDevArgs {
     int tw, th, nTX, k2, phases, chunk, nTiles, xcd;   // tw, th: the stride of the tiles or regions
     int single;   // regions: a footprint belongs to the one its first cell falls on
     long long cSize;
+    int adapt;          // phases and chunk chosen by cut_of, up to those above
+    int minEntries;     // then: entries a tile and phase keep on average
+    double phaseTaps;   // then: taps a phase spans
 };
 
 // The cOffset range of the binned entries, for phases over the part of the
@@ -629,6 +632,59 @@ __global__ __launch_bounds__(256) void k_plan_tile_keys(PlanDevArgs a, const int
 // that part's size.  Keys are floor(cOffset * k2 / cSize) by an integer
 // division (one-level binning) or an FP64 product (two-level): both are
 // monotone in cOffset, and the range covers what either gives at its ends.
+//
+// An adaptive plan's phases span phaseTaps of the range in use, as far as that
+// leaves minEntries to the work items of a tile and phase (the tiles that have
+// entries, counted by k_plan_touched): the count follows the part of the table
+// and of the grid that the visibilities lie on, which only the device knows.
+// 160 000 visibilities of width 129 on a quarter of 4096^2 and half of a 281 MB
+// table, grid + degrid in us: 4 phases 2965 + 2692, 16 1875 + 1894, 32 1381 +
+// 1166, 64 1699 + 1096; the same in FP16: 4 1980 + 1874, 16 1164 + 989, 64 1610 +
+// 1087; 100 003 of width 63 over 2047^2: 4 597 + 553, 8 477 + 473, 16 528 + 409,
+// 32 935 + 373, 64 1638 + 478 (a gridder's item flushes its tile with atomics).
+//
+// The chunk makes about kAdaptItems items of at least kAdaptChunk entries, so
+// that a tile with many entries is shared out: 2000 visibilities of width 129 on
+// 32 tiles, 96 items 304 + 118 us, 464 items 71 + 41; 30 000 of one plane on 694
+// tiles 1394 + 776 with 2048, 235 + 138 with 32.  Where the slots alone are
+// enough, an ordinary slot isn't cut (100 003 of width 63: 523 against 477).
+struct Cut {
+    int phases, chunk;
+};
+__device__ __forceinline__ Cut cut_of(const PlanDevArgs &a, const int *starts, const int *meta)
+{
+    if (!a.adapt) return Cut{a.phases, a.chunk};
+    const int n = starts[(long long)a.nTiles * a.k2];
+    const int cLo = (int)(0x7fffffffu - (unsigned)meta[4]), cHi = meta[5] - 1;
+    double target = cLo <= cHi ? ((double)cHi - cLo + 1) / a.phaseTaps : 1.0;
+    const double tiles = max(1, meta[8]);
+    target = fmin(target, (double)n / (tiles * a.minEntries));
+    int ph = 1;
+    if (target >= 6) {
+        ph = max(8, (int)(target / 8.0 + 0.5) * 8);   // a multiple of 8: whole shares for the XCDs
+    } else {
+        while (ph * 2 <= target) ph *= 2;
+    }
+    ph = min(ph, a.phases);
+    int chunk = n / kAdaptItems;
+    const double slots = tiles * ph, each = n / slots;
+    if (slots >= kAdaptItems / 4) chunk = max(chunk, (int)fmin(4 * each, 512.0));
+    else if (slots >= kAdaptItems / 32 && each < 1.5 * kAdaptChunk) chunk = max(chunk, (int)(2 * each));
+    return Cut{ph, max(kAdaptChunk, min(a.chunk, chunk))};
+}
+
+// Counts the tiles that have entries.
+__global__ __launch_bounds__(256) void k_plan_touched(PlanDevArgs a, const int *__restrict__ starts,
+                                                      int *__restrict__ meta)
+{
+    int n = 0;
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < a.nTiles; t += gridDim.x * blockDim.x)
+        n += starts[(long long)(t + 1) * a.k2] > starts[(long long)t * a.k2];
+    int total;
+    (void)block_exclusive_scan(n, &total);
+    if (threadIdx.x == 0 && total) atomicAdd(&meta[8], total);
+}
+
 __global__ __launch_bounds__(256) void k_plan_items(int pass, PlanDevArgs a,
                                                     const int *__restrict__ starts,
                                                     int *__restrict__ itemCount,
@@ -638,10 +694,15 @@ __global__ __launch_bounds__(256) void k_plan_items(int pass, PlanDevArgs a,
 {
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= a.phases * a.nTiles) return;
+    const Cut cut = cut_of(a, starts, meta);
     const int p = gid / a.nTiles, t = gid - p * a.nTiles;
+    if (p >= cut.phases) {
+        if (pass == 0) itemCount[gid] = 0;
+        return;
+    }
     // XCD-major slot order: sub-range p goes to XCD p % 8, so each XCD's items
     // are contiguous and its L2 only sees its share of a phase's C slices
-    const int id = a.xcd ? ((p & 7) * (a.phases >> 3) + (p >> 3)) * a.nTiles + t : gid;
+    const int id = a.xcd && cut.phases % 8 == 0 ? ((p & 7) * (cut.phases >> 3) + (p >> 3)) * a.nTiles + t : gid;
     const int cLo = (int)(0x7fffffffu - (unsigned)meta[4]), cHi = meta[5] - 1;
     int kLo = 0, kHi = a.k2 - 1;
     if (cLo <= cHi && !a.single) {
@@ -652,37 +713,44 @@ __global__ __launch_bounds__(256) void k_plan_items(int pass, PlanDevArgs a,
         kHi = min(a.k2 - 1, max(keyDiv(cHi), keyMul(cHi)));
     }
     const long long span = kHi + 1 - kLo;
-    const int k0 = kLo + (int)((long long)p * span / a.phases);
-    const int k1 = kLo + (int)((long long)(p + 1) * span / a.phases);
+    const int k0 = kLo + (int)((long long)p * span / cut.phases);
+    const int k1 = kLo + (int)((long long)(p + 1) * span / cut.phases);
     const long long b0 = (long long)t * a.k2;
     const int s = starts[b0 + k0], e = starts[b0 + k1];
     const int n = e - s;
-    const int nc = (n + a.chunk - 1) / a.chunk;
+    const int nc = (n + cut.chunk - 1) / cut.chunk;
     if (pass == 0) {
         itemCount[id] = nc;
     } else {
-        const int excl = (a.phases == 1 && nc == 1) ? 1 : 0;
+        const int excl = (cut.phases == 1 && nc == 1) ? 1 : 0;
         const int o = itemStart[id];
         for (int k = 0; k < nc; ++k) {
-            const int f = s + k * a.chunk;
-            items[o + k] = make_int4(t, f, min(a.chunk, e - f), excl);
+            const int f = s + k * cut.chunk;
+            items[o + k] = make_int4(t, f, min(cut.chunk, e - f), excl);
         }
     }
 }
 
 // meta: [0] items [1] queue head [2] entries [3] out of range [4..5] cOffset range
+//       [8] tiles with entries [9] phases [10] chunk
 //       [16..24] per-XCD item ranges (XCD-major plans), [32 + kHeadInts q] per-XCD
 //       queue heads (the binning cleared them)
-__global__ void k_plan_meta(const int *__restrict__ itemStart, int nItemSlots,
-                            const int *__restrict__ starts, long long nKeys, int xcdSlots,
-                            int *__restrict__ meta)
+// src: the meta block of the binning, meta: the item list's (they may be one).
+__global__ void k_plan_meta(PlanDevArgs a, const int *__restrict__ itemStart, const int *__restrict__ starts,
+                            const int *src, int *meta)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
-        meta[0] = itemStart[nItemSlots];
+        const Cut cut = cut_of(a, starts, src);
+        const int n = itemStart[a.phases * a.nTiles];
+        meta[0] = n;
         meta[1] = 0;
-        meta[2] = starts[nKeys];
+        meta[2] = starts[(long long)a.nTiles * a.k2];
+        meta[9] = cut.phases;
+        meta[10] = cut.chunk;
+        // without whole shares of phases: one range, or (adaptive plans) equal ones
+        const int share = a.xcd && cut.phases % 8 == 0 ? cut.phases / 8 * a.nTiles : 0;
         for (int x = 0; x <= 8; ++x)
-            meta[16 + x] = xcdSlots ? itemStart[x * xcdSlots] : (x ? meta[0] : 0);
+            meta[16 + x] = share ? itemStart[x * share] : a.adapt ? (int)((long long)n * x / 8) : x ? n : 0;
     }
 }
 
@@ -2068,7 +2136,8 @@ static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
     const PlanShape &sh = p->sh;
     g.sLo = sh.sLo;
     g.sHi = sh.sHi;
-    PlanDevArgs a{sh.bw, sh.bh, sh.nTX, sh.k2, sh.phases, sh.chunk, sh.nTiles, sh.xcd, sh.region > 0, g.cSize};
+    PlanDevArgs a{sh.bw, sh.bh, sh.nTX, sh.k2, sh.phases, sh.chunk, sh.nTiles, sh.xcd, sh.region > 0,
+                  g.cSize, sh.adapt, kAdaptDegrid, sh.phaseBytes / sh.tapBytes};
     tcv_status st;
     if ((st = launch_fill_u32(ctx, p->counts, 0, (size_t)sh.nKeys + 1)) != TCV_OK) return st;
     if ((st = launch_fill_u32(ctx, p->meta, 0, kMetaInts)) != TCV_OK) return st;
@@ -2125,12 +2194,18 @@ static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
                                     hipMemcpyDeviceToDevice, ctx->stream));
         if ((st = bin(1)) != TCV_OK) return st;
     }
+    if (sh.adapt) {
+        hipLaunchKernelGGL(k_plan_touched, dim3(std::min((sh.nTiles + 255) / 256, 64)), dim3(256), 0, ctx->stream, a,
+                           (const int *)p->starts, p->meta);
+        TCV_HIP(ctx, hipGetLastError());
+    }
     // work items: cuts of the sorted entries into (phase, tile) ranges
-    auto items = [&](int phases, int xcd, int *itemCount, int *itemStart, int4 *itemsOut,
+    auto items = [&](int phases, int xcd, int minEntries, int *itemCount, int *itemStart, int4 *itemsOut,
                      int *meta) -> tcv_status {
         PlanDevArgs b = a;
         b.phases = phases;
         b.xcd = xcd;
+        b.minEntries = minEntries;
         const int slots = phases * sh.nTiles;
         hipLaunchKernelGGL(k_plan_items, dim3((slots + 255) / 256), dim3(256), 0, ctx->stream, 0,
                            b, p->starts, itemCount, (const int *)itemStart, itemsOut,
@@ -2142,18 +2217,19 @@ static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
                            b, p->starts, itemCount, (const int *)itemStart, itemsOut,
                            (const int *)p->meta);
         TCV_HIP(ctx, hipGetLastError());
-        hipLaunchKernelGGL(k_plan_meta, dim3(1), dim3(64), 0, ctx->stream, (const int *)itemStart,
-                           slots, (const int *)p->starts, sh.nKeys,
-                           xcd ? (phases / 8) * sh.nTiles : 0, meta);
+        hipLaunchKernelGGL(k_plan_meta, dim3(1), dim3(64), 0, ctx->stream, b, (const int *)itemStart,
+                           (const int *)p->starts, (const int *)p->meta, meta);
         TCV_HIP(ctx, hipGetLastError());
         return TCV_OK;
     };
-    if ((st = items(sh.phases, sh.xcd, p->itemCount, p->itemStart, p->items, p->meta)) != TCV_OK)
+    const bool two = p->metaG != p->meta;
+    if ((st = items(sh.phases, sh.xcd, two ? kAdaptDegrid : kAdaptGrid, p->itemCount, p->itemStart, p->items,
+                    p->meta)) != TCV_OK)
         return st;
-    if (p->metaG != p->meta) {
+    if (two) {
         // the out-of-range count lives in meta[3]; the gridder's meta gets its own copy
         if ((st = launch_fill_u32(ctx, p->metaG, 0, kMetaInts)) != TCV_OK) return st;
-        if ((st = items(sh.phasesG, sh.xcdG, p->itemCountG, p->itemStartG, p->itemsG, p->metaG)) != TCV_OK)
+        if ((st = items(sh.phasesG, sh.xcdG, kAdaptGrid, p->itemCountG, p->itemStartG, p->itemsG, p->metaG)) != TCV_OK)
             return st;
     }
     return TCV_OK;

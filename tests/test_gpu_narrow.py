@@ -166,3 +166,53 @@ def test_regions_in_a_batch(ctx):
         for h, k in zip(hold, pick):
             assert np.array_equal(h[4].download(), reference(jobs[k])[1]), k
         b.close()
+
+
+@pytest.mark.parametrize("Sz,gSize,nVis,cluster,os_,planes", [
+    (65, 200, 1, 0, 2, 2),            # one entry to a tile
+    (65, 1500, 700, 0, 2, 3),         # fewer items than workgroups, one phase
+    (129, 400, 2500, 60, 8, 5),       # few tiles: cut to chunks of 32
+    (97, 700, 9000, 0, 8, 9),         # phases, one list of work items
+    (63, 900, 70000, 0, 8, 33),       # two lists: finer phases for the degridder
+    (63, 600, 120000, 12, 4, 4)])     # hot tiles
+def test_adaptive_work_items(ctx, Sz, gSize, nVis, cluster, os_, planes):
+    """Phases and chunks chosen on the device: exact results, and as many work items
+    as a plan with the same numbers given makes."""
+    from helpers import small_problem
+    iu, iv, co, data, C = small_problem(Sz + nVis, nVis, gSize, Sz, os_=os_, nPlanes=planes, margin=1,
+                                        cluster=cluster or None)
+    rng = np.random.default_rng(nVis)
+    C = ((rng.integers(-1, 2, C.size) + 1j * rng.integers(-1, 2, C.size)) / 4).astype(np.complex64)
+    data = (rng.integers(-2, 3, nVis) + 1j * rng.integers(-2, 3, nVis)).astype(np.complex64)
+    grid = (rng.integers(-2, 3, (gSize, gSize)) + 1j * rng.integers(-2, 3, (gSize, gSize))).astype(np.complex64)
+    vis = tcv.Visibilities(ctx, iu, iv, co, [Sz], gSize, C.size)
+    gref, oref = O.grid(data, iu, iv, co, C, gSize, Sz), O.degrid(grid, iu, iv, co, C, Sz)
+    plan = tcv.Plan(ctx, vis)
+    d_data, d_C, d_grid = ctx.to_device(data), ctx.to_device(C), ctx.to_device(grid)
+    for _ in range(2):
+        g = ctx.zeros((gSize, gSize), np.complex64)
+        plan.grid(d_data, d_C, g)
+        out = ctx.empty(nVis, np.complex64)
+        plan.degrid(d_grid, d_C, out)
+        assert np.array_equal(g.download(), gref)
+        assert np.array_equal(out.download(), oref)
+        plan.build()
+    info = plan.info()
+    given = tcv.Plan(ctx, vis, **{k: info[k] for k in ("tile_w", "tile_h", "chunk", "slice_keys", "phases",
+                                                       "grid_phases", "kernel", "degrid_kernel")}).info()
+    assert (given["items"], given["entries"], given["phases"], given["chunk"]) == \
+        (info["items"], info["entries"], info["phases"], info["chunk"])
+
+
+def test_adaptive_plan_of_nothing(ctx):
+    """Every visibility out of range: no items, cleared results."""
+    vis = tcv.Visibilities(ctx, [1, 2], [0, 0], [0, 0], [65], 100, 65 * 65)
+    plan = tcv.Plan(ctx, vis)
+    info = plan.info()
+    assert (info["items"], info["entries"], info["out_of_range"]) == (0, 0, 2)
+    C = ctx.to_device(np.ones(65 * 65, np.complex64))
+    g = ctx.zeros((100, 100), np.complex64)
+    plan.grid(ctx.to_device(np.ones(2, np.complex64)), C, g)
+    out = ctx.to_device(np.ones(2, np.complex64))
+    plan.degrid(g, C, out)
+    assert not g.download().any() and not out.download().any()
