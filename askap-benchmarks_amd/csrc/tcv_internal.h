@@ -196,7 +196,7 @@ struct tcv_plan {
     int *starts = nullptr;        // nKeys + 1
     int *cursor = nullptr;        // nKeys
     int *itemCount = nullptr;     // phases * nTiles + 1
-    int *itemStart = nullptr;     // phases * nTiles + 1
+    int *itemStart = nullptr;     // phases * nTiles + 1: the item counts of blocks of slots, then those scanned
     int *meta = nullptr;          // kMetaInts: [0] items [1] queue head [2] entries [3] bad,
                                   // [4..5] the entries' cOffset range (see note_c_range),
                                   // [8] tiles with entries [9] phases [10] chunk,

@@ -346,9 +346,10 @@ constexpr int SCAN_BS = 256;
 constexpr int SCAN_IPT = 16;
 constexpr int SCAN_TILE = SCAN_BS * SCAN_IPT;
 
+template <int BS = SCAN_BS>
 __device__ __forceinline__ int block_exclusive_scan(int x, int *total)
 {
-    __shared__ int wsum[SCAN_BS / 64];
+    __shared__ int wsum[BS / 64];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     int incl = x;
 #pragma unroll
@@ -360,7 +361,7 @@ __device__ __forceinline__ int block_exclusive_scan(int x, int *total)
     __syncthreads();
     int before = 0, all = 0;
 #pragma unroll
-    for (int k = 0; k < SCAN_BS / 64; ++k) {
+    for (int k = 0; k < BS / 64; ++k) {
         const int t = wsum[k];
         if (k < wv) before += t;
         all += t;
@@ -383,23 +384,43 @@ __global__ __launch_bounds__(SCAN_BS) void k_scan_reduce(const int *__restrict__
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
+// The sum of the sums[] of the blocks before this one (every thread's).
+__device__ __forceinline__ int sums_before(const int *__restrict__ sums)
+{
+    int t = 0, total;
+    for (int k = threadIdx.x; k < (int)blockIdx.x; k += SCAN_BS) t += sums[k];
+    (void)block_exclusive_scan(t, &total);
+    return total;
+}
+
+// offs: the scanned block sums, or (raw) the sums as they are.  out2 takes a copy
+// of the n results; touched, when given, the number of inputs that aren't zero.
 __global__ __launch_bounds__(SCAN_BS) void k_scan_apply(const int *__restrict__ in, long long n,
-                                                        const int *__restrict__ offs,
-                                                        int *__restrict__ out)
+                                                        const int *__restrict__ offs, int raw,
+                                                        int *__restrict__ out, int *__restrict__ out2, int *touched)
 {
     const long long base = (long long)blockIdx.x * SCAN_TILE + (long long)threadIdx.x * SCAN_IPT;
     int vals[SCAN_IPT];
-    int t = 0;
+    int t = 0, some = 0;
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; ++k) {
         vals[k] = (base + k < n) ? in[base + k] : 0;
         t += vals[k];
+        some += vals[k] != 0;
     }
     int total;
-    int run = block_exclusive_scan(t, &total) + (offs ? offs[blockIdx.x] : 0);
+    if (touched) {
+        (void)block_exclusive_scan(some, &total);
+        if (threadIdx.x == 0 && total) atomicAdd(touched, total);
+    }
+    const int before = !offs ? 0 : raw ? sums_before(offs) : offs[blockIdx.x];
+    int run = block_exclusive_scan(t, &total) + before;
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; ++k) {
-        if (base + k < n) out[base + k] = run;
+        if (base + k < n) {
+            out[base + k] = run;
+            if (out2) out2[base + k] = run;
+        }
         run += vals[k];
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == SCAN_BS - 1) out[n] = run;
@@ -418,7 +439,9 @@ struct PlanDevArgs {
 
 // The cOffset range of the binned entries, for phases over the part of the
 // table in use: meta[4] = max(0x7fffffff - c0), meta[5] = max(c0 + 1), so the
-// zeroed counters read as an empty range.  One atomic pair per wave.
+// zeroed counters read as an empty range.  One atomic pair per wave, where the
+// wave widens the range: atomics on one address take 12 ns each, one after the
+// other (5.4 M visibilities, every wave of a first pass: 130 us of a 150 us pass).
 __device__ __forceinline__ void note_c_range(int cLo, int cHi, int *meta)
 {
     for (int o = 32; o > 0; o >>= 1) {
@@ -426,8 +449,11 @@ __device__ __forceinline__ void note_c_range(int cLo, int cHi, int *meta)
         cHi = max(cHi, __shfl_xor(cHi, o, 64));
     }
     if ((threadIdx.x & 63) == 0 && cHi >= 0) {
-        atomicMax(reinterpret_cast<unsigned *>(meta + 4), 0x7fffffffu - (unsigned)cLo);
-        atomicMax(reinterpret_cast<unsigned *>(meta + 5), (unsigned)cHi + 1u);
+        const unsigned lo = 0x7fffffffu - (unsigned)cLo, hi = (unsigned)cHi + 1u;
+        unsigned *m = reinterpret_cast<unsigned *>(meta + 4);
+        // (a value read too early is only lower: one atomic more)
+        if (lo > __hip_atomic_load(m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(m, lo);
+        if (hi > __hip_atomic_load(m + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(m + 1, hi);
     }
 }
 
@@ -507,15 +533,16 @@ __global__ __launch_bounds__(256) void k_plan_bin(int pass, GeomDev g, PlanDevAr
 }
 
 // The same binning with the (tile, key) histogram aggregated in LDS, for key
-// spaces that fit (nKeys <= kLdsKeys): each block takes kBinVPT visibilities
-// per thread, counts locally, and touches each global counter at most once
+// spaces that fit (nKeys <= kLdsKeys): each block takes `each` visibilities
+// per thread (up to kBinVPT; fewer where the blocks would not fill the chip:
+// 100 003 visibilities on 25 blocks took 24 + 37 us), counts locally, and touches each global counter at most once
 // (pass 0: add the block's count; pass 1: reserve the block's range, then place
 // entries at range start + LDS rank).  Cuts the global atomics on hot tile
 // counters by the number of visibilities per block.
 constexpr int kBinVPT = 16;
 constexpr int kLdsKeys = 6144;   // 2 x 6144 ints = 48 KB of LDS in pass 1
 
-__global__ __launch_bounds__(256) void k_plan_bin_lds(int pass, GeomDev g, PlanDevArgs a,
+__global__ __launch_bounds__(256) void k_plan_bin_lds(int pass, int each, GeomDev g, PlanDevArgs a,
                                                       int *__restrict__ counts,
                                                       int *__restrict__ cursor,
                                                       int4 *__restrict__ entries,
@@ -527,10 +554,10 @@ __global__ __launch_bounds__(256) void k_plan_bin_lds(int pass, GeomDev g, PlanD
     int *rank = lds + nKeys;
     for (int k = threadIdx.x; k < (pass ? 2 : 1) * nKeys; k += blockDim.x) lds[k] = 0;
     __syncthreads();
-    const int base = blockIdx.x * blockDim.x * kBinVPT;
+    const int base = blockIdx.x * blockDim.x * each;
     int isBad = 0;
     int cLo = 0x7fffffff, cHi = -1;
-    for (int r = 0; r < kBinVPT; ++r) {
+    for (int r = 0; r < each; ++r) {
         const int d = base + r * blockDim.x + threadIdx.x;
         if (d >= g.nVis) break;
         const VisGeom vg = vis_geom(g, d);
@@ -541,7 +568,7 @@ __global__ __launch_bounds__(256) void k_plan_bin_lds(int pass, GeomDev g, PlanD
         if (!vg.mine) continue;
         cLo = min(cLo, vg.c0);
         cHi = max(cHi, vg.c0);
-        const int key2 = (int)(((long long)vg.c0 * a.k2) / a.cSize);
+        const int key2 = a.k2 > 1 ? (int)(((long long)vg.c0 * a.k2) / a.cSize) : 0;
         const int tx0 = vg.u0 / a.tw, tx1 = a.single ? tx0 : (vg.u0 + vg.s - 1) / a.tw;
         const int ty0 = vg.v0 / a.th, ty1 = a.single ? ty0 : (vg.v0 + vg.s - 1) / a.th;
         for (int ty = ty0; ty <= ty1; ++ty)
@@ -561,12 +588,12 @@ __global__ __launch_bounds__(256) void k_plan_bin_lds(int pass, GeomDev g, PlanD
     for (int k = threadIdx.x; k < nKeys; k += blockDim.x)
         if (hist[k]) hist[k] = atomicAdd(&cursor[k], hist[k]);
     __syncthreads();
-    for (int r = 0; r < kBinVPT; ++r) {
+    for (int r = 0; r < each; ++r) {
         const int d = base + r * blockDim.x + threadIdx.x;
         if (d >= g.nVis) break;
         const VisGeom vg = vis_geom(g, d);
         if (!vg.ok || !vg.mine) continue;
-        const int key2 = (int)(((long long)vg.c0 * a.k2) / a.cSize);
+        const int key2 = a.k2 > 1 ? (int)(((long long)vg.c0 * a.k2) / a.cSize) : 0;
         const int tx0 = vg.u0 / a.tw, tx1 = a.single ? tx0 : (vg.u0 + vg.s - 1) / a.tw;
         const int ty0 = vg.v0 / a.th, ty1 = a.single ? ty0 : (vg.v0 + vg.s - 1) / a.th;
         const int plane = g.wPlane ? g.wPlane[d] : 0;
@@ -583,8 +610,10 @@ __global__ __launch_bounds__(256) void k_plan_bin_lds(int pass, GeomDev g, PlanD
 // tile's entries (grouped by tile by the first level, in `tmp`) by C-slice
 // key with an LDS counting sort, writes them to `entries` and the tile's key
 // offsets to starts[tile * k2 + key].  Block 0 also writes the total at
-// starts[nTiles * k2].
-__global__ __launch_bounds__(256) void k_plan_tile_keys(PlanDevArgs a, const int *__restrict__ tileStart,
+// starts[nTiles * k2].  Bound by the tile with the most entries: BS = 1024 for
+// large jobs, and four loads in flight a thread.
+template <int BS>
+__global__ __launch_bounds__(BS) void k_plan_tile_keys(PlanDevArgs a, const int *__restrict__ tileStart,
                                                         const int4 *__restrict__ tmp,
                                                         int4 *__restrict__ entries,
                                                         int *__restrict__ starts,
@@ -598,17 +627,24 @@ __global__ __launch_bounds__(256) void k_plan_tile_keys(PlanDevArgs a, const int
     // computed the same way in both passes (an FP64 product, no division)
     const KeyRange kr = a.single ? key_range(meta, a.k2) : KeyRange{0, (double)a.k2 / (double)a.cSize};
     auto key_of = [&](int c0) { return range_key(kr, c0, a.k2); };
-    for (int k = threadIdx.x; k < a.k2; k += blockDim.x) hist[k] = 0;
+    for (int k = threadIdx.x; k < a.k2; k += BS) hist[k] = 0;
     __syncthreads();
-    for (int i = b + threadIdx.x; i < e; i += blockDim.x) atomicAdd(&hist[key_of(tmp[i].y)], 1);
+    for (int i = b + threadIdx.x; i < e; i += 4 * BS) {
+        int c[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) c[k] = tmp[min(i + k * BS, e - 1)].y;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (i + k * BS < e) atomicAdd(&hist[key_of(c[k])], 1);
+    }
     __syncthreads();
     // exclusive scan of hist: each thread a run of consecutive keys
-    const int per = (a.k2 + blockDim.x - 1) / blockDim.x;
+    const int per = (a.k2 + BS - 1) / BS;
     const int k0 = min((int)threadIdx.x * per, a.k2), k1 = min(k0 + per, a.k2);
     int run = 0;
     for (int k = k0; k < k1; ++k) run += hist[k];
     int total;
-    int off = block_exclusive_scan(run, &total);
+    int off = block_exclusive_scan<BS>(run, &total);
     for (int k = k0; k < k1; ++k) {
         const int c = hist[k];
         cur[k] = off;
@@ -617,9 +653,13 @@ __global__ __launch_bounds__(256) void k_plan_tile_keys(PlanDevArgs a, const int
     }
     if (t == 0 && threadIdx.x == 0) starts[(long long)a.nTiles * a.k2] = tileStart[a.nTiles];
     __syncthreads();
-    for (int i = b + threadIdx.x; i < e; i += blockDim.x) {
-        const int4 ent = tmp[i];
-        entries[b + atomicAdd(&cur[key_of(ent.y)], 1)] = ent;
+    for (int i = b + threadIdx.x; i < e; i += 4 * BS) {
+        int4 ent[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) ent[k] = tmp[min(i + k * BS, e - 1)];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (i + k * BS < e) entries[b + atomicAdd(&cur[key_of(ent[k].y)], 1)] = ent[k];
     }
 }
 
@@ -685,73 +725,106 @@ __global__ __launch_bounds__(256) void k_plan_touched(PlanDevArgs a, const int *
     if (threadIdx.x == 0 && total) atomicAdd(&meta[8], total);
 }
 
-__global__ __launch_bounds__(256) void k_plan_items(int pass, PlanDevArgs a,
-                                                    const int *__restrict__ starts,
-                                                    int *__restrict__ itemCount,
-                                                    const int *__restrict__ itemStart,
-                                                    int4 *__restrict__ items,
-                                                    const int *__restrict__ meta)
+// Slots are (phase, tile) pairs in item order; list blockIdx.y of a plan has its own
+// (the gridder's and the degridder's).  Pass 0 counts a slot's items and a block's,
+// pass 1 writes them after those of the blocks before (summed here, or scanned
+// where there are many) and the list's meta:
+//       [0] items [1] queue head [2] entries [9] phases [10] chunk
+//       [16..24] per-XCD item ranges (XCD-major plans), [32 + kHeadInts q] per-XCD
+//       queue heads (cleared ahead of the binning)
+// src: the meta block of the binning: [3] out of range [4..5] cOffset range [8] tiles
+// with entries.
+struct ItemList {
+    int phases, xcd, minEntries;
+    int *count, *sums;
+    const int *scanned;   // pass 1: the sums scanned, or null
+    int4 *items;
+    int *meta;
+};
+struct ItemLists {
+    ItemList l[2];
+};
+__global__ __launch_bounds__(SCAN_BS) void k_plan_items(int pass, PlanDevArgs a, ItemLists lists,
+                                                        const int *__restrict__ starts, const int *src)
 {
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    if (gid >= a.phases * a.nTiles) return;
-    const Cut cut = cut_of(a, starts, meta);
-    const int p = gid / a.nTiles, t = gid - p * a.nTiles;
-    if (p >= cut.phases) {
-        if (pass == 0) itemCount[gid] = 0;
-        return;
-    }
+    const ItemList L = lists.l[blockIdx.y];
+    a.phases = L.phases;
+    a.minEntries = L.minEntries;
+    const int slots = a.phases * a.nTiles, nb = (slots + SCAN_BS - 1) / SCAN_BS;
+    if ((int)blockIdx.x >= nb) return;
+    const Cut cut = cut_of(a, starts, src);
+    const int id = blockIdx.x * SCAN_BS + threadIdx.x;
     // XCD-major slot order: sub-range p goes to XCD p % 8, so each XCD's items
     // are contiguous and its L2 only sees its share of a phase's C slices
-    const int id = a.xcd && cut.phases % 8 == 0 ? ((p & 7) * (cut.phases >> 3) + (p >> 3)) * a.nTiles + t : gid;
-    const int cLo = (int)(0x7fffffffu - (unsigned)meta[4]), cHi = meta[5] - 1;
-    int kLo = 0, kHi = a.k2 - 1;
-    if (cLo <= cHi && !a.single) {
-        const double scale = (double)a.k2 / (double)a.cSize;
-        auto keyDiv = [&](int c) { return (int)(((long long)c * a.k2) / a.cSize); };
-        auto keyMul = [&](int c) { return min((int)((double)c * scale), a.k2 - 1); };
-        kLo = max(0, min(keyDiv(cLo), keyMul(cLo)));
-        kHi = min(a.k2 - 1, max(keyDiv(cHi), keyMul(cHi)));
-    }
-    const long long span = kHi + 1 - kLo;
-    const int k0 = kLo + (int)((long long)p * span / cut.phases);
-    const int k1 = kLo + (int)((long long)(p + 1) * span / cut.phases);
-    const long long b0 = (long long)t * a.k2;
-    const int s = starts[b0 + k0], e = starts[b0 + k1];
-    const int n = e - s;
-    const int nc = (n + cut.chunk - 1) / cut.chunk;
-    if (pass == 0) {
-        itemCount[id] = nc;
-    } else {
-        const int excl = (cut.phases == 1 && nc == 1) ? 1 : 0;
-        const int o = itemStart[id];
-        for (int k = 0; k < nc; ++k) {
-            const int f = s + k * cut.chunk;
-            items[o + k] = make_int4(t, f, min(cut.chunk, e - f), excl);
+    const int each = L.xcd && cut.phases % 8 == 0 ? cut.phases >> 3 : 0;
+    int nc = 0, s = 0, e = 0, t = 0;
+    if (id < cut.phases * a.nTiles && (pass == 0 || (nc = L.count[id]) > 0)) {
+        const int q = id / a.nTiles, p = each ? (q % each) * 8 + q / each : q;
+        t = id - q * a.nTiles;
+        const int cLo = (int)(0x7fffffffu - (unsigned)src[4]), cHi = src[5] - 1;
+        int kLo = 0, kHi = a.k2 - 1;
+        if (cLo <= cHi && !a.single) {
+            const double scale = (double)a.k2 / (double)a.cSize;
+            auto keyDiv = [&](int c) { return (int)(((long long)c * a.k2) / a.cSize); };
+            auto keyMul = [&](int c) { return min((int)((double)c * scale), a.k2 - 1); };
+            kLo = max(0, min(keyDiv(cLo), keyMul(cLo)));
+            kHi = min(a.k2 - 1, max(keyDiv(cHi), keyMul(cHi)));
         }
+        const long long span = kHi + 1 - kLo;
+        const int k0 = kLo + (int)((long long)p * span / cut.phases);
+        const int k1 = kLo + (int)((long long)(p + 1) * span / cut.phases);
+        const long long b0 = (long long)t * a.k2;
+        s = starts[b0 + k0];
+        e = starts[b0 + k1];
+        nc = (e - s + cut.chunk - 1) / cut.chunk;
+    }
+    int total;
+    int o = block_exclusive_scan(nc, &total);
+    if (pass == 0) {
+        if (id < slots) L.count[id] = nc;
+        if (threadIdx.x == 0) L.sums[blockIdx.x] = total;
+        return;
+    }
+    const int before = L.scanned ? L.scanned[blockIdx.x] : sums_before(L.sums);
+    o += before;
+    const int excl = (cut.phases == 1 && nc == 1) ? 1 : 0;
+    for (int k = 0; k < nc; ++k) {
+        const int f = s + k * cut.chunk;
+        L.items[o + k] = make_int4(t, f, min(cut.chunk, e - f), excl);
+    }
+    const int share = each * a.nTiles;
+    if (share && id < 8 * share && id % share == 0) L.meta[16 + id / share] = o;
+    if ((int)blockIdx.x == nb - 1 && threadIdx.x == 0) {
+        const int n = before + total;
+        L.meta[0] = n;
+        L.meta[1] = 0;
+        L.meta[2] = starts[(long long)a.nTiles * a.k2];
+        L.meta[9] = cut.phases;
+        L.meta[10] = cut.chunk;
+        // without whole shares of phases: one range, or (adaptive plans) equal ones
+        for (int x = 0; x < 8 && !share; ++x) L.meta[16 + x] = a.adapt ? (int)((long long)n * x / 8) : x ? n : 0;
+        L.meta[24] = n;
     }
 }
 
-// meta: [0] items [1] queue head [2] entries [3] out of range [4..5] cOffset range
-//       [8] tiles with entries [9] phases [10] chunk
-//       [16..24] per-XCD item ranges (XCD-major plans), [32 + kHeadInts q] per-XCD
-//       queue heads (the binning cleared them)
-// src: the meta block of the binning, meta: the item list's (they may be one).
-__global__ void k_plan_meta(PlanDevArgs a, const int *__restrict__ itemStart, const int *__restrict__ starts,
-                            const int *src, int *meta)
+// Clears a plan's counters and meta blocks (metaG may be null) in one launch.
+__global__ __launch_bounds__(256) void k_plan_clear(int *__restrict__ counts, long long n, int *meta, int *metaG)
 {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        const Cut cut = cut_of(a, starts, src);
-        const int n = itemStart[a.phases * a.nTiles];
-        meta[0] = n;
-        meta[1] = 0;
-        meta[2] = starts[(long long)a.nTiles * a.k2];
-        meta[9] = cut.phases;
-        meta[10] = cut.chunk;
-        // without whole shares of phases: one range, or (adaptive plans) equal ones
-        const int share = a.xcd && cut.phases % 8 == 0 ? cut.phases / 8 * a.nTiles : 0;
-        for (int x = 0; x <= 8; ++x)
-            meta[16 + x] = share ? itemStart[x * share] : a.adapt ? (int)((long long)n * x / 8) : x ? n : 0;
+    const long long i0 = blockIdx.x * 256ll + threadIdx.x;
+    for (long long i = i0; i < n; i += gridDim.x * 256ll) counts[i] = 0;
+    for (long long i = i0; i < kMetaInts; i += gridDim.x * 256ll) {
+        meta[i] = 0;
+        if (metaG) metaG[i] = 0;
     }
+}
+
+// Clears a degridder's results and its queue heads.
+__global__ __launch_bounds__(256) void k_clear_out(unsigned long long *__restrict__ out, long long n, int *meta)
+{
+    const long long i0 = blockIdx.x * 256ll + threadIdx.x;
+    for (long long i = i0; i < n; i += gridDim.x * 256ll) out[i] = 0;
+    if (i0 < 8) meta[32 + kHeadInts * i0] = 0;
+    if (i0 == 8) meta[1] = 0;
 }
 
 __global__ void k_reset_queue(int *meta)
@@ -2109,27 +2182,35 @@ long long scan_tmp_len(long long n)
     return len + 2;
 }
 
-static tcv_status scan_exclusive(tcv_ctx *ctx, const int *in, int *out, long long n, int *tmp)
+// Blocks whose sums a following kernel's blocks add up themselves, a launch less
+// than scanning them (4 M counters, 1024 blocks: 3 launches 14 us, 2 10).
+constexpr long long kRawSums = 2048;
+
+// out2: a second copy of the n results; touched: see k_scan_apply.
+static tcv_status scan_exclusive(tcv_ctx *ctx, const int *in, int *out, long long n, int *tmp, int *out2 = nullptr,
+                                 int *touched = nullptr)
 {
-    const long long nb = (n + SCAN_TILE - 1) / SCAN_TILE;
-    if (nb <= 1) {
-        hipLaunchKernelGGL(k_scan_apply, dim3(1), dim3(SCAN_BS), 0, ctx->stream, in, n,
-                           (const int *)nullptr, out);
-        TCV_HIP(ctx, hipGetLastError());
-        return TCV_OK;
-    }
+    const long long nb = std::max(1ll, (n + SCAN_TILE - 1) / SCAN_TILE);
     int *sums = tmp;
     int *sumsScan = tmp + nb + 1;
-    hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_BS), 0, ctx->stream, in, n,
-                       sums);
-    TCV_HIP(ctx, hipGetLastError());
-    tcv_status st = scan_exclusive(ctx, sums, sumsScan, nb, tmp + 2 * (nb + 1));
-    if (st != TCV_OK) return st;
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SCAN_BS), 0, ctx->stream, in, n,
-                       (const int *)sumsScan, out);
+    if (nb > 1) {
+        hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_BS), 0, ctx->stream, in, n,
+                           sums);
+        TCV_HIP(ctx, hipGetLastError());
+        if (nb > kRawSums) {
+            tcv_status st = scan_exclusive(ctx, sums, sumsScan, nb, tmp + 2 * (nb + 1));
+            if (st != TCV_OK) return st;
+        }
+    }
+    const int *offs = nb <= 1 ? nullptr : nb > kRawSums ? sumsScan : sums;
+    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SCAN_BS), 0, ctx->stream, in, n, offs,
+                       nb <= kRawSums ? 1 : 0, out, out2, touched);
     TCV_HIP(ctx, hipGetLastError());
     return TCV_OK;
 }
+
+// Visibilities from which k_plan_tile_keys runs 1024 threads a tile.
+constexpr int kBigTiles = 1 << 20;
 
 static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
 {
@@ -2139,15 +2220,22 @@ static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
     PlanDevArgs a{sh.bw, sh.bh, sh.nTX, sh.k2, sh.phases, sh.chunk, sh.nTiles, sh.xcd, sh.region > 0,
                   g.cSize, sh.adapt, kAdaptDegrid, sh.phaseBytes / sh.tapBytes};
     tcv_status st;
-    if ((st = launch_fill_u32(ctx, p->counts, 0, (size_t)sh.nKeys + 1)) != TCV_OK) return st;
-    if ((st = launch_fill_u32(ctx, p->meta, 0, kMetaInts)) != TCV_OK) return st;
+    const bool two = p->metaG != p->meta;   // the gridder's own list of work items
+    const long long nCounts = p->entriesTmp ? sh.nTiles : sh.nKeys;
+    hipLaunchKernelGGL(k_plan_clear, dim3((unsigned)std::min<long long>((nCounts + 1023) / 1024, 2048)), dim3(256), 0,
+                       ctx->stream, p->counts, nCounts, p->meta, two ? p->metaG : nullptr);
+    TCV_HIP(ctx, hipGetLastError());
+    int *touched = sh.adapt ? p->meta + 8 : nullptr;
     const bool lds = sh.nKeys <= kLdsKeys;
-    const int nb = lds ? (g.nVis + 256 * kBinVPT - 1) / (256 * kBinVPT) : (g.nVis + 255) / 256;
+    // visibilities a thread, and blocks, of the LDS binning
+    const int each = std::max(1, std::min(kBinVPT, g.nVis / (256 * std::max(1, ctx->cus))));
+    const int nbLds = (g.nVis + 256 * each - 1) / (256 * each);
+    const int nb = lds ? nbLds : (g.nVis + 255) / 256;
     auto bin = [&](int pass) -> tcv_status {
         if (g.nVis <= 0) return TCV_OK;
         if (lds)
             hipLaunchKernelGGL(k_plan_bin_lds, dim3(nb), dim3(256),
-                               (size_t)(pass ? 2 : 1) * sh.nKeys * sizeof(int), ctx->stream, pass,
+                               (size_t)(pass ? 2 : 1) * sh.nKeys * sizeof(int), ctx->stream, pass, each,
                                g, a, p->counts, p->cursor, p->entries, p->meta);
         else
             hipLaunchKernelGGL(k_plan_bin, dim3(nb), dim3(256), 0, ctx->stream, pass, g, a,
@@ -2163,23 +2251,23 @@ static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
         PlanDevArgs t1 = a;
         t1.k2 = 1;
         int *tileCount = p->counts, *tileStart = p->cursor, *tileCursor = p->cursor + sh.nTiles + 1;
-        const int nb1 = (g.nVis + 256 * kBinVPT - 1) / (256 * kBinVPT);
         if (g.nVis > 0) {
-            hipLaunchKernelGGL(k_plan_bin_lds, dim3(nb1), dim3(256), (size_t)sh.nTiles * sizeof(int),
-                               ctx->stream, 0, g, t1, tileCount, tileCursor, p->entriesTmp, p->meta);
+            hipLaunchKernelGGL(k_plan_bin_lds, dim3(nbLds), dim3(256), (size_t)sh.nTiles * sizeof(int),
+                               ctx->stream, 0, each, g, t1, tileCount, tileCursor, p->entriesTmp, p->meta);
             TCV_HIP(ctx, hipGetLastError());
         }
-        if ((st = scan_exclusive(ctx, tileCount, tileStart, sh.nTiles, p->scanTmp)) != TCV_OK) return st;
-        TCV_HIP(ctx, hipMemcpyAsync(tileCursor, tileStart, sizeof(int) * sh.nTiles,
-                                    hipMemcpyDeviceToDevice, ctx->stream));
+        if ((st = scan_exclusive(ctx, tileCount, tileStart, sh.nTiles, p->scanTmp, tileCursor, touched)) != TCV_OK)
+            return st;
         if (g.nVis > 0) {
-            hipLaunchKernelGGL(k_plan_bin_lds, dim3(nb1), dim3(256), (size_t)2 * sh.nTiles * sizeof(int),
-                               ctx->stream, 1, g, t1, tileCount, tileCursor, p->entriesTmp, p->meta);
+            hipLaunchKernelGGL(k_plan_bin_lds, dim3(nbLds), dim3(256), (size_t)2 * sh.nTiles * sizeof(int),
+                               ctx->stream, 1, each, g, t1, tileCount, tileCursor, p->entriesTmp, p->meta);
             TCV_HIP(ctx, hipGetLastError());
         }
-        hipLaunchKernelGGL(k_plan_tile_keys, dim3(sh.nTiles), dim3(256), (size_t)2 * sh.k2 * sizeof(int),
-                           ctx->stream, a, (const int *)tileStart, (const int4 *)p->entriesTmp,
-                           p->entries, p->starts, (const int *)p->meta);
+        const bool big = g.nVis >= kBigTiles;
+        hipLaunchKernelGGL(big ? k_plan_tile_keys<1024> : k_plan_tile_keys<256>, dim3(sh.nTiles),
+                           dim3(big ? 1024 : 256), (size_t)2 * sh.k2 * sizeof(int), ctx->stream, a,
+                           (const int *)tileStart, (const int4 *)p->entriesTmp, p->entries, p->starts,
+                           (const int *)p->meta);
         TCV_HIP(ctx, hipGetLastError());
     } else {
         if (sh.region > 0 && g.nVis > 0) {
@@ -2188,50 +2276,37 @@ static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
             TCV_HIP(ctx, hipGetLastError());
         }
         if ((st = bin(0)) != TCV_OK) return st;
-        if ((st = scan_exclusive(ctx, p->counts, p->starts, sh.nKeys, p->scanTmp)) != TCV_OK)
+        if ((st = scan_exclusive(ctx, p->counts, p->starts, sh.nKeys, p->scanTmp, p->cursor)) != TCV_OK)
             return st;
-        TCV_HIP(ctx, hipMemcpyAsync(p->cursor, p->starts, sizeof(int) * sh.nKeys,
-                                    hipMemcpyDeviceToDevice, ctx->stream));
         if ((st = bin(1)) != TCV_OK) return st;
-    }
-    if (sh.adapt) {
-        hipLaunchKernelGGL(k_plan_touched, dim3(std::min((sh.nTiles + 255) / 256, 64)), dim3(256), 0, ctx->stream, a,
-                           (const int *)p->starts, p->meta);
-        TCV_HIP(ctx, hipGetLastError());
+        if (touched) {
+            hipLaunchKernelGGL(k_plan_touched, dim3(std::min((sh.nTiles + 255) / 256, 64)), dim3(256), 0, ctx->stream,
+                               a, (const int *)p->starts, p->meta);
+            TCV_HIP(ctx, hipGetLastError());
+        }
     }
     // work items: cuts of the sorted entries into (phase, tile) ranges
-    auto items = [&](int phases, int xcd, int minEntries, int *itemCount, int *itemStart, int4 *itemsOut,
-                     int *meta) -> tcv_status {
-        PlanDevArgs b = a;
-        b.phases = phases;
-        b.xcd = xcd;
-        b.minEntries = minEntries;
-        const int slots = phases * sh.nTiles;
-        hipLaunchKernelGGL(k_plan_items, dim3((slots + 255) / 256), dim3(256), 0, ctx->stream, 0,
-                           b, p->starts, itemCount, (const int *)itemStart, itemsOut,
-                           (const int *)p->meta);
-        TCV_HIP(ctx, hipGetLastError());
-        tcv_status s2 = scan_exclusive(ctx, itemCount, itemStart, slots, p->scanTmp);
-        if (s2 != TCV_OK) return s2;
-        hipLaunchKernelGGL(k_plan_items, dim3((slots + 255) / 256), dim3(256), 0, ctx->stream, 1,
-                           b, p->starts, itemCount, (const int *)itemStart, itemsOut,
-                           (const int *)p->meta);
-        TCV_HIP(ctx, hipGetLastError());
-        hipLaunchKernelGGL(k_plan_meta, dim3(1), dim3(64), 0, ctx->stream, b, (const int *)itemStart,
-                           (const int *)p->starts, (const int *)p->meta, meta);
-        TCV_HIP(ctx, hipGetLastError());
-        return TCV_OK;
-    };
-    const bool two = p->metaG != p->meta;
-    if ((st = items(sh.phases, sh.xcd, two ? kAdaptDegrid : kAdaptGrid, p->itemCount, p->itemStart, p->items,
-                    p->meta)) != TCV_OK)
-        return st;
-    if (two) {
-        // the out-of-range count lives in meta[3]; the gridder's meta gets its own copy
-        if ((st = launch_fill_u32(ctx, p->metaG, 0, kMetaInts)) != TCV_OK) return st;
-        if ((st = items(sh.phasesG, sh.xcdG, kAdaptGrid, p->itemCountG, p->itemStartG, p->itemsG, p->metaG)) != TCV_OK)
-            return st;
+    ItemLists lists{};
+    lists.l[0] = ItemList{sh.phases, sh.xcd, two ? kAdaptDegrid : kAdaptGrid, p->itemCount, p->itemStart, nullptr,
+                          p->items, p->meta};
+    lists.l[1] = ItemList{sh.phasesG, sh.xcdG, kAdaptGrid, p->itemCountG, p->itemStartG, nullptr, p->itemsG, p->metaG};
+    long long most = 0;
+    for (int k = 0; k < (two ? 2 : 1); ++k)
+        most = std::max(most, ((long long)lists.l[k].phases * sh.nTiles + SCAN_BS - 1) / SCAN_BS);
+    const dim3 blocks((unsigned)most, two ? 2 : 1);
+    hipLaunchKernelGGL(k_plan_items, blocks, dim3(SCAN_BS), 0, ctx->stream, 0, a, lists, (const int *)p->starts,
+                       (const int *)p->meta);
+    TCV_HIP(ctx, hipGetLastError());
+    for (int k = 0; k < (two ? 2 : 1); ++k) {
+        ItemList &l = lists.l[k];
+        const long long nb = ((long long)l.phases * sh.nTiles + SCAN_BS - 1) / SCAN_BS;
+        if (nb <= kRawSums) continue;
+        if ((st = scan_exclusive(ctx, l.sums, l.sums + nb, nb, p->scanTmp)) != TCV_OK) return st;
+        l.scanned = l.sums + nb;
     }
+    hipLaunchKernelGGL(k_plan_items, blocks, dim3(SCAN_BS), 0, ctx->stream, 1, a, lists, (const int *)p->starts,
+                       (const int *)p->meta);
+    TCV_HIP(ctx, hipGetLastError());
     return TCV_OK;
 }
 
@@ -2471,8 +2546,11 @@ tcv_status launch_degrid_tiled(tcv_ctx *ctx, tcv_plan *p, const float2 *grid, co
 {
     ItemSource<false> src{make_job_desc(p, false, nullptr, C, const_cast<float2 *>(grid), out, half),
                           nullptr, nullptr, 0, p->meta + 1, p->sh.xcd, ctx->d_bcast};
-    tcv_status st = launch_fill_u32(ctx, out, 0, (size_t)p->nVis * 2);
-    if (st != TCV_OK) return st;
+    const long long fill = std::max(1ll, std::min((p->nVis + 1023ll) / 1024, (long long)ctx->cus * 8));
+    hipLaunchKernelGGL(k_clear_out, dim3((unsigned)fill), dim3(256), 0, ctx->stream,
+                       reinterpret_cast<unsigned long long *>(out), (long long)p->nVis, p->meta);
+    TCV_HIP(ctx, hipGetLastError());
+    tcv_status st = TCV_OK;
     for (auto &q : p->parts) {
         // results stored into the cleared output, beside those the tiles add up
         st = launch_narrow(ctx, make_job_desc(q.get(), false, nullptr, C, const_cast<float2 *>(grid), out, half),
@@ -2480,8 +2558,6 @@ tcv_status launch_degrid_tiled(tcv_ctx *ctx, tcv_plan *p, const float2 *grid, co
         if (st != TCV_OK) return st;
     }
     if (p->sh.region > 0) return launch_narrow(ctx, src.one, p->sh.region, half != nullptr, true);
-    hipLaunchKernelGGL(k_reset_queue, dim3(1), dim3(64), 0, ctx->stream, p->meta);
-    TCV_HIP(ctx, hipGetLastError());
     // the FP16 four-tap degridder needs kernel widths of at least 4
     const int kern = (half && p->sh.dkern == 4 && p->sh.minS < 4) ? 3 : p->sh.dkern;
     const double phaseBytes = (double)p->cSize * (half ? 4 : 8) / std::max(1, p->sh.phases);

@@ -1,8 +1,9 @@
-"""Plans that take narrow kernels by regions: every width that a region size is
+"""Plans: narrow kernels by regions at every width that a region size is
 built for (steps of the walk, odd and even, the widest of a class), grids that
 no region divides, the first and last slices of the table, widths mixed with
 wider ones, FP16 storage and batches.  Taps are multiples of 1/4 and values
-small integers, so every sum is exact and results equal the oracle's."""
+small integers, so every sum is exact and results equal the oracle's.  After them:
+work items sized on the device, and the counters and scans of the plan's build."""
 from __future__ import annotations
 
 import numpy as np
@@ -216,3 +217,17 @@ def test_adaptive_plan_of_nothing(ctx):
     out = ctx.to_device(np.ones(2, np.complex64))
     plan.degrid(g, C, out)
     assert not g.download().any() and not out.download().any()
+
+
+@pytest.mark.parametrize("keys,phases,nVis", [(256, 1, 5000), (64, 16, 5000), (16, 1, 300), (1, 1, 70000)])
+def test_plan_of_many_counters(ctx, keys, phases, nVis):
+    """65 536 tiles: counters and work-item slots beyond one block's scan, up to what
+    the following blocks add up themselves, and beyond it."""
+    j = job(keys + nVis, [9, 12], nVis, 4096, os_=8)
+    gref, oref = reference(j)
+    plan = tcv.Plan(ctx, visibilities(ctx, j), tile_w=8, tile_h=32, slice_keys=keys, phases=phases,
+                    grid_phases=2 * phases if keys > 16 else phases)
+    for _ in range(2):
+        g, o = run(ctx, plan, j)
+        assert np.array_equal(g, gref) and np.array_equal(o, oref)
+        plan.build()
