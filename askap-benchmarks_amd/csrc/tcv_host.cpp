@@ -493,7 +493,12 @@ static int default_phases(long long cSize, int tapBytes, int sliceKeys, const tc
 }
 
 constexpr double kDegridPhaseBytes = 5.5e6;
-constexpr int kItemEntries = 64;   // entries per work item the phase count keeps at least
+// Entries per work item that the phase count keeps at least.  Batches re-bin + grid
+// + degrid in ms with 64 and 32: 16 jobs of 10 000-500 000 visibilities 42.98 and
+// 40.40 (24: 40.46), 10 of 5000-150 000 16.15 and 15.34, 19 of up to 61 000 11.02
+// and 11.04.  Servers and the caller-scratch gridder keep 64: their plans' size is
+// what their memory was measured out for.
+constexpr int kItemEntries = 32, kItemEntriesFixed = 64;
 constexpr double kGridPhaseBytes = 5.5e6;   // the gridder may use its own count (grid_phases)
 // 128 x 64 tiles carry half again as many entries per work item: smaller phases
 // (measured optimum 256-320 phases on a 1.1 GB table, against 184-216 for 64 x 64)
@@ -622,6 +627,7 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
         auto it = ctx->tuned.find(tuning_class(g));
         if (it != ctx->tuned.end()) t = it->second;
     }
+    PlanShape &sh = p->sh;
     // a plan whose shape is left open takes its narrower kernels by regions
     struct Part { int lo, hi, region, chunk; };
     std::vector<Part> parts;   // the classes that the job's widths fall in
@@ -647,6 +653,8 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
     // items its own need no cutting (19 jobs of 5000-61 000 visibilities 11.2 ms,
     // cut 11.9).
     const bool adapt = !tilesOnly && open_shape(t) && t.item_entries <= 0;
+    if (tilesOnly && t.item_entries <= 0) t.item_entries = kItemEntriesFixed;
+    sh.colsOpen = t.grid_cols <= 0;
     auto_tuning(maxS, g, &t);
     if (!tiled_config_supported(t.tile_w, t.tile_h))
         return tcv_fail(ctx, TCV_ERR_UNSUPPORTED, "tile shape not built");
@@ -656,7 +664,6 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
         return tcv_fail(ctx, TCV_ERR_UNSUPPORTED,
                         "tuning.grid_cols must be tile_w, or tile_w / 2 or / 4 (at least 16) on tiles 64 wide "
                         "and up with tile_h >= 512 / grid_cols");
-    PlanShape &sh = p->sh;
     sh.tw = t.tile_w;
     sh.th = t.tile_h;
     sh.chunk = t.chunk;
@@ -1047,6 +1054,7 @@ tcv_status tcv_batch_create(tcv_ctx *ctx, int nJobs, const tcv_job *jobs, tcv_ba
     *out = nullptr;
     tcv_batch *b = new tcv_batch();
     std::vector<JobDesc> tiled, tiledD, narrow[2];
+    bool open = true;   // every plan leaves grid_cols open
     for (int j = 0; j < nJobs; j++) {
         const tcv_job &J = jobs[j];
         if (!J.plan || !J.d_C || !J.d_grid) {
@@ -1065,6 +1073,7 @@ tcv_status tcv_batch_create(tcv_ctx *ctx, int nJobs, const tcv_job *jobs, tcv_ba
             return tcv_fail(ctx, TCV_ERR_INVALID,
                             "tcv_batch_create: all plans of a batch need one tile shape, kernel and grid_cols");
         }
+        open = open && J.plan->sh.colsOpen;
         b->plans.push_back(J.plan);
         b->host.push_back(make_job_desc(J.plan, true, J.d_data, J.d_C, (float2 *)J.d_grid, (float2 *)J.d_out, nullptr));
         b->hostD.push_back(make_job_desc(J.plan, false, J.d_data, J.d_C, (float2 *)J.d_grid, (float2 *)J.d_out, nullptr));
@@ -1088,6 +1097,10 @@ tcv_status tcv_batch_create(tcv_ctx *ctx, int nJobs, const tcv_job *jobs, tcv_ba
             tiledD.push_back(b->hostD[j]);
         }
     }
+    // Jobs of many widths on 128 x 64 tiles: groups of 32 columns waste fewer lanes
+    // on the narrower ones (gridding 16 jobs of widths 63-131: 20.6 ms with 64, 19.5
+    // with 32; 10 jobs 7.4 and 7.0; one job of width 129: equal).
+    if (open && b->tw == 128 && b->th == 64) b->gridCols = 32;
     b->nJobs = (int)tiled.size();
     auto fail = [&](const char *m) {
         if (b->d_jobs) (void)hipFree(b->d_jobs);

@@ -168,6 +168,7 @@ struct PlanShape {
     int tapBytes;          // stored tap size the tuning was chosen for (8 or 4)
     int itemEntries;       // entries per work item the automatic phase counts aimed at
     int gridCols;          // pair gridder: columns per load instruction (tcv_tuning.grid_cols)
+    int colsOpen;          // 1: the tuning left gridCols open (a batch may take other groups)
     // narrow-kernel plans (tcv_narrow.hip): cells a side of the regions, which
     // overlap so that each footprint lies in one; 0: tiles of tw x th
     int region;

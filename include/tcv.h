@@ -255,7 +255,8 @@ typedef struct {
                         counts, which follow the table's size in bytes */
     int item_entries; /* fewest entries per work item (on average) the automatic phase
                         counts keep: finer phases keep a job's C slices in the L2s, but
-                        every work item zeroes and flushes its tile (0 = 64) */
+                        every work item zeroes and flushes its tile (0 = 32; 64 for
+                        servers; open plans size their items on the device) */
     int grid_cols;   /* pair gridder (kernel 3, FP32 and FP16 pairs): columns per load
                         instruction.  One instruction covers grid_cols columns over
                         128 / grid_cols rows; footprints narrower than the tile waste
