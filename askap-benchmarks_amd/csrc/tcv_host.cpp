@@ -574,6 +574,12 @@ constexpr WidthClass kClasses[] = {{19, 32, 128}, {31, 48, 64}};
 // 102 + 92 + 89 -> 48 + 86 + 38; 64 000 132 + 127 + 115 -> 74 + 387 + 142;
 // 500 000 401 + 670 + 488 -> 189 + 733 + 338.
 constexpr int kSmallJob = 8192, kDenseRegion = 8;
+// Entries that a job of footprints of the widest kernel makes on average.
+static double entries_expected(const tcv_geometry *g, const PlanShape &sh)
+{
+    return g->nVis * (1.0 + (sh.maxS - 1.0) / sh.tw) * (1.0 + (sh.maxS - 1.0) / sh.th);
+}
+
 // Array sizes that follow from a plan's shape, and the bytes of its buffers.
 static tcv_status plan_sizes(tcv_ctx *ctx, const tcv_geometry *g, tcv_plan *p, size_t *bytes);
 
@@ -654,6 +660,25 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
     // cut 11.9).
     const bool adapt = !tilesOnly && open_shape(t) && t.item_entries <= 0;
     if (tilesOnly && t.item_entries <= 0) t.item_entries = kItemEntriesFixed;
+    if (adapt && maxS >= 48 && t.tap_bytes != 4) {
+        // Open FP32 plans of many entries take 128 x 64 tiles from width 48 up: a
+        // quarter fewer entries, once phases and chunks fit the job.  Grid + degrid in
+        // us, 64 x 64 and 128 x 64: width 63, 100 003 visibilities, 2047^2 481 + 379 and
+        // 448 + 350; 49, 200 000, 4096^2 596 + 474 and 575 + 385; 87, 200 000, 2000^2 1110
+        // + 867 and 1028 + 716 (FP16, width 129, 160 000, 4096^2, a whole pass 2174 and
+        // 2214).  With fewer entries, or on few tiles, the smaller ones share out better:
+        // 49, 30 000, 600^2 135 + 81 and 174 + 72; 87, 66 000, 2000^2 582 + 360 and 522 + 507.
+        sh.maxS = maxS;
+        sh.tw = 128;
+        sh.th = 64;
+        const long long tiles = (long long)((g->gSize + 127) / 128) * ((g->gSize + 63) / 64);
+        int least = maxS;
+        for (int k = 0; k < g->nPlanes; k++) least = std::min(least, g->sSize[k]);
+        if (least >= 2 && tiles >= 128 && entries_expected(g, sh) > kAdaptItems * kAdaptChunk) {
+            t.tile_w = 128;
+            t.tile_h = 64;
+        }
+    }
     sh.colsOpen = t.grid_cols <= 0;
     auto_tuning(maxS, g, &t);
     if (!tiled_config_supported(t.tile_w, t.tile_h))
@@ -738,12 +763,6 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
         st = region_setup(ctx, g, parts.back().region, parts.back().chunk, parts.back().hi, parts.back().lo, p, bytes);
     *bytes += partBytes;
     return st;
-}
-
-// Entries that a job of footprints of the widest kernel makes on average.
-static double entries_expected(const tcv_geometry *g, const PlanShape &sh)
-{
-    return g->nVis * (1.0 + (sh.maxS - 1.0) / sh.tw) * (1.0 + (sh.maxS - 1.0) / sh.th);
 }
 
 static tcv_status plan_sizes(tcv_ctx *ctx, const tcv_geometry *g, tcv_plan *p, size_t *bytes)

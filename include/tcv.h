@@ -227,13 +227,15 @@ tcv_status tcv_range_errors(tcv_ctx *ctx, long long *count);
 
 typedef struct {
     int tile_w;      /* 8, 16, 32, 64 or 128 columns (0 = auto: 128 x 64 tiles for
-                        kernels 89 wide and up when the pair kernels apply); 128-wide
+                        kernels 89 wide and up when the pair kernels apply, and, with
+                        every field open, 48 and up on jobs of many entries); 128-wide
                         tiles take only the pair kernels (kernel and degrid_kernel 3) */
     int tile_h;      /* rows per tile: 32 or 64 for tiles 8..64 wide, 64 for 128-wide
                         tiles, and the tall shapes 64 x 128 and 32 x 256 (pair kernels
                         only); 0 = auto */
     int chunk;       /* max entries per work item (0 = auto: 2048, 1024 for jobs with
-                        kernels narrower than 24, 512 when all are) */
+                        kernels narrower than 24, 512 when all are; sized on the
+                        device when every field is open, as are the phase counts) */
     int slice_keys;  /* order entries in a tile by C-slice key, 0 = no ordering */
     int phases;      /* >1: split each tile's entries into C-slice phases: equal runs of
                         the slice keys the job's entries use (0 = auto) */

@@ -175,7 +175,8 @@ def test_regions_in_a_batch(ctx):
     (129, 400, 2500, 60, 8, 5),       # few tiles: cut to chunks of 32
     (97, 700, 9000, 0, 8, 9),         # phases, one list of work items
     (63, 900, 70000, 0, 8, 33),       # two lists: finer phases for the degridder
-    (63, 600, 120000, 12, 4, 4)])     # hot tiles
+    (63, 600, 120000, 12, 4, 4),      # hot tiles
+    (49, 1100, 170000, 0, 4, 9)])     # many entries: 128 x 64 tiles below width 89
 def test_adaptive_work_items(ctx, Sz, gSize, nVis, cluster, os_, planes):
     """Phases and chunks chosen on the device: exact results, and as many work items
     as a plan with the same numbers given makes."""
@@ -199,6 +200,7 @@ def test_adaptive_work_items(ctx, Sz, gSize, nVis, cluster, os_, planes):
         assert np.array_equal(out.download(), oref)
         plan.build()
     info = plan.info()
+    assert info["tile_w"] == (128 if Sz > 88 or nVis == 170000 else 64)
     given = tcv.Plan(ctx, vis, **{k: info[k] for k in ("tile_w", "tile_h", "chunk", "slice_keys", "phases",
                                                        "grid_phases", "kernel", "degrid_kernel")}).info()
     assert (given["items"], given["entries"], given["phases"], given["chunk"]) == \
