@@ -1345,6 +1345,18 @@ tcv_status tcv_autotune(tcv_ctx *ctx, const tcv_geometry *g, const float *d_data
                 auto_tuning(maxS, g, &t);   // phases and column groups for this tile shape
                 if ((st = consider(t)) != TCV_OK) return st;
             }
+        // the open plan, its device-sized work items spelled out
+        {
+            tcv_plan *p = nullptr;
+            tcv_tuning t{0, 0, 0, 0, 0, -1, 0, 0, 0, 0, 0, 0};
+            if (tcv_plan_create(ctx, g, &t, &p) == TCV_OK) {
+                const bool tiles = p->sh.region == 0 && p->parts.empty();
+                st = tcv_plan_info(ctx, p, &t, nullptr, nullptr, nullptr);
+                tcv_plan_destroy(ctx, p);
+                if (st == TCV_OK && tiles) st = consider(t);
+                if (st != TCV_OK) return st;
+            }
+        }
         if (!any) return tcv_fail(ctx, TCV_ERR_UNSUPPORTED, "tcv_autotune: no candidate could be planned");
         const tcv_tuning b0 = *best;
         if ((op & 1) && b0.kernel == 3)
