@@ -466,11 +466,13 @@ tcv_status tcv_range_errors(tcv_ctx *ctx, long long *count)
 // (concurrently running workgroups share the phase's slices in L2; fewer
 // phases when work items would get short), and, with 8 or more phases, work
 // items ordered XCD-major with one queue per XCD so each XCD walks its own
-// phases.  Kernels: kDefaultGridKernel / kDefaultDegridKernel.
+// phases.  Kernels: kDefaultGridKernel / kDefaultDegridKernel.  A plan with every
+// field open sizes phases and work items on the device (cut_of) and takes kernels
+// up to 31 wide by regions (kClasses).
 // C-slice phases: about `bytesPerPhase` of taps per phase, so that the slices
 // one phase touches stay in L2 / Infinity Cache while its tiles run (measured
-// best: ~5.5 MB for both kernels), but no more than leaves about 64 entries
-// per (tile, phase) work item on average: every item zeroes and flushes its
+// best: ~5.5 MB for both kernels), but no more than leaves itemEntries entries
+// to a (tile, phase) work item on average: every item zeroes and flushes its
 // tile.  From 8 phases up a multiple of 8, so the phases split evenly over
 // the XCDs.
 static int default_phases(long long cSize, int tapBytes, int sliceKeys, const tcv_geometry *g, int maxS,
