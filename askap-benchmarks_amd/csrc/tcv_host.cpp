@@ -18,6 +18,16 @@ tcv_status tcv_fail(tcv_ctx *ctx, tcv_status s, const std::string &msg)
     return s;
 }
 
+tcv_status ctx_wait(tcv_ctx *ctx)
+{
+    TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if (!ctx->lateFail || !*(volatile int *)ctx->lateFail) return TCV_OK;
+    *ctx->lateFail = 0;
+    return tcv_fail(ctx, TCV_ERR_DEVICE,
+                    "tcv_hogbom: the workgroups of the loop did not run together within the wait limit; "
+                    "its last iterations are not done");
+}
+
 ProfScope::ProfScope(tcv_ctx *c, const char *fam) : ctx(c), family(fam)
 {
     if (!ctx->profiling) return;
@@ -133,7 +143,13 @@ int tcv_device_cus(const tcv_ctx *ctx) { return ctx ? ctx->cus : 0; }
 tcv_status tcv_synchronize(tcv_ctx *ctx)
 {
     if (!ctx) return TCV_ERR_INVALID;
-    TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return ctx_wait(ctx);
+}
+
+tcv_status tcv_set_wait_limit(tcv_ctx *ctx, unsigned long long polls)
+{
+    if (!ctx) return TCV_ERR_INVALID;
+    ctx->waitPolls = polls;
     return TCV_OK;
 }
 
@@ -181,8 +197,7 @@ tcv_status tcv_download(tcv_ctx *ctx, void *dst, const void *d_src, size_t bytes
     if (!ctx || (bytes && (!dst || !d_src))) return TCV_ERR_INVALID;
     if (!bytes) return TCV_OK;
     TCV_HIP(ctx, hipMemcpyAsync(dst, d_src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return TCV_OK;
+    return ctx_wait(ctx);
 }
 
 tcv_status tcv_zero(tcv_ctx *ctx, void *d_ptr, size_t bytes)
@@ -241,7 +256,7 @@ tcv_status tcv_timer_stop(tcv_ctx *ctx, double *ms)
     float f = 0.f;
     TCV_HIP(ctx, hipEventElapsedTime(&f, ctx->timer0, ctx->timer1));
     *ms = f;
-    return TCV_OK;
+    return ctx_wait(ctx);
 }
 
 tcv_status tcv_set_profiling(tcv_ctx *ctx, int on)

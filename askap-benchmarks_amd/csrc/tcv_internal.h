@@ -33,6 +33,10 @@ struct tcv_ctx {
     std::map<int, void *> fftPlans, fftTwiddles;
     void *majorWs = nullptr;
     size_t majorWsBytes = 0;
+    // longest wait of workgroups on each other, and the flag (host memory) that
+    // reports one of a call that had returned
+    unsigned long long waitPolls = 1ull << 24;
+    int *lateFail = nullptr;
     // device address of the fixed scratch array of tcv_grid_noalloc on this
     // context's device (null, with the reason, when the lookup failed)
     void *scratch = nullptr;
@@ -54,6 +58,10 @@ void major_release(tcv_ctx *ctx);
 std::string tuning_class(const tcv_geometry *g);
 
 tcv_status tcv_fail(tcv_ctx *ctx, tcv_status s, const std::string &msg);
+
+// Waits for the context's stream and reports what a call that had returned
+// could not finish (ctx->lateFail).
+tcv_status ctx_wait(tcv_ctx *ctx);
 
 #define TCV_HIP(ctx, expr)                                                      \
     do {                                                                        \

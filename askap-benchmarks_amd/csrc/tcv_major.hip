@@ -305,8 +305,13 @@ __global__ __launch_bounds__(256) void k_peak_complex(const float2 *__restrict__
 // never more than one iteration ahead of the slowest, which must still find the
 // set before).  A slot holds the peak's key and the iteration's number (8 bits)
 // in one 64-bit word, so nothing else needs ordering.  The host launches it
-// cooperatively, so all workgroups are resident; the wait is bounded all the
-// same (*fail is set and every workgroup leaves).
+// cooperatively, so all workgroups are resident; the waits are bounded all the
+// same (another process may hold part of the device), and a launch is done whole
+// or not at all: nothing is written until every workgroup has finished the
+// iterations and added itself to *agree, and one whose wait runs out marks *agree
+// kLost unless all have.  Components wait in LDS until then, kLoopIters at most;
+// more iterations take more launches, each of which goes on only where the one
+// before was done (*chunks).
 // Key: |v| bits << 25 | (2^24 - 1 - index) << 1 | sign, as peak_key orders them.
 // Bound: the PSF's read, 67 MB at 4096^2 from the Infinity Cache, and the
 // exchange.  13.4 us an iteration at 4096^2, against 35.5 us for
@@ -317,13 +322,18 @@ struct HogbomLoop {
     float2 *model;                   // complex model image
     const unsigned long long *psfKey;   // PSF peak (peak_key)
     unsigned long long *slots;       // 2 x kSlots, zeroed
-    unsigned long long *first;       // first residual peak (peak_key)
-    int *fail;
-    int W, PW, niters;
+    unsigned long long *first;       // first residual peak (peak_key; the first launch)
+    unsigned *agree;                 // workgroups that finished, zeroed
+    int *chunks;                     // launches of this call done
+    int *hostFail;                   // host flag of a call that doesn't wait (or null)
+    unsigned long long polls;        // longest wait (of about a microsecond each)
+    int W, PW, niters, chunk;        // chunk: launches before this one
     int C;                           // column groups of four a row, rounded up to a power of two
     float gain;
 };
 constexpr int kSlots = 1024;
+constexpr int kLoopIters = 1024;
+constexpr unsigned kLost = 1u << 31;
 constexpr int kPsfPad = 64;   // floats before and after the plane that a group of four may read (unused)
 
 __device__ __forceinline__ unsigned long long loop_key(unsigned absBits, unsigned idx, bool neg)
@@ -336,9 +346,12 @@ __global__ __launch_bounds__(1024) void k_hogbom_loop(HogbomLoop a)
 {
 #pragma clang fp contract(off)
     constexpr int kBlk = GPT < 4 ? GPT : 4;   // groups whose PSF reads are issued together
-    constexpr unsigned long long kSpin = 1ull << 24;   // polls of about a microsecond
     __shared__ unsigned s_abs[16];
     __shared__ unsigned long long s_key, s_win[16];
+    __shared__ unsigned s_pos[kLoopIters];   // the components (the first workgroup's are used)
+    __shared__ float s_amp[kLoopIters];
+    __shared__ bool s_done;
+    if (*a.chunks != a.chunk) return;   // an earlier launch was not done
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int W = a.W, PW = a.PW, nWG = gridDim.x;
     // the workgroup's threads cover 1024 / C rows of C column groups a step
@@ -354,7 +367,8 @@ __global__ __launch_bounds__(1024) void k_hogbom_loop(HogbomLoop a)
     const unsigned ppos = key_index(kp);
     const int px = (int)(ppos % (unsigned)PW), py = (int)(ppos / (unsigned)PW);
     if (tid == 0) s_key = 0ull;
-    for (int it = 0;; ++it) {
+    bool lost = false;
+    for (int it = 0; it < max(a.niters, 1) && !lost; ++it) {
         // opaque copies: the rows' positions are worked out again in every
         // iteration instead of being kept in registers across them
         int yb = y0, xa = x;
@@ -394,9 +408,9 @@ __global__ __launch_bounds__(1024) void k_hogbom_loop(HogbomLoop a)
         unsigned long long *slots = a.slots + (it & 1) * kSlots;
         if (tid == 0)
             __hip_atomic_store(slots + blockIdx.x, s_key | tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        unsigned long long k = 0;
+        unsigned long long k = tid < nWG ? ~0ull : 0ull;
         if (tid < nWG) {
-            for (unsigned long long n = 0; n < kSpin; ++n) {
+            for (unsigned long long n = 0; n < a.polls; ++n) {
                 k = __hip_atomic_load(slots + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (k >> 56 == tag >> 56) break;
                 k = ~0ull;   // still the wrong one when the wait ends
@@ -408,26 +422,26 @@ __global__ __launch_bounds__(1024) void k_hogbom_loop(HogbomLoop a)
         unsigned long long win = 0;
 #pragma unroll
         for (int w = 0; w < 16; ++w) win = s_win[w] > win ? s_win[w] : win;
-        if (win == ~0ull) {
-            if (tid == 0) *a.fail = 1;
-            break;
-        }
-        win &= (1ull << 56) - 1;
+        // a lost workgroup ends the iteration on pixel 0 with a peak of zero (a break
+        // here costs 27 spilled registers)
+        lost = win == ~0ull;
+        win = lost ? loop_key(0u, 0u, false) : win & ((1ull << 56) - 1);
         const unsigned absBits = (unsigned)(win >> 25), pos = 0xffffffu - (unsigned)((win >> 1) & 0xffffffu);
         const float peak = __uint_as_float(absBits | ((unsigned)(win & 1) << 31));
         if (tid == 0) {
             s_key = 0ull;
-            if (it == 0 && blockIdx.x == 0) *a.first = peak_key(peak, pos);
+            if (it == 0 && a.chunk == 0 && blockIdx.x == 0) *a.first = peak_key(peak, pos);
         }
-        if (it == a.niters) break;
+        if (it == a.niters) break;   // none to do
         const int rx = (int)(pos % (unsigned)W), ry = (int)(pos / (unsigned)W);
         const int diffx = rx - px, diffy = ry - px;   // as in the reference
         const int startx = max(0, rx - px), starty = max(0, ry - py);
         const int stopx = min(W - 1, rx + (PW - px - 1)), stopy = min(W - 1, ry + (PW - py - 1));
         const float amp = a.gain * peak;
-        // one thread makes every model update, so that they follow each other;
-        // not in a wave that waits for the slots
-        if (blockIdx.x == 0 && tid == 1023) a.model[pos].x = a.model[pos].x + peak * a.gain;
+        if (tid == 1023) {   // not in a wave that waits for the slots
+            s_pos[it] = pos;
+            s_amp[it] = amp;
+        }
         bool col[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) col[c] = xa + c >= startx && xa + c <= stopx;
@@ -457,8 +471,34 @@ __global__ __launch_bounds__(1024) void k_hogbom_loop(HogbomLoop a)
             __builtin_amdgcn_sched_barrier(0);   // PSF reads of kBlk rows in flight: the registers' bound
         }
     }
-    // on a failed wait the residual is left as it was
-    if (__hip_atomic_load(a.fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+    if (tid == 0) {
+        unsigned n = lost ? atomicOr(a.agree, kLost) | kLost : atomicAdd(a.agree, 1u) + 1;
+        for (unsigned long long p = 0; p < a.polls && n != (unsigned)nWG && !(n & kLost); ++p)
+            n = __hip_atomic_load(a.agree, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        while (n != (unsigned)nWG && !(n & kLost)) {   // the wait ran out; each turn but the last finds one more
+            const unsigned seen = atomicCAS(a.agree, n, n | kLost);
+            n = seen == n ? n | kLost : seen;
+        }
+        s_done = n == (unsigned)nWG;
+        if (!s_done && a.hostFail) __hip_atomic_store(a.hostFail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __syncthreads();
+    if (!s_done) return;
+    if (blockIdx.x == 0) {
+        // a component a thread; the first at a pixel adds all of that pixel's in turn
+        if (tid == 0) *a.chunks = a.chunk + 1;
+        if (tid < a.niters) {
+            const unsigned at = s_pos[tid];
+            int j = 0;
+            while (j < tid && s_pos[j] != at) ++j;
+            if (j == tid) {
+                float m = a.model[at].x;
+                for (; j < a.niters; ++j)
+                    if (s_pos[j] == at) m = m + s_amp[j];
+                a.model[at].x = m;
+            }
+        }
+    }
     int yw = y0, xw = x;
     asm volatile("" : "+v"(yw), "+v"(xw));   // addresses worked out anew, not kept since the loads
 #pragma unroll
@@ -506,6 +546,8 @@ void major_release(tcv_ctx *ctx)
     if (ctx->majorWs) (void)hipFree(ctx->majorWs);
     ctx->majorWs = nullptr;
     ctx->majorWsBytes = 0;
+    if (ctx->lateFail) (void)hipHostFree(ctx->lateFail);
+    ctx->lateFail = nullptr;
 }
 
 // grow-only workspace: Hogbom's float planes and peak keys
@@ -524,6 +566,25 @@ static tcv_status major_ws(tcv_ctx *ctx, size_t bytes, void **p)
         ctx->majorWsBytes = bytes;
     }
     *p = ctx->majorWs;
+    return TCV_OK;
+}
+
+// The flag that the kernels of a call which doesn't wait set in host memory; the
+// calls that wait for the stream report it (ctx_wait).
+static tcv_status late_flag(tcv_ctx *ctx, int **d_flag)
+{
+    if (!ctx->lateFail) {
+        void *p = nullptr;
+        if (hipHostMalloc(&p, sizeof(int), hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+            (void)hipGetLastError();
+            return tcv_fail(ctx, TCV_ERR_NOMEM, "tcv_hogbom: host flag");
+        }
+        ctx->lateFail = (int *)p;
+        *ctx->lateFail = 0;
+    }
+    void *d = nullptr;
+    TCV_HIP(ctx, hipHostGetDevicePointer(&d, ctx->lateFail, 0));
+    *d_flag = (int *)d;
     return TCV_OK;
 }
 
@@ -553,7 +614,7 @@ static bool hogbom_loop_fits(const tcv_ctx *ctx, long long width, long long psfW
     return ctx->coopLaunch && width <= 4096 && psfWidth <= 32768 && hogbom_groups(ctx, width, &C, &nWG) > 0;
 }
 
-static tcv_status launch_hogbom_loop(tcv_ctx *ctx, HogbomLoop a)
+static hipError_t launch_hogbom_loop(tcv_ctx *ctx, HogbomLoop a)
 {
     unsigned nWG = 0;
     const int gpt = hogbom_groups(ctx, a.W, &a.C, &nWG);
@@ -563,8 +624,7 @@ static tcv_status launch_hogbom_loop(tcv_ctx *ctx, HogbomLoop a)
                     : gpt == 8 ? (const void *)k_hogbom_loop<8>
                                : (const void *)k_hogbom_loop<16>;
     void *args[] = {&a};
-    TCV_HIP(ctx, hipLaunchCooperativeKernel(k, dim3(nWG), dim3(1024), args, 0, ctx->stream));
-    return TCV_OK;
+    return hipLaunchCooperativeKernel(k, dim3(nWG), dim3(1024), args, 0, ctx->stream);
 }
 
 static tcv_status fft_run(tcv_ctx *ctx, float *d_grid, int gSize, int forward, int fix, float scale)
@@ -650,7 +710,7 @@ tcv_status tcv_find_peak(tcv_ctx *ctx, const float *d_image, long long nPixels, 
     TCV_HIP(ctx, hipGetLastError());
     unsigned long long k = 0;
     TCV_HIP(ctx, hipMemcpyAsync(&k, key, 8, hipMemcpyDeviceToHost, ctx->stream));
-    TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    if ((st = ctx_wait(ctx)) != TCV_OK) return st;
     const unsigned a = (unsigned)(k >> 33);
     float av;
     std::memcpy(&av, &a, 4);
@@ -669,47 +729,71 @@ tcv_status tcv_hogbom(tcv_ctx *ctx, float *d_residual, long long width, const fl
         width * width > 0xffffffffLL || psfWidth * psfWidth > 0xffffffffLL)
         return tcv_fail(ctx, TCV_ERR_INVALID, "tcv_hogbom: bad argument (widths below 65536)");
     const long long n = width * width, pn = psfWidth * psfWidth;
-    const bool loop = hogbom_loop_fits(ctx, width, psfWidth);
-    // PSF plane | keys, failure flag | slots of the loop, or residual plane
-    const size_t psfB = ((size_t)(pn + 2 * kPsfPad) * 4 + 255) & ~size_t(255);
-    const size_t resB = loop ? 2 * kSlots * sizeof(unsigned long long) : ((size_t)n * 4 + 255) & ~size_t(255);
-    void *ws;
-    tcv_status st = major_ws(ctx, psfB + 256 + resB, &ws);
-    if (st != TCV_OK) return st;
-    float *psf = (float *)ws + kPsfPad;
-    unsigned long long *keys = (unsigned long long *)((char *)ws + psfB);
-    void *rest = (char *)ws + psfB + 256;
+    const bool wait = psfPeakVal || psfPeakPos || dirtyPeakVal || dirtyPeakPos;
+    bool loop = hogbom_loop_fits(ctx, width, psfWidth);
+    int launched = 0, done = 0;   // launches of the loop made, and done
+    unsigned long long pk = 0, first = 0;
     ProfScope ps(ctx, "hogbom");
-    st = launch_fill_u32(ctx, keys, 0u, loop ? 64 + resB / 4 : 64);
-    if (st != TCV_OK) return st;
-    hipLaunchKernelGGL(k_peak_complex<true>, dim3(stream_blocks(ctx, pn, 8)), dim3(256), 0, ctx->stream,
-                       (const float2 *)d_psf, pn, psf, keys + 3);
-    TCV_HIP(ctx, hipGetLastError());
-    unsigned long long first = 0;
-    int failed = 0;
-    if (loop) {
-        HogbomLoop a{(float2 *)d_residual, psf, (float2 *)d_model, keys + 3, (unsigned long long *)rest,
-                     keys, (int *)(keys + 8), (int)width, (int)psfWidth, niters, 0, gain};
-        st = launch_hogbom_loop(ctx, a);
+    for (;;) {
+        // PSF plane | keys, launches done | count of finished workgroups and slots
+        // of the loop, or residual plane
+        const size_t psfB = ((size_t)(pn + 2 * kPsfPad) * 4 + 255) & ~size_t(255);
+        const size_t resB =
+            loop ? 256 + 2 * kSlots * sizeof(unsigned long long) : ((size_t)n * 4 + 255) & ~size_t(255);
+        void *ws;
+        tcv_status st = major_ws(ctx, psfB + 256 + resB, &ws);
         if (st != TCV_OK) return st;
-        if (dirtyPeakVal || dirtyPeakPos)
-            TCV_HIP(ctx, hipMemcpyAsync(&first, keys, 8, hipMemcpyDeviceToHost, ctx->stream));
-        if (psfPeakVal || psfPeakPos || dirtyPeakVal || dirtyPeakPos)
-            TCV_HIP(ctx, hipMemcpyAsync(&failed, a.fail, 4, hipMemcpyDeviceToHost, ctx->stream));
-    } else {
+        float *psf = (float *)ws + kPsfPad;
+        unsigned long long *keys = (unsigned long long *)((char *)ws + psfB);
+        void *rest = (char *)ws + psfB + 256;
+        st = launch_fill_u32(ctx, keys, 0u, loop ? 64 + resB / 4 : 64);
+        if (st != TCV_OK) return st;
+        hipLaunchKernelGGL(k_peak_complex<true>, dim3(stream_blocks(ctx, pn, 8)), dim3(256), 0, ctx->stream,
+                           (const float2 *)d_psf, pn, psf, keys + 3);
+        TCV_HIP(ctx, hipGetLastError());
+        if (loop) {
+            HogbomLoop a{(float2 *)d_residual, psf, (float2 *)d_model, keys + 3,
+                         (unsigned long long *)((char *)rest + 256), keys, (unsigned *)rest, (int *)(keys + 8),
+                         nullptr, ctx->waitPolls, (int)width, (int)psfWidth, 0, 0, 0, gain};
+            if (!wait && (st = late_flag(ctx, &a.hostFail)) != TCV_OK) return st;
+            do {
+                a.chunk = launched;
+                a.niters = std::min(niters - launched * kLoopIters, kLoopIters);
+                if (launched && (st = launch_fill_u32(ctx, rest, 0u, resB / 4)) != TCV_OK) return st;
+                const hipError_t e = launch_hogbom_loop(ctx, a);
+                if (e != hipSuccess && !launched) break;   // not launched together: one launch an iteration
+                TCV_HIP(ctx, e);
+                ++launched;
+            } while (launched * (long long)kLoopIters < niters);
+            if (!launched) {
+                (void)hipGetLastError();
+                loop = false;
+                continue;
+            }
+            if (wait) {
+                TCV_HIP(ctx, hipMemcpyAsync(&first, keys, 8, hipMemcpyDeviceToHost, ctx->stream));
+                TCV_HIP(ctx, hipMemcpyAsync(&pk, keys + 3, 8, hipMemcpyDeviceToHost, ctx->stream));
+                TCV_HIP(ctx, hipMemcpyAsync(&done, a.chunks, 4, hipMemcpyDeviceToHost, ctx->stream));
+                if ((st = ctx_wait(ctx)) != TCV_OK) return st;
+                if (done < launched) {   // a wait ran out: the rest in one launch an iteration
+                    loop = false;
+                    continue;
+                }
+            }
+            break;
+        }
         float *res = (float *)rest;
         hipLaunchKernelGGL(k_peak_complex<true>, dim3(stream_blocks(ctx, n, 8)), dim3(256), 0, ctx->stream,
                            (const float2 *)d_residual, n, res, keys + 0);
         TCV_HIP(ctx, hipGetLastError());
-        if (dirtyPeakVal || dirtyPeakPos)
-            TCV_HIP(ctx, hipMemcpyAsync(&first, keys, 8, hipMemcpyDeviceToHost, ctx->stream));
+        if (wait && !done) TCV_HIP(ctx, hipMemcpyAsync(&first, keys, 8, hipMemcpyDeviceToHost, ctx->stream));
         HogbomArgs a{res, psf, (float2 *)d_model, keys, (int)width, (int)psfWidth, gain};
         // four pixels a thread when the rows are whole float4s
         const bool vec = width % 4 == 0;
         const long long perRow = vec ? width / 4 : width;
         const int bx = (int)std::min<long long>((perRow + 255) / 256, 64);
         const int by = (int)std::max<long long>(1, std::min<long long>(width, (long long)ctx->cus * 8 / bx));
-        for (int i = 0; i < niters; ++i) {
+        for (int i = 0; i < niters - done * kLoopIters; ++i) {
             if (vec)
                 hipLaunchKernelGGL(k_hogbom_step<true>, dim3(bx, by), dim3(256), 0, ctx->stream, a, i);
             else
@@ -719,13 +803,13 @@ tcv_status tcv_hogbom(tcv_ctx *ctx, float *d_residual, long long width, const fl
         hipLaunchKernelGGL(k_real_writeback, dim3(stream_blocks(ctx, n, 4)), dim3(256), 0, ctx->stream,
                            (float2 *)d_residual, (const float *)res, n);
         TCV_HIP(ctx, hipGetLastError());
+        if (wait) {
+            TCV_HIP(ctx, hipMemcpyAsync(&pk, keys + 3, 8, hipMemcpyDeviceToHost, ctx->stream));
+            if ((st = ctx_wait(ctx)) != TCV_OK) return st;
+        }
+        break;
     }
-    unsigned long long pk = 0;
-    if (psfPeakVal || psfPeakPos)
-        TCV_HIP(ctx, hipMemcpyAsync(&pk, keys + 3, 8, hipMemcpyDeviceToHost, ctx->stream));
-    if (psfPeakVal || psfPeakPos || dirtyPeakVal || dirtyPeakPos) {
-        TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (failed) return tcv_fail(ctx, TCV_ERR_DEVICE, "tcv_hogbom: the workgroups lost each other");
+    if (wait) {
         auto val = [](unsigned long long k) {
             const unsigned a2 = (unsigned)(k >> 33);
             float f;

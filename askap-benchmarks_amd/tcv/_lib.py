@@ -67,6 +67,7 @@ SIGS = {
     "tcv_status_string": (ct.c_char_p, [I]),
     "tcv_device_cus": (I, [P]),
     "tcv_synchronize": (I, [P]),
+    "tcv_set_wait_limit": (I, [P, ct.c_ulonglong]),
     "tcv_malloc": (I, [P, ct.c_size_t, ct.POINTER(P)]),
     "tcv_free": (I, [P, P]),
     "tcv_upload": (I, [P, P, P, ct.c_size_t]),

@@ -62,6 +62,11 @@ class Context:
     def sync(self):
         self.check(lib().tcv_synchronize(self.h), "synchronize")
 
+    def set_wait_limit(self, polls: int):
+        """Longest wait of a launch whose workgroups wait for each other, in
+        polls of about a microsecond (tcv_set_wait_limit)."""
+        self.check(lib().tcv_set_wait_limit(self.h, int(polls)), "set_wait_limit")
+
     # -- memory -------------------------------------------------------------
     def empty(self, shape, dtype) -> "DeviceArray":
         return DeviceArray(self, shape, dtype)

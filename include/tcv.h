@@ -50,6 +50,11 @@ const char *tcv_status_string(tcv_status s);
 /* Number of compute units of the context's device. */
 int tcv_device_cus(const tcv_ctx *ctx);
 tcv_status tcv_synchronize(tcv_ctx *ctx);
+/* Longest wait of a launch whose workgroups wait for each other (tcv_hogbom's
+ * loop), in polls of about a microsecond (default 2^24).  The launch is
+ * cooperative, so the limit is met only where another process keeps part of
+ * the device for that long; 0: such launches give up at once. */
+tcv_status tcv_set_wait_limit(tcv_ctx *ctx, unsigned long long polls);
 
 /* ---- device memory -------------------------------------------------------- */
 
@@ -475,7 +480,12 @@ tcv_status tcv_find_peak(tcv_ctx *ctx, const float *d_image, long long nPixels,
  * offset follows the reference (ry - px), and PSF rows it would place outside
  * the PSF are skipped.  No host round trip per iteration.  The four peak
  * outputs (PSF peak, first residual peak) may be NULL; when any is given the
- * call blocks until the loop has finished.  Widths below 65536. */
+ * call blocks until the loop has finished, and goes on with one launch an
+ * iteration where the wait limit was met (tcv_set_wait_limit).  With all four
+ * NULL that is TCV_ERR_DEVICE from the next tcv_synchronize, tcv_download,
+ * tcv_timer_stop, tcv_find_peak or blocking tcv_hogbom; residual and model
+ * then hold the iterations done before, whole multiples of 1024 (or none).
+ * Widths below 65536. */
 tcv_status tcv_hogbom(tcv_ctx *ctx, float *d_residual, long long width, const float *d_psf,
                       long long psfWidth, float *d_model, int niters, float gain,
                       float *psfPeakVal, long long *psfPeakPos, float *dirtyPeakVal,

@@ -117,6 +117,51 @@ def test_hogbom_small_psf_and_off_diagonal_peak(ctx, g, pw):
     assert np.array_equal(d_model.download(), m_ref)
 
 
+@pytest.mark.parametrize("g,niters", [(64, 1024), (64, 1025), (37, 2100), (300, 0)])
+@pytest.mark.parametrize("peaks", [True, False])
+def test_hogbom_many_iterations(ctx, g, niters, peaks):
+    """Up to and beyond the iterations of one launch, most of them at pixels that
+    earlier ones cleaned; and none."""
+    dirty, psf = _dirty_and_psf(g + niters, g, nSrc=5)
+    model0 = np.full_like(dirty, 0.125 - 1j)
+    r_ref, m_ref, pk_ref, _ = O.deconvolve(dirty, psf, model0, niters, 0.1)
+    dk_ref = O.find_peak(dirty)   # (the oracle's loop notes it in its first iteration)
+    d_res, d_psf, d_model = ctx.to_device(dirty), ctx.to_device(psf), ctx.to_device(model0)
+    got = M.deconvolve(ctx, d_res, g, d_psf, g, d_model, niters, 0.1, peaks=peaks)
+    assert got == ((pk_ref, dk_ref) if peaks else None)
+    assert np.array_equal(d_res.download(), r_ref)
+    assert np.array_equal(d_model.download(), m_ref)
+
+
+@pytest.mark.parametrize("g,niters", [(64, 50), (101, 1500)])
+def test_hogbom_wait_limit(g, niters):
+    """A loop whose workgroups may not wait for each other at all: a call that asks
+    for the peaks finishes by one launch an iteration, one that doesn't reports it
+    at the next waiting call and leaves residual and model alone."""
+    dirty, psf = _dirty_and_psf(g, g)
+    model0 = np.full_like(dirty, 0.5)
+    r_ref, m_ref, pk_ref, dk_ref = O.deconvolve(dirty, psf, model0, niters, 0.1)
+    with tcv.Context(0) as c:
+        d_psf = c.to_device(psf)
+        c.set_wait_limit(0)
+        d_res, d_model = c.to_device(dirty), c.to_device(model0)
+        assert M.deconvolve(c, d_res, g, d_psf, g, d_model, niters, 0.1) == (pk_ref, dk_ref)
+        assert np.array_equal(d_res.download(), r_ref)
+        assert np.array_equal(d_model.download(), m_ref)
+        for waiting in (c.sync, lambda: d_res.download(), lambda: M.findPeak(c, d_psf)):
+            d_res, d_model = c.to_device(dirty), c.to_device(model0)
+            M.deconvolve(c, d_res, g, d_psf, g, d_model, niters, 0.1, peaks=False)
+            with pytest.raises(tcv.TcvError, match="hogbom"):
+                waiting()
+            c.sync()   # reported once
+            assert np.array_equal(d_res.download(), dirty)
+            assert np.array_equal(d_model.download(), model0)
+        c.set_wait_limit(1 << 24)
+        M.deconvolve(c, d_res, g, d_psf, g, d_model, niters, 0.1, peaks=False)
+        assert np.array_equal(d_res.download(), r_ref)
+        assert np.array_equal(d_model.download(), m_ref)
+
+
 def test_hogbom_twice_reuses_workspace(ctx):
     dirty, psf = _dirty_and_psf(5, 128)
     for niters in (30, 7):
