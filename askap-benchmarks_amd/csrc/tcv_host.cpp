@@ -677,6 +677,7 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
     // cut 11.9).
     const bool adapt = !tilesOnly && open_shape(t) && t.item_entries <= 0;
     if (tilesOnly && t.item_entries <= 0) t.item_entries = kItemEntriesFixed;
+    sh.widened = 0;
     if (adapt && maxS >= 48 && t.tap_bytes != 4) {
         // Open FP32 plans of many entries take 128 x 64 tiles from width 48 up: a
         // quarter fewer entries, once phases and chunks fit the job.  Grid + degrid in
@@ -694,6 +695,7 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
         if (least >= 2 && tiles >= 128 && entries_expected(g, sh) > kAdaptItems * kAdaptChunk) {
             t.tile_w = 128;
             t.tile_h = 64;
+            sh.widened = maxS < kWideTileMinWidth;
         }
     }
     sh.colsOpen = t.grid_cols <= 0;
@@ -1084,32 +1086,46 @@ tcv_status tcv_degrid_tiled_half(tcv_ctx *ctx, tcv_plan *p, const float *d_grid,
 
 // ---- batching ------------------------------------------------------------------
 
+static void free_batch(tcv_batch *b)
+{
+    for (tcv_batch *t : {b, b->wide.get()}) {
+        if (!t) continue;
+        for (JobDesc *d : {t->d_jobs, t->d_jobsD, t->d_narrow[0], t->d_narrow[1]})
+            if (d) (void)hipFree(d);
+        if (t->d_prefix) (void)hipFree(t->d_prefix);
+        if (t->d_queue) (void)hipFree(t->d_queue);
+    }
+    delete b;
+}
+
 tcv_status tcv_batch_create(tcv_ctx *ctx, int nJobs, const tcv_job *jobs, tcv_batch **out)
 {
     if (!ctx || !out || nJobs < 1 || !jobs) return tcv_fail(ctx, TCV_ERR_INVALID, "tcv_batch_create: bad argument");
     *out = nullptr;
-    tcv_batch *b = new tcv_batch();
-    std::vector<JobDesc> tiled, tiledD, narrow[2];
+    std::unique_ptr<tcv_batch, void (*)(tcv_batch *)> b(new tcv_batch(), free_batch);
+    b->wide.reset(new tcv_batch());
+    std::vector<JobDesc> tiled[2], tiledD[2], narrow[2];   // [1]: of widened plans
     bool open = true;   // every plan leaves grid_cols open
     for (int j = 0; j < nJobs; j++) {
         const tcv_job &J = jobs[j];
-        if (!J.plan || !J.d_C || !J.d_grid) {
-            delete b;
+        if (!J.plan || !J.d_C || !J.d_grid)
             return tcv_fail(ctx, TCV_ERR_INVALID, "tcv_batch_create: job " + std::to_string(j) + " incomplete");
-        }
+        const PlanShape &sh = J.plan->sh;
+        // the shape by widths alone: which of the two a widened plan's size chose
+        // doesn't matter here
+        const int tw = sh.widened ? 64 : sh.tw, th = sh.widened ? 64 : sh.th;
         if (j == 0) {
-            b->tw = J.plan->sh.tw;
-            b->th = J.plan->sh.th;
-            b->kern = J.plan->sh.kern;
-            b->dkern = J.plan->sh.dkern;
-            b->gridCols = J.plan->sh.gridCols;
-        } else if (J.plan->sh.tw != b->tw || J.plan->sh.th != b->th || J.plan->sh.kern != b->kern ||
-                   J.plan->sh.dkern != b->dkern || J.plan->sh.gridCols != b->gridCols) {
-            delete b;
+            b->tw = tw;
+            b->th = th;
+            b->kern = sh.kern;
+            b->dkern = sh.dkern;
+            b->gridCols = sh.gridCols;
+        } else if (tw != b->tw || th != b->th || sh.kern != b->kern || sh.dkern != b->dkern ||
+                   sh.gridCols != b->gridCols) {
             return tcv_fail(ctx, TCV_ERR_INVALID,
                             "tcv_batch_create: all plans of a batch need one tile shape, kernel and grid_cols");
         }
-        open = open && J.plan->sh.colsOpen;
+        open = open && sh.colsOpen;
         b->plans.push_back(J.plan);
         b->host.push_back(make_job_desc(J.plan, true, J.d_data, J.d_C, (float2 *)J.d_grid, (float2 *)J.d_out, nullptr));
         b->hostD.push_back(make_job_desc(J.plan, false, J.d_data, J.d_C, (float2 *)J.d_grid, (float2 *)J.d_out, nullptr));
@@ -1129,39 +1145,45 @@ tcv_status tcv_batch_create(tcv_ctx *ctx, int nJobs, const tcv_job *jobs, tcv_ba
         if (J.plan->sh.region > 0) {
             by_regions(J.plan);
         } else {
-            tiled.push_back(b->host[j]);
-            tiledD.push_back(b->hostD[j]);
+            tiled[J.plan->sh.widened].push_back(b->host[j]);
+            tiledD[J.plan->sh.widened].push_back(b->hostD[j]);
         }
     }
     // Jobs of many widths on 128 x 64 tiles: groups of 32 columns waste fewer lanes
     // on the narrower ones (gridding 16 jobs of widths 63-131: 20.6 ms with 64, 19.5
     // with 32; 10 jobs 7.4 and 7.0; one job of width 129: equal).
     if (open && b->tw == 128 && b->th == 64) b->gridCols = 32;
-    b->nJobs = (int)tiled.size();
-    auto fail = [&](const char *m) {
-        if (b->d_jobs) (void)hipFree(b->d_jobs);
-        if (b->d_jobsD) (void)hipFree(b->d_jobsD);
-        if (b->d_prefix) (void)hipFree(b->d_prefix);
-        if (b->d_queue) (void)hipFree(b->d_queue);
-        for (JobDesc *d : b->d_narrow)
-            if (d) (void)hipFree(d);
-        delete b;
-        return tcv_fail(ctx, TCV_ERR_NOMEM, m);
-    };
+    // Widened plans in a launch of their own.  Gridding eight jobs of width 63, 5000 to
+    // 400 000 visibilities, three of them widened: 3.42 ms with groups of 32 columns,
+    // 3.87 with 64 (all on 64 x 64 tiles 3.32, and degridding 2.58 against 2.53); twelve
+    // of width 49, five widened: 4.80, 5.44 (4.77, and 3.38 against 3.12).
+    b->wide->tw = 128;
+    b->wide->th = 64;
+    b->wide->kern = b->kern;
+    b->wide->dkern = b->dkern;
+    b->wide->gridCols = 32;
     auto upload = [](JobDesc **d, const std::vector<JobDesc> &v) {
         return hipMalloc((void **)d, sizeof(JobDesc) * std::max<size_t>(1, v.size())) == hipSuccess &&
                (v.empty() || hipMemcpy(*d, v.data(), sizeof(JobDesc) * v.size(), hipMemcpyHostToDevice) == hipSuccess);
     };
-    if (!upload(&b->d_jobs, tiled) || !upload(&b->d_jobsD, tiledD) ||
-        hipMalloc((void **)&b->d_prefix, sizeof(int) * 9 * (b->nJobs + 1)) != hipSuccess ||
-        hipMalloc((void **)&b->d_queue, kBatchQueueBytes) != hipSuccess)
-        return fail("tcv_batch_create: allocation or upload failed");
+    if (tiled[1].empty()) b->wide.reset();
+    bool ok = true;
+    for (int k = 0; k < (b->wide ? 2 : 1); ++k) {
+        tcv_batch *t = k ? b->wide.get() : b.get();
+        t->nJobs = (int)tiled[k].size();
+        ok = ok && upload(&t->d_jobs, tiled[k]) && upload(&t->d_jobsD, tiledD[k]) &&
+             hipMalloc((void **)&t->d_prefix, sizeof(int) * 9 * (t->nJobs + 1)) == hipSuccess &&
+             hipMalloc((void **)&t->d_queue, kBatchQueueBytes) == hipSuccess;
+    }
     for (int r = 0; r < 2; ++r) {
         b->nNarrow[r] = (int)narrow[r].size();
-        if (b->nNarrow[r] && !upload(&b->d_narrow[r], narrow[r]))
-            return fail("tcv_batch_create: allocation or upload failed");
+        ok = ok && (!b->nNarrow[r] || upload(&b->d_narrow[r], narrow[r]));
     }
-    *out = b;
+    if (!ok) {
+        (void)hipGetLastError();
+        return tcv_fail(ctx, TCV_ERR_NOMEM, "tcv_batch_create: allocation or upload failed");
+    }
+    *out = b.release();
     return TCV_OK;
 }
 
@@ -1171,13 +1193,7 @@ tcv_status tcv_batch_destroy(tcv_ctx *ctx, tcv_batch *b)
     if (!b) return TCV_OK;
     TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (b->graph) (void)hipGraphExecDestroy(b->graph);
-    (void)hipFree(b->d_jobs);
-    (void)hipFree(b->d_jobsD);
-    (void)hipFree(b->d_prefix);
-    (void)hipFree(b->d_queue);
-    for (JobDesc *d : b->d_narrow)
-        if (d) (void)hipFree(d);
-    delete b;
+    free_batch(b);
     return TCV_OK;
 }
 

@@ -177,6 +177,9 @@ struct PlanShape {
     int itemEntries;       // entries per work item the automatic phase counts aimed at
     int gridCols;          // pair gridder: columns per load instruction (tcv_tuning.grid_cols)
     int colsOpen;          // 1: the tuning left gridCols open (a batch may take other groups)
+    // 1: an open plan on 128 x 64 tiles for its size, where its widths alone give
+    // 64 x 64 (batches take it beside plans on those)
+    int widened;
     // narrow-kernel plans (tcv_narrow.hip): cells a side of the regions, which
     // overlap so that each footprint lies in one; 0: tiles of tw x th
     int region;
@@ -241,7 +244,7 @@ bool plan_two_level(const PlanShape &sh);
 constexpr int kRegions[] = {32, 48};   // region sizes built (cells a side)
 
 struct tcv_batch {
-    int nJobs = 0;      // jobs that have tiles: d_jobs, d_jobsD
+    int nJobs = 0;      // jobs that have tiles of tw x th: d_jobs, d_jobsD
     int tw = 0, th = 0, kern = kDefaultGridKernel, dkern = kDefaultDegridKernel;
     int gridCols = 0;   // pair gridder column groups (PlanShape::gridCols of every plan)
     bool half = false;
@@ -250,6 +253,8 @@ struct tcv_batch {
     // the jobs' parts by regions, one list per region size
     JobDesc *d_narrow[2] = {nullptr, nullptr};
     int nNarrow[2] = {0, 0};
+    // the jobs of widened plans, with their own device arrays and queue
+    std::unique_ptr<tcv_batch> wide;
     JobDesc *d_jobs = nullptr, *d_jobsD = nullptr;
     int *d_prefix = nullptr;      // 9 x (nJobs + 1): item prefix, then one per XCD
     int *d_queue = nullptr;       // kBatchQueueBytes: the queue and the per-XCD counters

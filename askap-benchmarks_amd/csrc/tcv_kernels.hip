@@ -2571,6 +2571,9 @@ tcv_status launch_degrid_tiled(tcv_ctx *ctx, tcv_plan *p, const float2 *grid, co
     return tcv_fail(ctx, TCV_ERR_UNSUPPORTED, "tile shape not built");
 }
 
+// the jobs of one tile shape
+static tcv_status launch_batch_tiles(tcv_ctx *ctx, tcv_batch *b, bool degrid);
+
 tcv_status launch_batch(tcv_ctx *ctx, tcv_batch *b, bool degrid)
 {
     if (degrid)
@@ -2583,6 +2586,13 @@ tcv_status launch_batch(tcv_ctx *ctx, tcv_batch *b, bool degrid)
         tcv_status st = launch_narrow_many(ctx, b->d_narrow[r], b->nNarrow[r], kRegions[r], degrid);
         if (st != TCV_OK) return st;
     }
+    tcv_status st = launch_batch_tiles(ctx, b, degrid);
+    if (st == TCV_OK && b->wide) st = launch_batch_tiles(ctx, b->wide.get(), degrid);
+    return st;
+}
+
+static tcv_status launch_batch_tiles(tcv_ctx *ctx, tcv_batch *b, bool degrid)
+{
     if (!b->nJobs) return TCV_OK;
     hipLaunchKernelGGL(k_batch_prefix, dim3(1), dim3(64), 0, ctx->stream,
                        (const JobDesc *)(degrid ? b->d_jobsD : b->d_jobs), b->nJobs, b->d_prefix,

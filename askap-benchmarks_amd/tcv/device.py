@@ -372,7 +372,8 @@ class Batch:
     """Many jobs in one persistent launch over a device work queue (tcv_batch).
 
     jobs: sequence of (plan, data, C, grid, out) with DeviceArrays (data or
-    out may be None).  All plans must share one tile shape."""
+    out may be None).  All plans must share one tile shape (open plans of
+    widths 48 to 88 count as 64 x 64 ones)."""
 
     def __init__(self, ctx: Context, jobs):
         self.ctx = ctx

@@ -361,7 +361,9 @@ tcv_status tcv_degrid_tiled_half(tcv_ctx *ctx, tcv_plan *plan, const float *d_gr
  * Taylor terms, snapshots) of uneven size share one launch over a device work
  * queue. */
 typedef struct {
-    tcv_plan *plan;        /* built plan of the job; all plans of a batch share tile_w/tile_h */
+    tcv_plan *plan;        /* built plan of the job; all plans of a batch share tile_w/tile_h,
+                              kernels and grid_cols.  (Open plans of widths 48 to 88
+                              count as 64 x 64 on whichever tiles their size chose.) */
     const float *d_data;   /* complex64 visibilities to grid (may be NULL: degrid only) */
     const float *d_C;      /* complex64 C(w) taps of the job */
     float *d_grid;         /* complex64 gSize^2 grid (gridding accumulates into it) */

@@ -207,6 +207,49 @@ def test_adaptive_work_items(ctx, Sz, gSize, nVis, cluster, os_, planes):
         (info["items"], info["entries"], info["phases"], info["chunk"])
 
 
+def test_widened_plans_in_a_batch(ctx):
+    """Open plans of one width on either side of the size from which they take
+    128 x 64 tiles, beside one given 64 x 64: one batch, two of the jobs on one
+    grid.  Given 128 x 64 tiles stay refused."""
+    from helpers import exact_problem
+    from tcv.device import Batch
+    Sz, hold, ref, plans = 49, [], [], []
+    grids = {g: ctx.zeros((g, g), np.complex64) for g in (1100, 300)}
+    sums = {g: np.zeros((g, g), np.complex64) for g in grids}
+    for seed, (nVis, gSize, tuning) in enumerate([(3000, 1100, {}), (140000, 1100, {}), (2000, 300, dict(tile_w=64))]):
+        iu, iv, co, data, C, grid = exact_problem(seed, nVis, gSize, Sz, cluster=None)
+        plans.append(tcv.Plan(ctx, tcv.Visibilities(ctx, iu, iv, co, [Sz], gSize, C.size), **tuning))
+        hold.append((plans[-1], ctx.to_device(data), ctx.to_device(C), grids[gSize], ctx.empty(nVis, np.complex64)))
+        ref.append((iu, iv, co, C, grid, gSize))
+        O.grid(data, iu, iv, co, C, gSize, Sz, out=sums[gSize])
+    assert [p.info()["tile_w"] for p in plans] == [64, 128, 64]
+    given = tcv.Plan(ctx, plans[1].vis, tile_w=128)
+    for pair in ([(given,) + hold[1][1:], hold[0]], [hold[1], (given,) + hold[1][1:]]):
+        with pytest.raises(tcv.TcvError, match="one tile shape"):
+            Batch(ctx, pair)
+    for pick in ([0, 1, 2], [2, 1, 0]):
+        b = Batch(ctx, [hold[k] for k in pick])
+        for rep in range(3):   # captured once, replayed
+            for g in grids.values():
+                g.zero()
+            b.run_graph(3)
+            for gSize, g in grids.items():
+                assert np.array_equal(g.download(), sums[gSize]), (pick, rep)
+        b.close()
+    for gSize, g in grids.items():   # degridding one image into every job's output
+        g.upload(ref[1 if gSize == 1100 else 2][4])
+    want = [O.degrid(grids[gSize].download(), iu, iv, co, C, Sz) for iu, iv, co, C, _, gSize in ref]
+    for pick in ([0, 1, 2], [1]):
+        for h in hold:
+            h[4].zero()
+        b = Batch(ctx, [hold[k] for k in pick])
+        b.rebuild()
+        b.degrid()
+        for k in pick:
+            assert np.array_equal(hold[k][4].download(), want[k]), (pick, k)
+        b.close()
+
+
 def test_adaptive_plan_of_nothing(ctx):
     """Every visibility out of range: no items, cleared results."""
     vis = tcv.Visibilities(ctx, [1, 2], [0, 0], [0, 0], [65], 100, 65 * 65)
