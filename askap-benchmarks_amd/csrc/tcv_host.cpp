@@ -682,17 +682,24 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
         // Open FP32 plans of many entries take 128 x 64 tiles from width 48 up: a
         // quarter fewer entries, once phases and chunks fit the job.  Grid + degrid in
         // us, 64 x 64 and 128 x 64: width 63, 100 003 visibilities, 2047^2 481 + 379 and
-        // 448 + 350; 49, 200 000, 4096^2 596 + 474 and 575 + 385; 87, 200 000, 2000^2 1110
-        // + 867 and 1028 + 716 (FP16, width 129, 160 000, 4096^2, a whole pass 2174 and
-        // 2214).  With fewer entries, or on few tiles, the smaller ones share out better:
-        // 49, 30 000, 600^2 135 + 81 and 174 + 72; 87, 66 000, 2000^2 582 + 360 and 522 + 507.
+        // 448 + 350; 49, 200 000, 2048^2 935 and 811; 65, 400 000, 2048^2 2114 and 2048;
+        // 81, 400 000, 4096^2 4276 and 3596; 87, 200 000, 2000^2 1110 + 867 and 1028 +
+        // 716.  With fewer entries, or on few tiles, the smaller ones share out better:
+        // 49, 30 000, 600^2 135 + 81 and 174 + 72; 87, 66 000, 2000^2 582 + 360 and 522 +
+        // 507.  Below width 72 only up to 1024 tiles: FP16 launches on such a plan (made
+        // without tap_bytes 4) lose more there than FP32 ones gain: 49, 400 000, 4096^2
+        // FP16 897 + 615 and 1050 + 604 (FP32 1840 and 1621); 49, 400 000, 8192^2 966 + 810
+        // and 1104 + 1002 (2478 and 2317); 65, 100 000, 4096^2 413 + 341 and 416 + 453
+        // (1130 and 1062).  65, 200 000, 2048^2 657 + 461 and 706 + 428; 73, 100 000, 4096^2
+        // 506 + 385 and 464 + 495.
         sh.maxS = maxS;
         sh.tw = 128;
         sh.th = 64;
         const long long tiles = (long long)((g->gSize + 127) / 128) * ((g->gSize + 63) / 64);
         int least = maxS;
         for (int k = 0; k < g->nPlanes; k++) least = std::min(least, g->sSize[k]);
-        if (least >= 2 && tiles >= 128 && entries_expected(g, sh) > kAdaptItems * kAdaptChunk) {
+        if (least >= 2 && tiles >= 128 && (maxS >= 72 || tiles <= 1024) &&
+            entries_expected(g, sh) > kAdaptItems * kAdaptChunk) {
             t.tile_w = 128;
             t.tile_h = 64;
             sh.widened = maxS < kWideTileMinWidth;

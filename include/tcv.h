@@ -233,7 +233,8 @@ tcv_status tcv_range_errors(tcv_ctx *ctx, long long *count);
 typedef struct {
     int tile_w;      /* 8, 16, 32, 64 or 128 columns (0 = auto: 128 x 64 tiles for
                         kernels 89 wide and up when the pair kernels apply, and, with
-                        every field open, 48 and up on jobs of many entries); 128-wide
+                        every field open, 72 and up on jobs of many entries, 48 and
+                        up where the grid has no more than 1024 such tiles); 128-wide
                         tiles take only the pair kernels (kernel and degrid_kernel 3) */
     int tile_h;      /* rows per tile: 32 or 64 for tiles 8..64 wide, 64 for 128-wide
                         tiles, and the tall shapes 64 x 128 and 32 x 256 (pair kernels

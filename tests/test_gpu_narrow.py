@@ -207,6 +207,20 @@ def test_adaptive_work_items(ctx, Sz, gSize, nVis, cluster, os_, planes):
         (info["items"], info["entries"], info["phases"], info["chunk"])
 
 
+@pytest.mark.parametrize("Sz,gSize,nVis,tile_w", [
+    (49, 2048, 200000, 128), (71, 2048, 100000, 128), (71, 2816, 200000, 128), (71, 2944, 200000, 64), (49, 4096, 400000, 64),
+    (72, 4096, 200000, 128), (72, 4096, 50000, 64), (65, 900, 200000, 64)])
+def test_open_tile_shape(ctx, Sz, gSize, nVis, tile_w):
+    """128 x 64 tiles from width 72 up, and from 48 up to 1024 of them (2816^2 has
+    968, 2944^2 1058), for more than 262 144 entries on 128 and more of them.  A plan
+    made for FP16 stays on 64 x 64."""
+    rng = np.random.default_rng(Sz)
+    iu = rng.integers(Sz, gSize - Sz, nVis).astype(np.int32)
+    vis = tcv.Visibilities(ctx, iu, iu, np.zeros(nVis, np.int32), [Sz], gSize, Sz * Sz * 4)
+    assert tcv.Plan(ctx, vis).info()["tile_w"] == tile_w
+    assert tcv.Plan(ctx, vis, tap_bytes=4).info()["tile_w"] == 64
+
+
 def test_widened_plans_in_a_batch(ctx):
     """Open plans of one width on either side of the size from which they take
     128 x 64 tiles, beside one given 64 x 64: one batch, two of the jobs on one
