@@ -402,9 +402,25 @@ __global__ __launch_bounds__(SCAN_BS) void k_scan_apply(const int *__restrict__ 
     const long long base = (long long)blockIdx.x * SCAN_TILE + (long long)threadIdx.x * SCAN_IPT;
     int vals[SCAN_IPT];
     int t = 0, some = 0;
+    // whole runs by 16-byte accesses: by 4 bytes a wave's stores are 64 bytes apart
+    // (33.5 M counters and their copy 344 us, 98 so).  Not every array is aligned to 16.
+    const bool full = base + SCAN_IPT <= n;
+    if (full) {
+#pragma unroll
+        for (int k = 0; k < SCAN_IPT; k += 4) {
+            int4 q;
+            __builtin_memcpy(&q, in + base + k, 16);
+            vals[k] = q.x;
+            vals[k + 1] = q.y;
+            vals[k + 2] = q.z;
+            vals[k + 3] = q.w;
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < SCAN_IPT; ++k) vals[k] = base + k < n ? in[base + k] : 0;
+    }
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; ++k) {
-        vals[k] = (base + k < n) ? in[base + k] : 0;
         t += vals[k];
         some += vals[k] != 0;
     }
@@ -417,11 +433,23 @@ __global__ __launch_bounds__(SCAN_BS) void k_scan_apply(const int *__restrict__ 
     int run = block_exclusive_scan(t, &total) + before;
 #pragma unroll
     for (int k = 0; k < SCAN_IPT; ++k) {
-        if (base + k < n) {
-            out[base + k] = run;
-            if (out2) out2[base + k] = run;
+        const int v = vals[k];
+        vals[k] = run;
+        run += v;
+    }
+    for (int *o : {out, out2}) {
+        if (!o) continue;
+        if (full) {
+#pragma unroll
+            for (int k = 0; k < SCAN_IPT; k += 4) {
+                const int4 q = make_int4(vals[k], vals[k + 1], vals[k + 2], vals[k + 3]);
+                __builtin_memcpy(o + base + k, &q, 16);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < SCAN_IPT; ++k)
+                if (base + k < n) o[base + k] = vals[k];
         }
-        run += vals[k];
     }
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == SCAN_BS - 1) out[n] = run;
 }
@@ -439,16 +467,29 @@ struct PlanDevArgs {
 
 // The cOffset range of the binned entries, for phases over the part of the
 // table in use: meta[4] = max(0x7fffffff - c0), meta[5] = max(c0 + 1), so the
-// zeroed counters read as an empty range.  One atomic pair per wave, where the
-// wave widens the range: atomics on one address take 12 ns each, one after the
-// other (5.4 M visibilities, every wave of a first pass: 130 us of a 150 us pass).
+// zeroed counters read as an empty range.  One atomic pair per block (of 256
+// threads, which all call), where the block widens the range: atomics on one
+// address take 12 ns each, one after the other (5.4 M visibilities, every wave of a
+// first pass: 130 us of a 150 us pass; 200 000, whose waves are all in flight and
+// widen it: 90 of 115 us).
 __device__ __forceinline__ void note_c_range(int cLo, int cHi, int *meta)
 {
     for (int o = 32; o > 0; o >>= 1) {
         cLo = min(cLo, __shfl_xor(cLo, o, 64));
         cHi = max(cHi, __shfl_xor(cHi, o, 64));
     }
-    if ((threadIdx.x & 63) == 0 && cHi >= 0) {
+    __shared__ int s_lo[4], s_hi[4];
+    if ((threadIdx.x & 63) == 0) {
+        s_lo[threadIdx.x >> 6] = cLo;
+        s_hi[threadIdx.x >> 6] = cHi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w) {
+            cLo = min(cLo, s_lo[w]);
+            cHi = max(cHi, s_hi[w]);
+        }
+        if (cHi < 0) return;
         const unsigned lo = 0x7fffffffu - (unsigned)cLo, hi = (unsigned)cHi + 1u;
         unsigned *m = reinterpret_cast<unsigned *>(meta + 4);
         // (a value read too early is only lower: one atomic more)

@@ -290,3 +290,23 @@ def test_plan_of_many_counters(ctx, keys, phases, nVis):
         g, o = run(ctx, plan, j)
         assert np.array_equal(g, gref) and np.array_equal(o, oref)
         plan.build()
+
+
+@pytest.mark.parametrize("gSize,keys,lone", [(1500, 3, 0), (1501, 1, 256), (1500, 7, 100)])
+def test_plan_counter_remainders(ctx, gSize, keys, lone):
+    """Counters in one level, more than a block of the scan and no multiple of a
+    thread's 16; the two ends of the part of the table in use are one visibility's
+    each, in different blocks of the kernel that notes the range."""
+    j = job(gSize + keys, [9, 12], 513, gSize, os_=8)
+    j["plane"][:] = 1   # width 12: the table's second part, 64 slices
+    first = 9 * 9 * 64
+    j["co"] = (first + np.random.default_rng(keys).integers(20, 40, 513) * 144).astype(np.int32)
+    j["co"][lone], j["co"][512] = first, first + 63 * 144
+    j["iu"], j["iv"] = np.clip(j["iu"], 6, gSize - 6), np.minimum(j["iv"], gSize - 12)
+    gref, oref = reference(j)
+    plan = tcv.Plan(ctx, visibilities(ctx, j), tile_w=8, tile_h=32, slice_keys=keys, phases=min(keys, 4),
+                    grid_phases=min(keys, 4))
+    for _ in range(2):
+        g, o = run(ctx, plan, j)
+        assert np.array_equal(g, gref) and np.array_equal(o, oref)
+        plan.build()
