@@ -723,6 +723,9 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
     sh.xcd = (t.xcd_split > 0 && sh.phases % 8 == 0) ? 1 : 0;
     sh.phasesG = std::min(t.grid_phases, sh.k2);
     sh.xcdG = (t.xcd_split > 0 && sh.phasesG % 8 == 0) ? 1 : 0;
+    // what the host chooses for tiles of every width (tcv_plan_info of a plan with regions)
+    p->tiles = tcv_tuning{sh.tw, sh.th, sh.chunk, sh.k2, sh.phases, sh.xcd, 0, 0, sh.phasesG, t.tap_bytes,
+                          t.item_entries, t.grid_cols};
     sh.adapt = adapt;
     if (adapt) {
         sh.phaseBytes = t.tile_w * t.tile_h > 4096 ? kWidePhaseBytes : kDegridPhaseBytes;
@@ -968,9 +971,17 @@ tcv_status tcv_plan_info(tcv_ctx *ctx, tcv_plan *p, tcv_tuning *t, long long *en
                          long long *items, long long *outOfRange)
 {
     if (!ctx || !p) return TCV_ERR_INVALID;
-    if (t) *t = tcv_tuning{p->sh.tw, p->sh.th, p->sh.chunk, p->sh.k2, p->sh.phases, p->sh.xcd, p->sh.kern,
-                           p->sh.dkern, p->sh.phasesG, p->sh.tapBytes, p->sh.itemEntries,
-                           p->sh.gridCols};
+    const bool regions = p->sh.region > 0 || !p->parts.empty();
+    if (t) {
+        *t = tcv_tuning{p->sh.tw, p->sh.th, p->sh.chunk, p->sh.k2, p->sh.phases, p->sh.xcd, p->sh.kern,
+                        p->sh.dkern, p->sh.phasesG, p->sh.tapBytes, p->sh.itemEntries,
+                        p->sh.gridCols};
+        if (regions) {
+            *t = p->tiles;
+            t->kernel = p->sh.kern;
+            t->degrid_kernel = p->sh.dkern;
+        }
+    }
     int meta[12] = {0};   // items, queue head, entries, out of range, ..., [9] phases [10] chunk
     TCV_HIP(ctx, hipMemcpyAsync(meta, p->meta, sizeof(meta), hipMemcpyDeviceToHost, ctx->stream));
     TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -981,7 +992,7 @@ tcv_status tcv_plan_info(tcv_ctx *ctx, tcv_plan *p, tcv_tuning *t, long long *en
         meta[0] += more[0];
         meta[2] += more[2];
     }
-    if (t && p->sh.adapt) {
+    if (t && p->sh.adapt && !regions) {
         t->phases = t->grid_phases = meta[9];
         t->chunk = meta[10];
         if (p->metaG != p->meta) {

@@ -226,6 +226,7 @@ struct tcv_plan {
     void *block = nullptr;        // one device block holding every buffer above
     char *blockEnd = nullptr;     // one past the last buffer in it
     bool ownsBlock = false;       // block from hipMalloc (else from a caller's arena)
+    tcv_tuning tiles{};           // the host's choice if every kernel took tiles (but for the kernels)
     // plans of further classes of kernel widths (by regions), in the same block
     std::vector<std::unique_ptr<tcv_plan>> parts;
 };

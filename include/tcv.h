@@ -291,7 +291,11 @@ tcv_status tcv_plan_create(tcv_ctx *ctx, const tcv_geometry *g,
 tcv_status tcv_plan_build(tcv_ctx *ctx, tcv_plan *plan, const tcv_geometry *g);
 tcv_status tcv_plan_destroy(tcv_ctx *ctx, tcv_plan *plan);
 /* The tuning the plan resolved to, and after a build the number of entries
- * (visibility x tile pairs) and work items (blocking). */
+ * (visibility x tile pairs) and work items (blocking).  A plan that takes some
+ * kernels by regions has no tuning that repeats it but the open one: it reports
+ * the tiles that a plan without regions would take, which a plan made with them
+ * then does (slower: width 15, 300 000 visibilities, 2048^2 grid + degrid
+ * 156 us by regions and 475 by those tiles). */
 tcv_status tcv_plan_info(tcv_ctx *ctx, tcv_plan *plan, tcv_tuning *tuning,
                          long long *entries, long long *items,
                          long long *outOfRange);

@@ -84,6 +84,27 @@ def test_regions_equal_oracle(ctx, widths, nVis, gSize):
     assert np.array_equal(g, gref) and np.array_equal(o, oref)
 
 
+@pytest.mark.parametrize("widths,nVis,gSize,want", [
+    # tile_w, chunk, slice_keys, phases, grid_phases by the rules for tiles
+    ([15], 30000, 300, (16, 512, 256, 1, 1)), ([27], 20000, 256, (32, 2048, 256, 1, 1)),
+    ([9, 19, 40], 9000, 260, (32, 1024, 2048, 1, 1))])
+def test_regions_report_their_tiles(ctx, widths, nVis, gSize, want):
+    """info() of a plan with regions is the tuning of the tiles in their place: a plan
+    made with it reports the same and computes the same."""
+    j = job(nVis, widths, nVis, gSize, os_=16)
+    plan = tcv.Plan(ctx, visibilities(ctx, j))
+    info = plan.info()
+    assert tuple(info[k] for k in ("tile_w", "chunk", "slice_keys", "phases", "grid_phases")) == want
+    tuning = {k: v for k, v in info.items() if k not in ("entries", "items", "out_of_range")}
+    given = tcv.Plan(ctx, visibilities(ctx, j), **tuning)
+    again = given.info()
+    assert {k: again[k] for k in tuning} == tuning and again["entries"] > info["entries"]
+    gref, oref = reference(j)
+    for p in (plan, given):
+        g, o = run(ctx, p, j)
+        assert np.array_equal(g, gref) and np.array_equal(o, oref)
+
+
 def test_regions_out_of_range(ctx):
     j = job(5, [9, 25, 65], 900, 140)
     j["iu"][:3], j["iv"][3:6], j["co"][6:9] = 0, 139, j["C"].size
