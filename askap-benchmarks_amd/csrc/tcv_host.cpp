@@ -633,8 +633,10 @@ static bool open_shape(const tcv_tuning &t)
 }
 
 tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tuning, tcv_plan *p,
-                      size_t *bytes, bool tilesOnly)
+                      size_t *bytes, PlanFor use)
 {
+    const bool tilesOnly = use != PlanFor::caller;
+    if (use == PlanFor::server) p->metaInts = kMetaIntsBatch;
     int maxS = 0;
     tcv_status st = check_geometry(ctx, g, &maxS);
     if (st != TCV_OK) return st;
@@ -816,12 +818,12 @@ static tcv_status plan_sizes(tcv_ctx *ctx, const tcv_geometry *g, tcv_plan *p, s
     n += align256(sizeof(int4) * p->maxItems);
     n += 3 * align256(sizeof(int) * (sh.nKeys + 1));
     n += 2 * align256(sizeof(int) * (slots + 1));
-    n += align256(sizeof(int) * kMetaInts);
+    n += align256(sizeof(int) * p->metaInts);
     n += align256(sizeof(int) * p->scanTmpLen);
     if (twoLists) {
         n += align256(sizeof(int4) * p->maxItemsG);
         n += 2 * align256(sizeof(int) * (slotsG + 1));
-        n += align256(sizeof(int) * kMetaInts);
+        n += align256(sizeof(int) * p->metaInts);
     }
     *bytes = n;
     return TCV_OK;
@@ -846,14 +848,14 @@ void plan_bind(tcv_plan *p, char *block)
     p->cursor = (int *)take(sizeof(int) * (sh.nKeys + 1));
     p->itemCount = (int *)take(sizeof(int) * (slots + 1));
     p->itemStart = (int *)take(sizeof(int) * (slots + 1));
-    p->meta = (int *)take(sizeof(int) * kMetaInts);
+    p->meta = (int *)take(sizeof(int) * p->metaInts);
     p->scanTmp = (int *)take(sizeof(int) * p->scanTmpLen);
     if (p->maxItemsG) {
         const long long slotsG = (long long)sh.phasesG * sh.nTiles;
         p->itemsG = (int4 *)take(sizeof(int4) * p->maxItemsG);
         p->itemCountG = (int *)take(sizeof(int) * (slotsG + 1));
         p->itemStartG = (int *)take(sizeof(int) * (slotsG + 1));
-        p->metaG = (int *)take(sizeof(int) * kMetaInts);
+        p->metaG = (int *)take(sizeof(int) * p->metaInts);
     } else {
         p->itemsG = p->items;
         p->itemCountG = p->itemCount;

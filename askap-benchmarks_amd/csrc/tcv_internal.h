@@ -148,6 +148,7 @@ constexpr int kMaxPersistentBlocks = 8192;
 // after the other (12 ns each, measured), whichever of its words they go to.
 constexpr int kHeadInts = 32;
 constexpr int kMetaInts = 32 + 8 * kHeadInts;   // a plan's meta block (see tcv_plan::meta)
+constexpr int kMetaIntsBatch = 32;               // without the queue heads
 constexpr size_t kBatchQueueBytes = 9 * kHeadInts * sizeof(int);   // the queue, then one head per XCD
 
 // Work items that the build sizes on the device: about kAdaptItems of them and no
@@ -209,7 +210,8 @@ struct tcv_plan {
     int *cursor = nullptr;        // nKeys
     int *itemCount = nullptr;     // phases * nTiles + 1
     int *itemStart = nullptr;     // phases * nTiles + 1: the item counts of blocks of slots, then those scanned
-    int *meta = nullptr;          // kMetaInts: [0] items [1] queue head [2] entries [3] bad,
+    int metaInts = kMetaInts;     // of each meta block
+    int *meta = nullptr;          // [0] items [1] queue head [2] entries [3] bad,
                                   // [4..5] the entries' cOffset range (see note_c_range),
                                   // [8] tiles with entries [9] phases [10] chunk,
                                   // [16..24] per-XCD item ranges, [32 + kHeadInts q] per-XCD heads
@@ -233,9 +235,12 @@ struct tcv_plan {
 
 // Plan memory as one block: plan_setup fills the shape and returns the bytes
 // needed for geometry g; plan_bind carves the buffers out of such a block.
-// tilesOnly: no narrow-kernel regions (batches and servers run tiles).
+// For servers and the caller-scratch gridder: tiles only, in the bytes that their
+// memory was measured out for; a server's plans run in batches, which bring their
+// own queue heads.
+enum class PlanFor { caller, scratch, server };
 tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tuning, tcv_plan *p,
-                      size_t *bytes, bool tilesOnly = false);
+                      size_t *bytes, PlanFor use = PlanFor::caller);
 void plan_bind(tcv_plan *p, char *block);
 // Whether the plan bins in two levels (by tile in LDS, then by key per tile):
 // the tile histogram must fit the LDS binning kernel and the per-tile key

@@ -849,11 +849,12 @@ __global__ __launch_bounds__(SCAN_BS) void k_plan_items(int pass, PlanDevArgs a,
 }
 
 // Clears a plan's counters and meta blocks (metaG may be null) in one launch.
-__global__ __launch_bounds__(256) void k_plan_clear(int *__restrict__ counts, long long n, int *meta, int *metaG)
+__global__ __launch_bounds__(256) void k_plan_clear(int *__restrict__ counts, long long n, int *meta, int *metaG,
+                                                    int metaInts)
 {
     const long long i0 = blockIdx.x * 256ll + threadIdx.x;
     for (long long i = i0; i < n; i += gridDim.x * 256ll) counts[i] = 0;
-    for (long long i = i0; i < kMetaInts; i += gridDim.x * 256ll) {
+    for (long long i = i0; i < metaInts; i += gridDim.x * 256ll) {
         meta[i] = 0;
         if (metaG) metaG[i] = 0;
     }
@@ -2264,7 +2265,7 @@ static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
     const bool two = p->metaG != p->meta;   // the gridder's own list of work items
     const long long nCounts = p->entriesTmp ? sh.nTiles : sh.nKeys;
     hipLaunchKernelGGL(k_plan_clear, dim3((unsigned)std::min<long long>((nCounts + 1023) / 1024, 2048)), dim3(256), 0,
-                       ctx->stream, p->counts, nCounts, p->meta, two ? p->metaG : nullptr);
+                       ctx->stream, p->counts, nCounts, p->meta, two ? p->metaG : nullptr, p->metaInts);
     TCV_HIP(ctx, hipGetLastError());
     int *touched = sh.adapt ? p->meta + 8 : nullptr;
     const bool lds = sh.nKeys <= kLdsKeys;

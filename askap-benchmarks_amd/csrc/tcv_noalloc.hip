@@ -15,7 +15,10 @@ namespace {
 // Every GPU the library runs on holds one copy of this array until the process
 // ends.  Host code never uses its name as an address: the per-device address
 // comes from hipGetSymbolAddress (noalloc_setup) and is kept in the context.
-static __device__ __align__(256) unsigned char scratch[TCV_NOALLOC_SCRATCH_BYTES];
+// Beside the plan's TCV_NOALLOC_SCRATCH_BYTES it has room for the queue heads of the
+// plan's two lists of work items, so that they don't count against what fits.
+constexpr size_t kHeads = 2 * 8 * kHeadInts * sizeof(int);
+static __device__ __align__(256) unsigned char scratch[TCV_NOALLOC_SCRATCH_BYTES + kHeads];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;
@@ -67,8 +70,9 @@ extern "C" tcv_status tcv_grid_noalloc(tcv_ctx *ctx, const tcv_geometry *g, cons
     for (int keys = 2048;; keys /= 2) {
         p = tcv_plan{};
         const tcv_tuning t{0, 0, 0, keys, 0, -1, 0, 0, 0, 0, 0, 0};
-        tcv_status st = plan_setup(ctx, g, &t, &p, &bytes, true);
+        tcv_status st = plan_setup(ctx, g, &t, &p, &bytes, PlanFor::scratch);
         if (st != TCV_OK) return st;
+        bytes -= p.maxItemsG ? kHeads : kHeads / 2;
         if (bytes <= TCV_NOALLOC_SCRATCH_BYTES || keys == 1) break;
     }
     if (bytes > TCV_NOALLOC_SCRATCH_BYTES)

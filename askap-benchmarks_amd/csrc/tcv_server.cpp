@@ -368,7 +368,7 @@ static tcv_status prepare(tcv_server *s, const tcv_request *req, Req *r)
     if (G.nPlanes < 1 || !G.sSize) return TCV_ERR_INVALID;
     r->sSize.assign(G.sSize, G.sSize + G.nPlanes);
     r->r.geom.sSize = r->sSize.data();
-    tcv_status st = plan_setup(s->ctx, &r->r.geom, &s->tuning, &r->plan, &r->planBytes, true);
+    tcv_status st = plan_setup(s->ctx, &r->r.geom, &s->tuning, &r->plan, &r->planBytes, PlanFor::server);
     if (st != TCV_OK) return st;
     if (r->plan.sh.tw != s->tuning.tile_w || r->plan.sh.th != s->tuning.tile_h ||
         r->plan.sh.kern != s->tuning.kernel || r->plan.sh.dkern != s->tuning.degrid_kernel)

@@ -202,3 +202,21 @@ def test_server_config_rejects_negative_limits(ctx):
         tcv.Server(ctx, GB, max_batch_points=-1)
     with pytest.raises(tcv.TcvError):
         tcv.Server(ctx, GB, max_batch=-2)
+
+
+@pytest.mark.parametrize("config,nVis,gSize,Sz,cSize,grid,degrid", [
+    ({}, 5000, 1024, 129, 129 ** 2 * 64 * 9, 11613440, 3265024),
+    ({}, 100000, 512, 33, 33 ** 2 * 64 * 65, 16481792, 15184640),
+    (dict(tile_w=128), 60000, 2048, 65, 65 ** 2 * 64 * 33, 53872640, 20798208),
+    (dict(item_entries=16), 60000, 2048, 65, 65 ** 2 * 64 * 33, 66801664, 33727232)])
+def test_footprints(ctx, config, nVis, gSize, Sz, cSize, grid, degrid):
+    """Arena bytes of requests, to the byte: what an arena was sized for still fits."""
+    some, vals = ctx.empty(4, np.int32), ctx.empty(4, np.complex64)
+    vis = tcv.Visibilities(ctx, some, some, some, [Sz], gSize, cSize)
+    vis.nVis = nVis
+    srv = tcv.Server(ctx, 1 << 28, **config)
+    try:
+        assert srv.footprint(tcv.Server.GRID, vis, vals, data=vals) == grid
+        assert srv.footprint(tcv.Server.DEGRID, vis, vals, grid=vals) == degrid
+    finally:
+        srv.close()

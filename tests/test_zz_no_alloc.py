@@ -110,3 +110,22 @@ def test_noalloc_refuses_jobs_beyond_the_scratch_array(ctx):
     assert tcv.lib().tcv_grid_noalloc(ctx.h, ct.byref(g), None, None, None) == 0
     g.nVis = 10
     assert tcv.lib().tcv_grid_noalloc(ctx.h, ct.byref(g), None, d.ptr, d.ptr) == 1
+
+
+def test_noalloc_limit(ctx):
+    """The largest plan that fits the 64 MiB (one tile, one key, an entry a
+    visibility), to the byte, and one visibility more."""
+    n = 4185984
+    rng = np.random.default_rng(904)
+    iu, iv = rng.integers(0, 8, (2, n)).astype(np.int32)
+    co = rng.integers(0, 4, n).astype(np.int32)
+    data = (rng.integers(-1, 2, n) + 1j * rng.integers(-1, 2, n)).astype(np.complex64)
+    C = np.array([1, -1, 1j, 0.5], np.complex64)
+    vis = tcv.Visibilities(ctx, iu, iv, co, [1], 8, C.size)
+    d_data, d_C, grid = ctx.to_device(data), ctx.to_device(C), ctx.zeros((8, 8), np.complex64)
+    ctx.check(_noalloc(ctx, vis, d_data, d_C, grid), "grid_noalloc")
+    ref = np.zeros(64, np.complex128)
+    np.add.at(ref, iv * 8 + iu, data.astype(np.complex128) * C[co])
+    assert np.array_equal(grid.download().ravel(), ref.astype(np.complex64))   # every sum exact
+    vis.nVis += 1   # (refused before any of it is read)
+    assert _noalloc(ctx, vis, d_data, d_C, grid) == 6
