@@ -514,6 +514,7 @@ tcv_status launch_narrow_many(tcv_ctx *ctx, const JobDesc *d_jobs, int nJobs, in
     // job's waves end early and leave their place to the next one's
     const int full = std::max(1, ctx->cus) * per;
     const int x = std::min(full, std::max(16, 4 * full / nJobs));
+    ProfScope ps(ctx, degrid ? "degrid_batch" : "grid_batch");
     for (int j0 = 0; j0 < nJobs; j0 += 65535) {
         hipLaunchKernelGGL(k, dim3(x, std::min(nJobs - j0, 65535)), dim3(64), 0, ctx->stream, JobDesc{}, d_jobs + j0);
         TCV_HIP(ctx, hipGetLastError());

@@ -228,6 +228,26 @@ def test_adaptive_work_items(ctx, Sz, gSize, nVis, cluster, os_, planes):
         (info["items"], info["entries"], info["phases"], info["chunk"])
 
 
+def test_regions_in_the_kernel_statistics(ctx):
+    """A batch's launches by regions count in its kernel families: two region sizes
+    and tiles, of one job each."""
+    from tcv.device import Batch
+    jobs = [job(k, w, 300, 150) for k, w in enumerate([[15, 31], [31], [9, 40]])]
+    hold = [(tcv.Plan(ctx, visibilities(ctx, j)), ctx.to_device(j["data"]), ctx.to_device(j["C"]),
+             ctx.zeros((150, 150), np.complex64), ctx.empty(300, np.complex64)) for j in jobs]
+    b = Batch(ctx, hold)
+    ctx.set_profiling(True)
+    try:
+        ctx.reset_stats()
+        b.grid()
+        b.degrid()
+        for family in ("grid_batch", "degrid_batch"):
+            n, ms = ctx.kernel_stats(family)
+            assert n == 3 and ms > 0, family
+    finally:
+        ctx.set_profiling(False)
+
+
 @pytest.mark.parametrize("Sz,gSize,nVis,tile_w", [
     (49, 2048, 200000, 128), (71, 2048, 100000, 128), (71, 2816, 200000, 128), (71, 2944, 200000, 64), (49, 4096, 400000, 64),
     (72, 4096, 200000, 128), (72, 4096, 50000, 64), (65, 900, 200000, 64)])
