@@ -114,8 +114,8 @@ __host__ __device__ constexpr int padded(int i) { return i + (i >> 4); }
 // column pass 76 us: its four columns a workgroup (what 4096 rows leave room
 // for at 16 values a thread) are 32-byte segments.  Holding it to 64 registers,
 // for two workgroups a CU, left it at 75-84 us.
-// OUT 0: as is; 1: times (-1)^(x+y) on input (row pass); 2: on output;
-// 3: on output with fftFix (real part * scale, imaginary part 0).
+// OUT 1: times (-1)^(x+y) on input (row pass); 2: on output; 3: on output with
+// fftFix (real part * scale, imaginary part 0).
 template <int N, int COLS, int DIR, int OUT>
 __global__ __launch_bounds__(COLS ? N / 16 * COLS : 256) void k_fft_pass(float2 *__restrict__ g,
                                                                            const float2 *__restrict__ tw,

@@ -513,7 +513,10 @@ constexpr double kDegridPhaseBytes = 5.5e6;
 // Entries per work item that the phase count keeps at least.  Batches re-bin + grid
 // + degrid in ms with 64 and 32: 16 jobs of 10 000-500 000 visibilities 42.98 and
 // 40.40 (24: 40.46), 10 of 5000-150 000 16.15 and 15.34, 19 of up to 61 000 11.02
-// and 11.04.  Servers and the caller-scratch gridder keep 64: their plans' size is
+// and 11.04.  Single jobs of a given tile shape in us: width 63, 100 003, 2047^2 1035
+// and 797; 129, 160 000, 4096^2 6703 and 5424; 129, 20 000, 1024^2 523 and 473; 129,
+// 500, 512^2 331 and 190; 65, 5000, 1024^2 152 and 120; 33, 3000, 512^2 101 and 78; the
+// one that lost, 129, 6000, 2048^2, 372 and 377.  Servers and the caller-scratch gridder keep 64: their plans' size is
 // what their memory was measured out for.
 constexpr int kItemEntries = 32, kItemEntriesFixed = 64;
 constexpr double kGridPhaseBytes = 5.5e6;   // the gridder may use its own count (grid_phases)
@@ -584,7 +587,7 @@ static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 // 1885 against 1900 + 2648 + 1658), and a class of widths up to 9 by regions of
 // 24 cells costs more binning (350) than it saves.
 struct WidthClass { int width, region, chunk; };
-constexpr WidthClass kClasses[] = {{19, 32, 128}, {31, 48, 64}};
+constexpr WidthClass kClasses[] = {{kRegionWidths[0], kRegions[0], 128}, {kRegionWidths[1], kRegions[1], 64}};
 // Kernels of 20 to 31 only: a region's flush costs as much as two or three of
 // their footprints, so a job that is neither small nor dense keeps its tiles.
 // Width 31, 4096^2 (51 984 regions), re-bin + grid + degrid: 8000 visibilities

@@ -121,7 +121,7 @@ tcv_status launch_degrid_plain_f64(tcv_ctx *ctx, const GeomDev &g, const float2 
 struct JobDesc {
     const int4 *items;
     const int4 *entries;
-    int *meta;                  // meta[0] = number of work items, per-XCD queues at [8..24]
+    int *meta;                  // meta[0] = number of work items (see tcv_plan::meta)
     const void *data;           // visibilities to grid (float2, or half2 in FP16 storage)
     const void *C;              // taps (float2, or half2)
     float2 *grid;
@@ -247,7 +247,8 @@ void plan_bind(tcv_plan *p, char *block);
 // histogram one workgroup's LDS.
 bool plan_two_level(const PlanShape &sh);
 
-constexpr int kRegions[] = {32, 48};   // region sizes built (cells a side)
+constexpr int kRegions[] = {32, 48};        // region sizes built (cells a side)
+constexpr int kRegionWidths[] = {19, 31};   // the widest kernel of each
 
 struct tcv_batch {
     int nJobs = 0;      // jobs that have tiles of tw x th: d_jobs, d_jobsD

@@ -457,7 +457,7 @@ __global__ __launch_bounds__(SCAN_BS) void k_scan_apply(const int *__restrict__ 
 // ---- tiled path: plan kernels -------------------------------------------------
 
 struct PlanDevArgs {
-    int tw, th, nTX, k2, phases, chunk, nTiles, xcd;   // tw, th: the stride of the tiles or regions
+    int tw, th, nTX, k2, phases, chunk, nTiles;   // tw, th: the stride of the tiles or regions
     int single;   // regions: a footprint belongs to the one its first cell falls on
     long long cSize;
     int adapt;          // phases and chunk chosen by cut_of, up to those above
@@ -2259,7 +2259,7 @@ static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
     const PlanShape &sh = p->sh;
     g.sLo = sh.sLo;
     g.sHi = sh.sHi;
-    PlanDevArgs a{sh.bw, sh.bh, sh.nTX, sh.k2, sh.phases, sh.chunk, sh.nTiles, sh.xcd, sh.region > 0,
+    PlanDevArgs a{sh.bw, sh.bh, sh.nTX, sh.k2, sh.phases, sh.chunk, sh.nTiles, sh.region > 0,
                   g.cSize, sh.adapt, kAdaptDegrid, sh.phaseBytes / sh.tapBytes};
     tcv_status st;
     const bool two = p->metaG != p->meta;   // the gridder's own list of work items
@@ -2464,8 +2464,10 @@ tcv_status grid_tiled_t(tcv_ctx *ctx, const ItemSource<BATCH> &src, int kern_kin
 
 // manyWaves: the pair degridder on 8192-cell tiles runs eight-wave workgroups.
 // Measured on 128 x 64 tiles: 16 % faster with 3.8 MB phases (spectral
-// workload) and on the uneven batch, 22 % slower with 70 MB phases (a 160 000
-// visibility job cut into 4 phases), where more waves only add misses.
+// workload) and on the uneven batch, slower with phases of 70 MB and more, where
+// more waves only add misses: width 129, 160 000 visibilities, 4096^2, 4 phases of 70
+// MB 3258 us with four waves and 3300 with eight, on a quarter of the grid 3179 and
+// 3387; 65, 300 000, 2048^2, one of 71 MB 990 and 1188.
 template <int TW, int TH, bool HALF, bool BATCH>
 tcv_status degrid_tiled_t(tcv_ctx *ctx, const ItemSource<BATCH> &src, int kern_kind, bool manyWaves)
 {
@@ -2602,6 +2604,12 @@ tcv_status launch_degrid_tiled(tcv_ctx *ctx, tcv_plan *p, const float2 *grid, co
     if (p->sh.region > 0) return launch_narrow(ctx, src.one, p->sh.region, half != nullptr, true);
     // the FP16 four-tap degridder needs kernel widths of at least 4
     const int kern = (half && p->sh.dkern == 4 && p->sh.minS < 4) ? 3 : p->sh.dkern;
+    // An open plan's phases are chosen on the device, so the most it can have counts
+    // here.  Where it takes far fewer, four waves would be up to 3 % faster (width
+    // 129, 33 000 visibilities on a quarter of 4096^2, 4 phases of up to 16: 700 us
+    // and 721) or as fast (on all of it, one phase: 747 and 747); where it takes that
+    // many, eight are by 3 to 30 % (129, 160 000, 4096^2 2424 and 2356; 65, 200 000,
+    // 1024^2 609 and 432; 81, 200 000, 4096^2 1328 and 1124).
     const double phaseBytes = (double)p->cSize * (half ? 4 : 8) / std::max(1, p->sh.phases);
     const bool many = phaseBytes <= kManyWavesPhaseBytes;
 #define X(a, b)                                                                        \

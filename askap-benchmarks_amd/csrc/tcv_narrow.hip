@@ -15,10 +15,12 @@
 //    for a run of entries of one width, so an entry costs a handful of adds
 //    beside its multiply-adds; the taps of the next entries are loaded while
 //    the present ones are worked on.
-// Regions of 32 cells (widths up to 19: 14 cells apart at the widest) keep 20
-// gridding waves a CU in flight, of 48 cells (widths up to 31) 8.
+// Regions of 32 cells (widths up to 19: 14 cells apart at the widest) keep 18
+// gridding waves a CU in flight (8704 bytes of LDS each) and 16 degridding ones, of
+// 48 cells (widths up to 31) 8.
 //
-// Bound: LDS and vector instruction issue (an entry's taps come from the L2s).
+// Bound: LDS and vector instruction issue (an entry's taps come from the L2s); of
+// the gridder's LDS cycles on widths 7-19 60 % are bank conflicts.
 // 3.8 M visibilities of widths 7-19 on 4096^2 (509 M grid points): gridder 1860 us
 // by tiles, 360 by regions (11 TFLOP/s); degridder 1685 and 264 (15 TFLOP/s).
 #include <hip/hip_runtime.h>
@@ -36,15 +38,20 @@ namespace {
 // in each plane whatever the column's parity, and the lanes of a wave read and
 // write each plane contiguously along a row.  The last column of a plane and
 // the cells beyond it are never part of the grid: the cell after a
-// footprint of odd width may fall there, and the stride spreads a narrow
-// footprint's rows over the banks.
+// footprint of odd width may fall there.  (Rows are 34 dwords apart, 50 in a region of
+// 48: a step's rows of a narrow footprint share banks.)
 template <int R>
 struct Region {
     static constexpr int RS = R / 2 + 1, PC = R * RS;
     static constexpr unsigned PB = PC * 8u;   // bytes a plane
-    // steps of 64 pairs that its widest footprint takes
-    static constexpr int kSteps = R == 32 ? 4 : 8;
 };
+
+// Steps of 64 pairs that footprints take: up to 3 in a region of 32, 4 to 8 in one
+// of 48.
+constexpr int pairs_of(int s) { return ((s + 1) >> 1) * s; }
+static_assert(kRegions[0] == 32 && pairs_of(kRegionWidths[0]) <= 3 * 64, "steps of the smaller regions");
+static_assert(kRegions[1] == 48 && pairs_of(kRegionWidths[0] + 1) > 3 * 64 && pairs_of(kRegionWidths[1]) <= 8 * 64,
+              "steps of the larger regions");
 
 // Orders this wave's LDS accesses for the compiler (the hardware runs a wave's
 // LDS instructions in order): lanes read cells that other lanes wrote.
@@ -259,17 +266,14 @@ void k_grid_narrow(JobDesc one, const JobDesc *__restrict__ jobs)
                     if (__any(lane >= i && lane < i1 && tap0 + s * s >= nTaps)) run(jTag, std::true_type{}, s, i, i1);
                     else run(jTag, std::false_type{}, s, i, i1);
                 };
-                if constexpr (R <= 32) {
+                if constexpr (R == 32) {
                     if (n <= 64) by_edge(std::integral_constant<int, 1>{});
                     else if (n <= 128) by_edge(std::integral_constant<int, 2>{});
-                    else if constexpr (R == 32) {
-                        if (n <= 192) by_edge(std::integral_constant<int, 3>{});
-                        else by_edge(std::integral_constant<int, 4>{});
-                    }
+                    else by_edge(std::integral_constant<int, 3>{});
                 } else {
-                    if (n <= 64 * T::kSteps / 2) by_edge(std::integral_constant<int, T::kSteps / 2>{});
-                    else if (n <= 64 * T::kSteps * 3 / 4) by_edge(std::integral_constant<int, T::kSteps * 3 / 4>{});
-                    else by_edge(std::integral_constant<int, T::kSteps>{});
+                    if (n <= 64 * 4) by_edge(std::integral_constant<int, 4>{});
+                    else if (n <= 64 * 6) by_edge(std::integral_constant<int, 6>{});
+                    else by_edge(std::integral_constant<int, 8>{});
                 }
                 i = i1;
             }
@@ -459,15 +463,14 @@ void k_degrid_narrow(JobDesc one, const JobDesc *__restrict__ jobs)
                 const int i1 = min(m, i + run_length(width, i, m, lane));
                 const int n = ((s + 1) >> 1) * s;
                 using W = std::integral_constant<int, 64>;
-                if constexpr (R <= 32) {
+                if constexpr (R == 32) {
                     if (n <= 64) by_steps(std::integral_constant<int, 16>{}, s, i, i1, (n + 15) / 16);
                     else if (n <= 128) by_steps(std::integral_constant<int, 32>{}, s, i, i1, (n + 31) / 32);
-                    else if constexpr (R == 32) by_steps(W{}, s, i, i1, (n + 63) / 64);
+                    else by_edge(W{}, std::integral_constant<int, 3>{}, s, i, i1);
                 } else {
-                    if (n <= 64 * T::kSteps / 2) by_edge(W{}, std::integral_constant<int, T::kSteps / 2>{}, s, i, i1);
-                    else if (n <= 64 * T::kSteps * 3 / 4)
-                        by_edge(W{}, std::integral_constant<int, T::kSteps * 3 / 4>{}, s, i, i1);
-                    else by_edge(W{}, std::integral_constant<int, T::kSteps>{}, s, i, i1);
+                    if (n <= 64 * 4) by_edge(W{}, std::integral_constant<int, 4>{}, s, i, i1);
+                    else if (n <= 64 * 6) by_edge(W{}, std::integral_constant<int, 6>{}, s, i, i1);
+                    else by_edge(W{}, std::integral_constant<int, 8>{}, s, i, i1);
                 }
                 i = i1;
             }
