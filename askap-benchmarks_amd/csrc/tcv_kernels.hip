@@ -728,7 +728,10 @@ __global__ __launch_bounds__(BS) void k_plan_tile_keys(PlanDevArgs a, const int 
 // that a tile with many entries is shared out: 2000 visibilities of width 129 on
 // 32 tiles, 96 items 304 + 118 us, 464 items 71 + 41; 30 000 of one plane on 694
 // tiles 1394 + 776 with 2048, 235 + 138 with 32.  Where the slots alone are
-// enough, an ordinary slot isn't cut (100 003 of width 63: 523 against 477).
+// enough, an ordinary slot isn't cut (100 003 of width 63: 523 against 477).  Where
+// they aren't, items hold twice kAdaptItems' share, up to 128 entries: the flushes
+// bound finer ones (100 000 of widths 33 and 63 on 2048^2, 32 entries 462 + 200, 54
+// 333 + 188; of width 65 602 + 264 and 401 + 238).
 struct Cut {
     int phases, chunk;
 };
@@ -747,10 +750,14 @@ __device__ __forceinline__ Cut cut_of(const PlanDevArgs &a, const int *starts, c
         while (ph * 2 <= target) ph *= 2;
     }
     ph = min(ph, a.phases);
-    int chunk = n / kAdaptItems;
     const double slots = tiles * ph, each = n / slots;
-    if (slots >= kAdaptItems / 4) chunk = max(chunk, (int)fmin(4 * each, 512.0));
-    else if (slots >= kAdaptItems / 32 && each < 1.5 * kAdaptChunk) chunk = max(chunk, (int)(2 * each));
+    int chunk = n / kAdaptItems;
+    if (slots >= kAdaptItems / 4) {
+        chunk = max(chunk, (int)fmin(4 * each, 512.0));
+    } else {
+        chunk = max(chunk, min(2 * chunk, 4 * kAdaptChunk));
+        if (slots >= kAdaptItems / 32 && each < 1.5 * kAdaptChunk) chunk = max(chunk, (int)(2 * each));
+    }
     return Cut{ph, max(kAdaptChunk, min(a.chunk, chunk))};
 }
 

@@ -305,6 +305,25 @@ def test_widened_plans_in_a_batch(ctx):
         b.close()
 
 
+@pytest.mark.parametrize("nVis,chunk", [(5000, 32), (100000, 72), (300000, 128)])
+def test_adaptive_chunk_of_few_slots(ctx, nVis, chunk):
+    """Work items of few tiles in one phase: 1 / 4096 of the entries, from 32 up to
+    128 (2.97 entries a visibility here)."""
+    from helpers import exact_problem
+    Sz, gSize = 33, 300
+    iu, iv, co, data, C, grid = exact_problem(nVis, nVis, gSize, Sz, cluster=None)
+    vis = tcv.Visibilities(ctx, iu, iv, co, [Sz], gSize, C.size)
+    plan = tcv.Plan(ctx, vis)
+    info = plan.info()
+    assert info["phases"] == info["grid_phases"] == 1
+    assert info["chunk"] == chunk == max(32, min(2 * (info["entries"] // 8192), 128))
+    g, out = ctx.zeros((gSize, gSize), np.complex64), ctx.empty(nVis, np.complex64)
+    plan.grid(ctx.to_device(data), ctx.to_device(C), g)
+    plan.degrid(ctx.to_device(grid), ctx.to_device(C), out)
+    assert np.array_equal(g.download(), O.grid(data, iu, iv, co, C, gSize, Sz))
+    assert np.array_equal(out.download(), O.degrid(grid, iu, iv, co, C, Sz))
+
+
 def test_adaptive_plan_of_nothing(ctx):
     """Every visibility out of range: no items, cleared results."""
     vis = tcv.Visibilities(ctx, [1, 2], [0, 0], [0, 0], [65], 100, 65 * 65)
