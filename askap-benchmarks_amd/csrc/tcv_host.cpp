@@ -588,12 +588,24 @@ static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 // 24 cells costs more binning (350) than it saves.
 struct WidthClass { int width, region, chunk; };
 constexpr WidthClass kClasses[] = {{kRegionWidths[0], kRegions[0], 128}, {kRegionWidths[1], kRegions[1], 64}};
-// Kernels of 20 to 31 only: a region's flush costs as much as two or three of
-// their footprints, so a job that is neither small nor dense keeps its tiles.
-// Width 31, 4096^2 (51 984 regions), re-bin + grid + degrid: 8000 visibilities
-// 102 + 92 + 89 -> 48 + 86 + 38; 64 000 132 + 127 + 115 -> 74 + 387 + 142;
-// 500 000 401 + 670 + 488 -> 189 + 733 + 338.
-constexpr int kSmallJob = 8192, kDenseRegion = 8;
+// A region's flush costs as much as several of its widest footprints, so a class
+// whose visibilities lie thinly goes to the tiles instead: a plan counts the
+// visibilities and the regions they touch when it is made (thin_classes).  Grid +
+// degrid in us, tiles and regions, on a 4096^2 grid covered evenly, at visibilities a
+// region: width 20, 6: 282 and 386, 12: 460 and 485, 16: 581 and 524; 27, 8: 621 and
+// 853, 16: 1104 and 1094, 32: 2055 and 1529; 31, 3: 460 and 962, 16: 1817 and 1858;
+// with few regions 31, 1024^2, 4: 77 and 88, 12: 160 and 135.  Widths up to 19 alone
+// are level with tiles that take 200 us more to bin (19, 4: 587 and 668; 17, 2: 271
+// and 310; 15, 4: 336 and 339), but for many regions (19, 8192^2, 3: 1811 and 2335);
+// beside tiles that run anyway they save less (9, 15, 27 and 63, 1.9 to a region
+// of the narrower two: 359 and 448).
+constexpr int kSmallJob = 8192;   // no class of a smaller job is thin
+static double dense_region(const PlanShape &sh, bool tiles, int touched)
+{
+    if (sh.region == kRegions[1]) return touched <= 8192 ? 8 : sh.sHi < 24 ? 12 : 16;
+    return tiles ? 4 : sh.sHi >= 18 && touched > 131072 ? 5 : 0;
+}
+
 // Entries that a job of footprints of the widest kernel makes on average.
 static double entries_expected(const tcv_geometry *g, const PlanShape &sh)
 {
@@ -636,7 +648,7 @@ static bool open_shape(const tcv_tuning &t)
 }
 
 tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tuning, tcv_plan *p,
-                      size_t *bytes, PlanFor use)
+                      size_t *bytes, PlanFor use, int classes)
 {
     const bool tilesOnly = use != PlanFor::caller;
     if (use == PlanFor::server) p->metaInts = kMetaIntsBatch;
@@ -663,14 +675,12 @@ tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tun
     if (!tilesOnly && open_shape(t)) {
         int least = maxS;
         for (int k = 0; k < g->nPlanes; k++) least = std::min(least, g->sSize[k]);
-        const long long across = (g->gSize + kClasses[1].region - maxS) / std::max(1, kClasses[1].region - maxS + 1);
-        const bool sparse = least > kClasses[0].width && maxS <= kClasses[1].width && g->nVis > kSmallJob &&
-                            g->nVis < kDenseRegion * across * across;
-        if (least >= 2 && !sparse)   // pairs of taps need widths of two
-            for (const WidthClass &c : kClasses) {
+        if (least >= 2)   // pairs of taps need widths of two
+            for (int k = 0; k < classes; ++k) {
+                const WidthClass &c = kClasses[k];
                 int hi = 0;
-                for (int k = 0; k < g->nPlanes; k++)
-                    if (g->sSize[k] >= tilesLo && g->sSize[k] <= c.width) hi = std::max(hi, g->sSize[k]);
+                for (int j = 0; j < g->nPlanes; j++)
+                    if (g->sSize[j] >= tilesLo && g->sSize[j] <= c.width) hi = std::max(hi, g->sSize[j]);
                 if (hi) parts.push_back({tilesLo, hi, c.region, c.chunk});
                 tilesLo = c.width + 1;
             }
@@ -893,6 +903,32 @@ void mark_shared_grids(std::vector<JobDesc> &jobs)
 
 extern "C" {
 
+// How many classes of widths a plan just built had better keep by regions.
+static tcv_status thin_classes(tcv_ctx *ctx, const tcv_geometry *g, tcv_plan *p, int *keep)
+{
+    *keep = kAllClasses;
+    tcv_plan *by[kAllClasses] = {nullptr, nullptr};
+    for (auto &q : p->parts) by[q->sh.region == kRegions[0] ? 0 : 1] = q.get();
+    if (p->sh.region > 0) by[p->sh.region == kRegions[0] ? 0 : 1] = p;
+    if ((!by[0] && !by[1]) || g->nVis <= kSmallJob) return TCV_OK;
+    int meta[kAllClasses][9] = {};   // [2] visibilities [8] regions touched
+    for (int k = 0; k < kAllClasses; ++k) {
+        if (!by[k]) continue;
+        tcv_status st = launch_plan_touched(ctx, by[k]);
+        if (st != TCV_OK) return st;
+        TCV_HIP(ctx, hipMemcpyAsync(meta[k], by[k]->meta, sizeof(meta[k]), hipMemcpyDeviceToHost, ctx->stream));
+    }
+    TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    bool tiles = p->sh.region == 0;
+    for (int k = kAllClasses - 1; k >= 0; --k) {   // (a class goes only after the wider one)
+        if (!by[k]) continue;
+        if (meta[k][2] >= dense_region(by[k]->sh, tiles, meta[k][8]) * meta[k][8]) break;
+        *keep = k;
+        tiles = true;
+    }
+    return TCV_OK;
+}
+
 tcv_status tcv_plan_create(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tuning,
                            tcv_plan **out)
 {
@@ -900,38 +936,33 @@ tcv_status tcv_plan_create(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning
     *out = nullptr;
     if (!ctx) return TCV_ERR_INVALID;
     TCV_HIP(ctx, hipSetDevice(ctx->device));
-    tcv_plan *p = new tcv_plan();
-    size_t bytes = 0;
-    tcv_status st = plan_setup(ctx, g, tuning, p, &bytes);
-    if (st != TCV_OK) {
-        delete p;
-        return st;
+    auto release = [](tcv_plan *q) {
+        free_plan(q);
+        delete q;
+    };
+    for (int classes = kAllClasses;;) {   // twice at most
+        const int built = classes;
+        std::unique_ptr<tcv_plan, decltype(release)> p(new tcv_plan(), release);
+        size_t bytes = 0;
+        tcv_status st = plan_setup(ctx, g, tuning, p.get(), &bytes, PlanFor::caller, classes);
+        if (st != TCV_OK) return st;
+        void *block = nullptr;
+        if (hipMalloc(&block, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            return tcv_fail(ctx, TCV_ERR_NOMEM, "plan allocation of " + std::to_string(bytes) + " bytes failed");
+        }
+        plan_bind(p.get(), (char *)block);
+        p->ownsBlock = true;
+        if (hipMemcpy(p->d_sSize, g->sSize, sizeof(int) * g->nPlanes, hipMemcpyHostToDevice) != hipSuccess)
+            return tcv_fail(ctx, TCV_ERR_DEVICE, "plan upload failed");
+        if ((st = tcv_plan_build(ctx, p.get(), g)) != TCV_OK) return st;
+        if (classes == kAllClasses && (st = thin_classes(ctx, g, p.get(), &classes)) != TCV_OK) return st;
+        if (classes == built) {
+            TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            *out = p.release();
+            return TCV_OK;
+        }
     }
-    void *block = nullptr;
-    if (hipMalloc(&block, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        delete p;
-        return tcv_fail(ctx, TCV_ERR_NOMEM, "plan allocation of " + std::to_string(bytes) + " bytes failed");
-    }
-    plan_bind(p, (char *)block);
-    p->ownsBlock = true;
-    if (hipMemcpy(p->d_sSize, g->sSize, sizeof(int) * g->nPlanes, hipMemcpyHostToDevice) != hipSuccess) {
-        free_plan(p);
-        delete p;
-        return tcv_fail(ctx, TCV_ERR_DEVICE, "plan upload failed");
-    }
-    st = tcv_plan_build(ctx, p, g);
-    if (st == TCV_OK) {
-        hipError_t e = hipStreamSynchronize(ctx->stream);
-        if (e != hipSuccess) st = tcv_fail(ctx, TCV_ERR_DEVICE, hipGetErrorString(e));
-    }
-    if (st != TCV_OK) {
-        free_plan(p);
-        delete p;
-        return st;
-    }
-    *out = p;
-    return TCV_OK;
 }
 
 tcv_status tcv_plan_build(tcv_ctx *ctx, tcv_plan *p, const tcv_geometry *g)

@@ -238,9 +238,11 @@ struct tcv_plan {
 // For servers and the caller-scratch gridder: tiles only, in the bytes that their
 // memory was measured out for; a server's plans run in batches, which bring their
 // own queue heads.
+// classes: how many of the classes of narrower widths may take regions.
 enum class PlanFor { caller, scratch, server };
+constexpr int kAllClasses = 2;
 tcv_status plan_setup(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning *tuning, tcv_plan *p,
-                      size_t *bytes, PlanFor use = PlanFor::caller);
+                      size_t *bytes, PlanFor use = PlanFor::caller, int classes = kAllClasses);
 void plan_bind(tcv_plan *p, char *block);
 // Whether the plan bins in two levels (by tile in LDS, then by key per tile):
 // the tile histogram must fit the LDS binning kernel and the per-tile key
@@ -277,6 +279,8 @@ struct HalfStorage {
 };
 
 tcv_status plan_build_kernels(tcv_ctx *ctx, tcv_plan *p, const GeomDev &g);
+// Counts the tiles or regions that have entries into meta[8] of a plan by regions.
+tcv_status launch_plan_touched(tcv_ctx *ctx, tcv_plan *p);
 // Sets JobDesc::sharedGrid on every job whose grid overlaps another job's.
 void mark_shared_grids(std::vector<JobDesc> &jobs);
 // half == nullptr: FP32 taps and data

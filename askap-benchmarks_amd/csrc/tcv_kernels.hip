@@ -762,12 +762,12 @@ __device__ __forceinline__ Cut cut_of(const PlanDevArgs &a, const int *starts, c
 }
 
 // Counts the tiles that have entries.
-__global__ __launch_bounds__(256) void k_plan_touched(PlanDevArgs a, const int *__restrict__ starts,
+__global__ __launch_bounds__(256) void k_plan_touched(int nTiles, int k2, const int *__restrict__ starts,
                                                       int *__restrict__ meta)
 {
     int n = 0;
-    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < a.nTiles; t += gridDim.x * blockDim.x)
-        n += starts[(long long)(t + 1) * a.k2] > starts[(long long)t * a.k2];
+    for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nTiles; t += gridDim.x * blockDim.x)
+        n += starts[(long long)(t + 1) * k2] > starts[(long long)t * k2];
     int total;
     (void)block_exclusive_scan(n, &total);
     if (threadIdx.x == 0 && total) atomicAdd(&meta[8], total);
@@ -2261,6 +2261,15 @@ static tcv_status scan_exclusive(tcv_ctx *ctx, const int *in, int *out, long lon
 // Visibilities from which k_plan_tile_keys runs 1024 threads a tile.
 constexpr int kBigTiles = 1 << 20;
 
+tcv_status launch_plan_touched(tcv_ctx *ctx, tcv_plan *p)
+{
+    const PlanShape &sh = p->sh;
+    hipLaunchKernelGGL(k_plan_touched, dim3(std::min((sh.nTiles + 255) / 256, 64)), dim3(256), 0, ctx->stream,
+                       sh.nTiles, sh.k2, (const int *)p->starts, p->meta);
+    TCV_HIP(ctx, hipGetLastError());
+    return TCV_OK;
+}
+
 static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
 {
     const PlanShape &sh = p->sh;
@@ -2328,11 +2337,7 @@ static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
         if ((st = scan_exclusive(ctx, p->counts, p->starts, sh.nKeys, p->scanTmp, p->cursor)) != TCV_OK)
             return st;
         if ((st = bin(1)) != TCV_OK) return st;
-        if (touched) {
-            hipLaunchKernelGGL(k_plan_touched, dim3(std::min((sh.nTiles + 255) / 256, 64)), dim3(256), 0, ctx->stream,
-                               a, (const int *)p->starts, p->meta);
-            TCV_HIP(ctx, hipGetLastError());
-        }
+        if (touched && (st = launch_plan_touched(ctx, p)) != TCV_OK) return st;
     }
     // work items: cuts of the sorted entries into (phase, tile) ranges
     ItemLists lists{};

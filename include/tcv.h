@@ -275,8 +275,12 @@ typedef struct {
 
 /* A tuning with every field open but tap_bytes and item_entries takes kernels up
  * to 31 wide by overlapping regions of 32 or 48 cells a side that one wave
- * grids or degrids (a job of widths 20 to 31 only, when it has at most 8192
- * visibilities or at least 8 to a region), wider ones by tiles. */
+ * grids or degrids, wider ones by tiles.  Of a job of more than 8192
+ * visibilities, tcv_plan_create counts the visibilities of widths up to 19 and
+ * of 20 to 31 and the regions they touch, and leaves the class to the tiles
+ * where they lie thinly (widths 20 to 31: fewer than 8 to 16 to a region; up to
+ * 19: fewer than 4 beside other tiles, or 5 of widths 18 and 19 on more than
+ * 131 072 regions).  tcv_plan_build keeps that choice. */
 typedef struct tcv_plan tcv_plan;
 
 /* Allocates a plan for jobs of this geometry class (device buffers sized from

@@ -84,6 +84,43 @@ def test_regions_equal_oracle(ctx, widths, nVis, gSize):
     assert np.array_equal(g, gref) and np.array_equal(o, oref)
 
 
+@pytest.mark.parametrize("widths,nVis,near,regions", [
+    ([27], 8192, (), 1), ([27], 8193, (), 0), ([27], 9000, (0,), 1), ([21], 30000, (), 0),
+    ([9], 9000, (), 1), ([19, 18], 9000, (), 1),          # alone: never thin on so few regions
+    ([9, 27], 20000, (), 0), ([9, 27], 20000, (0,), .5), ([9, 27], 20000, (0, 1), 1), ([9, 27], 20000, (1,), 1),
+    ([17, 40], 20000, (), 0), ([17, 40], 20000, (0,), .5), ([5, 25, 63], 30000, (0, 2), 1 / 3)])
+def test_thin_classes(ctx, widths, nVis, near, regions):
+    """Classes whose visibilities lie thinly go to the tiles (`near`: widths whose
+    visibilities lie close together); results are exact either way, and after other
+    visibilities come into the plan."""
+    gSize = 2048
+    j = job(nVis + len(near), widths, nVis, gSize)
+    rng = np.random.default_rng(nVis)
+    for k in near:
+        at = np.flatnonzero(j["plane"] == k)
+        j["iu"][at], j["iv"][at] = rng.integers(200, 300, (2, at.size))
+    gref, oref = reference(j)
+    plan = tcv.Plan(ctx, visibilities(ctx, j))
+    info = plan.info()
+    g, o = run(ctx, plan, j)
+    assert np.array_equal(g, gref) and np.array_equal(o, oref)
+    # a visibility makes one entry by regions, and four or more of the widest by tiles
+    w = j["w"][j["plane"]]
+    order = sorted(set(widths))
+    by = [w == x for x in order]
+    share = {0: [], 1: order, .5: order[:1], 1 / 3: order[:1]}[regions]
+    tile_w, tile_h = info["tile_w"], info["tile_h"]
+    u0, v0 = j["iu"] - w // 2, j["iv"]
+    tiles = ((u0 + w - 1) // tile_w - u0 // tile_w + 1) * ((v0 + w - 1) // tile_h - v0 // tile_h + 1)
+    assert info["entries"] == sum(int(m.sum()) if x in share else int(tiles[m].sum()) for x, m in zip(order, by))
+    j2 = dict(j, iu=np.ascontiguousarray(j["iu"][::-1]), iv=np.ascontiguousarray(j["iv"][::-1]),
+              plane=np.ascontiguousarray(j["plane"][::-1]), co=np.ascontiguousarray(j["co"][::-1]))
+    plan.build(visibilities(ctx, j2))
+    gref, oref = reference(j2)
+    g, o = run(ctx, plan, j2)
+    assert np.array_equal(g, gref) and np.array_equal(o, oref)
+
+
 @pytest.mark.parametrize("widths,nVis,gSize,want", [
     # tile_w, chunk, slice_keys, phases, grid_phases by the rules for tiles
     ([15], 30000, 300, (16, 512, 256, 1, 1)), ([27], 20000, 256, (32, 2048, 256, 1, 1)),
