@@ -730,7 +730,9 @@ tcv_status tcv_hogbom(tcv_ctx *ctx, float *d_residual, long long width, const fl
         return tcv_fail(ctx, TCV_ERR_INVALID, "tcv_hogbom: bad argument (widths below 65536)");
     const long long n = width * width, pn = psfWidth * psfWidth;
     const bool wait = psfPeakVal || psfPeakPos || dirtyPeakVal || dirtyPeakPos;
-    bool loop = hogbom_loop_fits(ctx, width, psfWidth);
+    // (a few iterations on a small image take less than the cooperative launch: one on
+    // 250^2 27 us, 37 by the loop; five on 64^2 43 and 45)
+    bool loop = hogbom_loop_fits(ctx, width, psfWidth) && (niters >= 8 || width > 512);
     int launched = 0, done = 0;   // launches of the loop made, and done
     unsigned long long pk = 0, first = 0;
     ProfScope ps(ctx, "hogbom");
