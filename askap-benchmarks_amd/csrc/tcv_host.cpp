@@ -911,18 +911,18 @@ static tcv_status thin_classes(tcv_ctx *ctx, const tcv_geometry *g, tcv_plan *p,
     for (auto &q : p->parts) by[q->sh.region == kRegions[0] ? 0 : 1] = q.get();
     if (p->sh.region > 0) by[p->sh.region == kRegions[0] ? 0 : 1] = p;
     if ((!by[0] && !by[1]) || g->nVis <= kSmallJob) return TCV_OK;
-    int meta[kAllClasses][9] = {};   // [2] visibilities [8] regions touched
-    for (int k = 0; k < kAllClasses; ++k) {
-        if (!by[k]) continue;
-        tcv_status st = launch_plan_touched(ctx, by[k]);
-        if (st != TCV_OK) return st;
-        TCV_HIP(ctx, hipMemcpyAsync(meta[k], by[k]->meta, sizeof(meta[k]), hipMemcpyDeviceToHost, ctx->stream));
-    }
+    int count[kAllClasses][2] = {};   // regions touched, visibilities
+    int *d_count = reinterpret_cast<int *>(ctx->d_counters + 6);
+    tcv_status st = launch_fill_u32(ctx, d_count, 0, 2 * kAllClasses);
+    for (int k = 0; k < kAllClasses && st == TCV_OK; ++k)
+        if (by[k]) st = launch_plan_touched(ctx, by[k], d_count + 2 * k, d_count + 2 * k + 1);
+    if (st != TCV_OK) return st;
+    TCV_HIP(ctx, hipMemcpyAsync(count, d_count, sizeof(count), hipMemcpyDeviceToHost, ctx->stream));
     TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
     bool tiles = p->sh.region == 0;
     for (int k = kAllClasses - 1; k >= 0; --k) {   // (a class goes only after the wider one)
         if (!by[k]) continue;
-        if (meta[k][2] >= dense_region(by[k]->sh, tiles, meta[k][8]) * meta[k][8]) break;
+        if (count[k][1] >= dense_region(by[k]->sh, tiles, count[k][0]) * count[k][0]) break;
         *keep = k;
         tiles = true;
     }
@@ -936,29 +936,39 @@ tcv_status tcv_plan_create(tcv_ctx *ctx, const tcv_geometry *g, const tcv_tuning
     *out = nullptr;
     if (!ctx) return TCV_ERR_INVALID;
     TCV_HIP(ctx, hipSetDevice(ctx->device));
-    auto release = [](tcv_plan *q) {
-        free_plan(q);
-        delete q;
-    };
-    for (int classes = kAllClasses;;) {   // twice at most
+    std::unique_ptr<void, hipError_t (*)(void *)> block(nullptr, hipFree);
+    size_t have = 0;
+    for (int classes = kAllClasses;;) {
         const int built = classes;
-        std::unique_ptr<tcv_plan, decltype(release)> p(new tcv_plan(), release);
+        std::unique_ptr<tcv_plan> p(new tcv_plan());
         size_t bytes = 0;
         tcv_status st = plan_setup(ctx, g, tuning, p.get(), &bytes, PlanFor::caller, classes);
         if (st != TCV_OK) return st;
-        void *block = nullptr;
-        if (hipMalloc(&block, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            return tcv_fail(ctx, TCV_ERR_NOMEM, "plan allocation of " + std::to_string(bytes) + " bytes failed");
+        if (bytes > have) {
+            block.reset();
+            void *q = nullptr;
+            if (hipMalloc(&q, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                if (p->sh.region > 0 || !p->parts.empty()) {   // the tiles alone may fit
+                    classes = 0;
+                    have = 0;
+                    continue;
+                }
+                return tcv_fail(ctx, TCV_ERR_NOMEM, "plan allocation of " + std::to_string(bytes) + " bytes failed");
+            }
+            block.reset(q);
+            have = bytes;
         }
-        plan_bind(p.get(), (char *)block);
-        p->ownsBlock = true;
+        plan_bind(p.get(), (char *)block.get());
         if (hipMemcpy(p->d_sSize, g->sSize, sizeof(int) * g->nPlanes, hipMemcpyHostToDevice) != hipSuccess)
             return tcv_fail(ctx, TCV_ERR_DEVICE, "plan upload failed");
         if ((st = tcv_plan_build(ctx, p.get(), g)) != TCV_OK) return st;
+        // (a first build with regions of thin classes is followed by one without)
         if (classes == kAllClasses && (st = thin_classes(ctx, g, p.get(), &classes)) != TCV_OK) return st;
         if (classes == built) {
             TCV_HIP(ctx, hipStreamSynchronize(ctx->stream));
+            p->ownsBlock = true;
+            block.release();
             *out = p.release();
             return TCV_OK;
         }

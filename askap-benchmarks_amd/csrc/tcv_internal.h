@@ -23,7 +23,8 @@ struct tcv_ctx {
     std::vector<hipEvent_t> pool;
     struct Stat { long launches = 0; double ms = 0.0; };
     std::map<std::string, Stat> stats;
-    // device counters: [0] visibilities skipped by the plain kernels (range)
+    // device counters: [0] visibilities skipped by the plain kernels (range), [6..7] (as
+    // ints) what thin_classes counts
     unsigned long long *d_counters = nullptr;
     // one int per persistent workgroup: work-item hand-over without LDS
     int *d_bcast = nullptr;
@@ -279,8 +280,9 @@ struct HalfStorage {
 };
 
 tcv_status plan_build_kernels(tcv_ctx *ctx, tcv_plan *p, const GeomDev &g);
-// Counts the tiles or regions that have entries into meta[8] of a plan by regions.
-tcv_status launch_plan_touched(tcv_ctx *ctx, tcv_plan *p);
+// Adds the number of a built plan's tiles or regions that have entries to *touched
+// (device); *entries (device, may be null): the entries.
+tcv_status launch_plan_touched(tcv_ctx *ctx, const tcv_plan *p, int *touched, int *entries);
 // Sets JobDesc::sharedGrid on every job whose grid overlaps another job's.
 void mark_shared_grids(std::vector<JobDesc> &jobs);
 // half == nullptr: FP32 taps and data

@@ -761,16 +761,18 @@ __device__ __forceinline__ Cut cut_of(const PlanDevArgs &a, const int *starts, c
     return Cut{ph, max(kAdaptChunk, min(a.chunk, chunk))};
 }
 
-// Counts the tiles that have entries.
+// Adds the number of tiles that have entries to *touched; *entries, when given:
+// how many they have.
 __global__ __launch_bounds__(256) void k_plan_touched(int nTiles, int k2, const int *__restrict__ starts,
-                                                      int *__restrict__ meta)
+                                                      int *__restrict__ touched, int *__restrict__ entries)
 {
     int n = 0;
     for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nTiles; t += gridDim.x * blockDim.x)
         n += starts[(long long)(t + 1) * k2] > starts[(long long)t * k2];
     int total;
     (void)block_exclusive_scan(n, &total);
-    if (threadIdx.x == 0 && total) atomicAdd(&meta[8], total);
+    if (threadIdx.x == 0 && total) atomicAdd(touched, total);
+    if (entries && blockIdx.x == 0 && threadIdx.x == 0) *entries = starts[(long long)nTiles * k2];
 }
 
 // Slots are (phase, tile) pairs in item order; list blockIdx.y of a plan has its own
@@ -2261,11 +2263,11 @@ static tcv_status scan_exclusive(tcv_ctx *ctx, const int *in, int *out, long lon
 // Visibilities from which k_plan_tile_keys runs 1024 threads a tile.
 constexpr int kBigTiles = 1 << 20;
 
-tcv_status launch_plan_touched(tcv_ctx *ctx, tcv_plan *p)
+tcv_status launch_plan_touched(tcv_ctx *ctx, const tcv_plan *p, int *touched, int *entries)
 {
     const PlanShape &sh = p->sh;
     hipLaunchKernelGGL(k_plan_touched, dim3(std::min((sh.nTiles + 255) / 256, 64)), dim3(256), 0, ctx->stream,
-                       sh.nTiles, sh.k2, (const int *)p->starts, p->meta);
+                       sh.nTiles, sh.k2, (const int *)p->starts, touched, entries);
     TCV_HIP(ctx, hipGetLastError());
     return TCV_OK;
 }
@@ -2337,7 +2339,7 @@ static tcv_status plan_build_one(tcv_ctx *ctx, tcv_plan *p, GeomDev g)
         if ((st = scan_exclusive(ctx, p->counts, p->starts, sh.nKeys, p->scanTmp, p->cursor)) != TCV_OK)
             return st;
         if ((st = bin(1)) != TCV_OK) return st;
-        if (touched && (st = launch_plan_touched(ctx, p)) != TCV_OK) return st;
+        if (touched && (st = launch_plan_touched(ctx, p, touched, nullptr)) != TCV_OK) return st;
     }
     // work items: cuts of the sorted entries into (phase, tile) ranges
     ItemLists lists{};
